@@ -283,8 +283,12 @@ static int grow(T** buf, int64_t* cap, int64_t count) {
   return RM_OK;
 }
 
+constexpr size_t LDS_BYTES = 160 * 1024;   // LDS of a CU, the most one workgroup may use
+
 // Workgroups of `kern` a CU holds with `lds` bytes of dynamic LDS, asked
-// once per (kernel, LDS size) -- the query costs more than a launch.
+// once per (kernel, LDS size) -- the query costs more than a launch.  0 when
+// the dynamic LDS and the kernel's own (the adaptive rule's Gram matrix, ...)
+// together exceed a CU's: such a launch would abort.
 static inline hipError_t occupancy(const void* kern, int threads, size_t lds, int* occ) {
   struct Entry { const void* k; size_t lds; int occ; };
   static std::mutex mu;
@@ -296,9 +300,14 @@ static inline hipError_t occupancy(const void* kern, int threads, size_t lds, in
       return hipSuccess;
     }
   int o = 0;
-  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kern, threads, lds);
+  hipFuncAttributes fa;
+  hipError_t e = hipFuncGetAttributes(&fa, kern);
   if (e != hipSuccess) return e;
-  if (o < 1) o = 1;
+  if (fa.sharedSizeBytes + lds <= LDS_BYTES) {
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kern, threads, lds);
+    if (e != hipSuccess) return e;
+    if (o < 1) o = 1;
+  }
   cache.push_back({kern, lds, o});
   *occ = o;
   return hipSuccess;

@@ -928,7 +928,7 @@ int long_run(void** scratch, const SubOp* d_ops, const int4* d_blk, const std::v
     const size_t vbytes = region_layout(lv, lx, 1, kcap, f32, false);
     const size_t lds_v = (f32 ? xl_bytes<true>() : xl_bytes<false>()) + vbytes;
     int gres_v = 0;
-    if (lds_v <= 160 * 1024) HIPCHK((resident<BLOCK, true, true>(n_cu, lds_v, &gres_v)));
+    if (lds_v <= LDS_BYTES) HIPCHK((resident<BLOCK, true, true>(n_cu, lds_v, &gres_v)));
     if (gres_v > 0) {
       // same offsets as the global region's vectors (lmax differs: a layout of their own)
       lv.ws = wb;

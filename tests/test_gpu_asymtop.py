@@ -113,3 +113,22 @@ def test_water_wide_operator_classes(device, jmax, fixed):
     assert np.abs(psi_d - psi_o).max() <= TOL_PSI
     if not fixed:
         assert np.array_equal(k_d, k_o)
+
+
+@pytest.mark.parametrize("precision,fixed", [("fp64", 0), ("fp32", 0), ("fp64", 12)])
+def test_block_form_lds_limit(device, precision, fixed):
+    """Domains of 70 and 76 rows (J <= 5): under the adaptive rule their
+    vectors fit a CU's LDS, but not beside the kernel's own Gram matrix, so
+    they stay in the global region; with a fixed dimension they fit."""
+    from richmol_amd import ensemble
+    from richmol_amd.tdse import TDSE
+    h0, leaves, bas = water(5)
+    fields = water_fields(385.0 + DT * np.arange(4))
+    X = ensemble.basis_rows(286, [0, 5, 20, 60])
+    ref, _ = _oracle(h0, leaves, fields, X, fixed=fixed or None)
+    ens = ensemble.Ensemble(_summed(leaves, fields, 0), h0, TDSE(t_end=20.0, dt=DT, t_units="fs").exp_fac, X,
+                            krylov_fixed=fixed)
+    ens.set_kernel("block")
+    ens.set_precision(precision)
+    ens.propagate(None, table=ens.prepare(fields, per_term=True))
+    assert np.abs(ens.psi.cpu().numpy() - ref).max() <= (TOL_PSI if precision == "fp64" else 2e-6)
