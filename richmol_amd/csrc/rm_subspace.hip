@@ -475,12 +475,17 @@ __global__ __launch_bounds__(64) void k_sub_pair(SubArgs a) {
   const int npair = (a.nitems + 1) >> 1;
   for (int pr = blockIdx.x; pr < npair; pr += gridDim.x) {
     const int itm = 2 * pr + h;
-    const int4 item = itm < a.nitems ? a.items[itm] : make_int4(-1, 0, 0, a.items[2 * pr].w);
-    const int b = item.x, lo = item.y, len = b >= 0 ? item.z : 0;
-    const SubOp op = a.ops ? a.ops[item.w] : a.op0;   // the same for both halves
+    int4 item = itm < a.nitems ? a.items[itm] : make_int4(-1, 0, 0, 0);
+    // an empty half repeats its partner's wavepacket and stores nothing: with
+    // rows of zeros it would take the exact-breakdown path (a Gram-Schmidt of
+    // every basis vector) in each iteration, which its partner waits for
+    const bool own = item.x >= 0;
+    if (!own) item = a.items[itm ^ 1];
+    const int b = item.x, lo = item.y, len = item.z;
+    const SubOp op = a.ops ? a.ops[__builtin_amdgcn_readfirstlane(item.w)] : a.op0;   // the same for both halves
     if (op.stale && *op.stale == op.call_id) {
       // reused domains that failed their check: both wavepackets are left as they are
-      if (i == 0 && b >= 0 && op.status) op.status[b - op.kcol0] |= RM_STALE_DOMAIN;
+      if (i == 0 && own && op.status) op.status[b - op.kcol0] |= RM_STALE_DOMAIN;
       continue;
     }
     const int n = op.n, W = op.w;
@@ -616,7 +621,7 @@ __global__ __launch_bounds__(64) void k_sub_pair(SubArgs a) {
         if ((step + 1) % OBK == 0 || step + 1 == op.nsteps) {
           wave_sync();
           const int nk = step % OBK + 1, s0 = step + 1 - nk;
-          if (i < nk && b >= 0 && op.expect) {
+          if (i < nk && own && op.expect) {
             double2 acc = zero;
             for (int r = 0; r < len; ++r) acc = cadd(acc, s_ob[i][32 * h + r]);
             op.expect[(int64_t)(s0 + i) * op.expect_ld + b - op.kcol0] = acc;
@@ -645,7 +650,7 @@ __global__ __launch_bounds__(64) void k_sub_pair(SubArgs a) {
       double2 vk = op.phase ? cmul(st, ph) : st;
       if (sf == 0) {
         st = op.phase ? cmul(vk, ph) : vk;
-        if (i == 0 && b >= 0 && op.kused) op.kused[(int64_t)step * op.kused_ld + b - op.kcol0] = 0;
+        if (i == 0 && own && op.kused) op.kused[(int64_t)step * op.kused_ld + b - op.kcol0] = 0;
         observe(step);
         continue;
       }
@@ -734,21 +739,25 @@ __global__ __launch_bounds__(64) void k_sub_pair(SubArgs a) {
           vp = vk;
           vk = cscale(ib, Wr);
         } else {
-          // exact breakdown: Gram-Schmidt of ones against the basis (tdse.py:459-465)
+          // exact breakdown: Gram-Schmidt of ones against the basis (tdse.py:459-465);
+          // once the basis spans the domain (nothing left, the vector is zero)
+          // every later one is zero too
           vp = vk;
-          Wr = ok ? make_double2(1.0, 0.0) : zero;
-          for (int j = 0; j < it; ++j) {
-            double d0 = 0.0, d1 = 0.0;
-            if (ok) {
-              const double2 x = s_V[j * 64 + l];
-              d0 = x.x * Wr.x + x.y * Wr.y;
-              d1 = x.x * Wr.y - x.y * Wr.x;
+          {
+            Wr = ok ? make_double2(1.0, 0.0) : zero;
+            for (int j = 0; j < it; ++j) {
+              double d0 = 0.0, d1 = 0.0;
+              if (ok) {
+                const double2 x = s_V[j * 64 + l];
+                d0 = x.x * Wr.x + x.y * Wr.y;
+                d1 = x.x * Wr.y - x.y * Wr.x;
+              }
+              const double2 proj = make_double2(half_allsum32(d0), half_allsum32(d1));
+              if (ok) Wr = csub(Wr, cmul(proj, s_V[j * 64 + l]));
             }
-            const double2 proj = make_double2(half_allsum32(d0), half_allsum32(d1));
-            if (ok) Wr = csub(Wr, cmul(proj, s_V[j * 64 + l]));
+            const double nv = sqrt(half_allsum32(Wr.x * Wr.x + Wr.y * Wr.y));
+            vk = nv > 0.0 ? make_double2(Wr.x / nv, Wr.y / nv) : zero;
           }
-          const double nv = sqrt(half_allsum32(Wr.x * Wr.x + Wr.y * Wr.y));
-          vk = nv > 0.0 ? make_double2(Wr.x / nv, Wr.y / nv) : zero;
         }
         s_V[it * 64 + l] = vk;
         sb[it] = beta;
@@ -790,11 +799,11 @@ __global__ __launch_bounds__(64) void k_sub_pair(SubArgs a) {
       if (j < k - 1) u0 = cfma(sc[j], s_V[j * 64 + vrow], u0);
       const double2 uu = cfma(sc[k - 1], vk, cadd(u0, u1));
       st = ok ? (op.phase ? cmul(uu, ph) : uu) : zero;
-      if (i == 0 && b >= 0 && op.kused) op.kused[(int64_t)step * op.kused_ld + b - op.kcol0] = k;
+      if (i == 0 && own && op.kused) op.kused[(int64_t)step * op.kused_ld + b - op.kcol0] = k;
       observe(step);
       wave_sync();
     }
-    if (ok) op.psi[(int64_t)b * op.ld + orig] = st;
+    if (ok && own) op.psi[(int64_t)b * op.ld + orig] = st;
   }
 }
 
