@@ -273,7 +273,7 @@ def asymtop_leg(nsteps, cpu_steps=3):
     return out
 
 
-def kron_leg(nsteps=3, ncols=64, jmax=80, krylov=12, t0_fs=50000.0, kernel="gemm", cpu_matvecs=0,
+def kron_leg(nsteps=3, ncols=64, jmax=80, krylov=12, t0_fs=50000.0, kernel="prim", cpu_matvecs=0,
              accuracy_steps=0):
     """The large asymmetric-top configuration: H2S-like rotor (A, B, C =
     10.36, 9.02, 4.73 cm^-1), J <= jmax with all m (N = 708 561 at J <= 80),
@@ -399,7 +399,7 @@ def main():
                     help="timed steps of the large asymmetric-top (Kronecker-block) leg (0: skip)")
     ap.add_argument("--kron-accuracy-steps", type=int, default=60,
                     help="steps of the large-top FP32-vs-FP64 comparison (0: skip)")
-    ap.add_argument("--kron-kernel", default="gemm", choices=["gemm", "mfma", "fused"],
+    ap.add_argument("--kron-kernel", default="prim", choices=["prim", "gemm", "mfma", "fused"],
                     help="matvec form of the large asymmetric-top leg")
     ap.add_argument("--kron-only", action="store_true",
                     help="only the large asymmetric-top leg (for profiling its kernels) and exit")

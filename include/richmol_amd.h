@@ -414,7 +414,9 @@ int rm_kplan_destroy(rm_kplan* plan);
 /* n: states per wavepacket; gemm_flops_per_col: real flops of one matvec's
  * dense products per wavepacket. */
 int rm_kplan_info(const rm_kplan* plan, int64_t* n, double* gemm_flops_per_col);
-/* Matvec form (no reference counterpart).  RM_KKERNEL_GEMM (default): the
+/* Matvec form (no reference counterpart).  RM_KKERNEL_PRIM (default of a plan
+ * with K factors, rm_kplan_set_factors): the operator as a stencil in the
+ * primitive symmetric-top basis.  RM_KKERNEL_GEMM (default without): the
  * m-mixed input (MF_w X) stored, then one rocBLAS product per output J, the
  * build of the next J chunk overlapping the products of the last.
  * RM_KKERNEL_FUSED: one launch per matvec on the matrix cores, the m-mixed
@@ -425,7 +427,16 @@ int rm_kplan_info(const rm_kplan* plan, int64_t* n, double* gemm_flops_per_col);
 #define RM_KKERNEL_FUSED 0
 #define RM_KKERNEL_GEMM  1
 #define RM_KKERNEL_MFMA  2
+#define RM_KKERNEL_PRIM  3
 int rm_kplan_set_kernel(rm_kplan* plan, int32_t kernel);
+/* The factors of the K blocks of a rigid rotor, K = C1^H P C2 (no reference
+ * counterpart; labtens.py:482-496 forms K this way), which make
+ * RM_KKERNEL_PRIM available and the plan's choice.  C: per J (in the plan's
+ * order) the (2J+1) x (2J+1) unitary matrix of the states' coefficients,
+ * complex row-major (primitive k = -J..J, state).  P: per block
+ * [5][2 J1 + 1] complex, row s + 2 the elements between primitive k1 and
+ * k1 - s (0 where |k1 - s| > J2). */
+int rm_kplan_set_factors(rm_kplan* plan, const double* C, const double* P);
 /* y = H(F) x for ncols wavepackets (device, complex, row b at b*ld, internal
  * order); fprod_dev: device, nslot complex.  precision RM_PREC_FP32: the
  * products in FP32 (complex64 operands, FP32 accumulation). */

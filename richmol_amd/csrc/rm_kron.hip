@@ -26,7 +26,7 @@
 #include <algorithm>
 #include <vector>
 
-#include "rm_common.h"
+#include "rm_kprim.h"
 
 namespace {
 
@@ -70,8 +70,14 @@ struct rm_kplan {
   KBlk* d_blk = nullptr;
   double2* d_mf = nullptr;
   int64_t mf_count = 0;
+  // the K blocks and, built from them on the first use of a form that needs
+  // them, its stacks
+  std::vector<double> h_K;
+  std::vector<int64_t> h_koff;
   std::vector<double*> kbig64;            // per J index: (2 Ktot) x (2 dk) row-major
   std::vector<float*> kbig32;
+  // the operator in the primitive basis (rm_kplan_set_factors)
+  KPrim* prim = nullptr;
   rocblas_handle rb = nullptr;
   // fused form: per J1 the stacked K with columns padded to groups of four
   // (FGK) and the rows of a group interleaved [re x 4 | im x 4], output
@@ -80,6 +86,8 @@ struct rm_kplan {
   int32_t kernel = RM_KKERNEL_GEMM;
   std::vector<int32_t> kpad, npad;      // per J index
   std::vector<int64_t> kf_off, cm_off;  // per J index
+  int64_t kf_count = 0, cm_count = 0;   // elements of the K stack and the column map
+  bool kbig_ready = false;
   double* d_kf64 = nullptr;
   float* d_kf32 = nullptr;
   int32_t* d_colmap = nullptr;
@@ -974,6 +982,7 @@ void kplan_free(rm_kplan* p) {
   for (hipEvent_t e : p->ev)
     if (e) (void)hipEventDestroy(e);
   if (p->gs) (void)hipStreamDestroy(p->gs);
+  kprim_free(p->prim);
   delete p;
 }
 
@@ -1076,33 +1085,10 @@ extern "C" int rm_kplan_create(int32_t nJ, const int32_t* Js, int32_t nslot, int
     kplan_free(p);
     return rc;
   }
-  // per J1: the real form of the stacked K, [[Kr^T, Ki^T], [-Ki^T, Kr^T]] (2 Ktot x 2 dk1)
   p->kbig64.assign(nJ, nullptr);
   p->kbig32.assign(nJ, nullptr);
-  for (int a = 0; a < nJ; ++a) {
-    if (p->src[a].empty()) continue;
-    const int64_t dk1 = jdim(Js[a]), kt = p->ktot[a], ncol = 2 * dk1;
-    std::vector<double> kb((size_t)(2 * kt * ncol), 0.0);
-    for (int q : p->src[a]) {
-      const int64_t dk2 = jdim(J2[q]), ko = p->kq_off[q];
-      const double* Kq = K + 2 * k_off[q];   // complex (dk1 x dk2) row-major
-      for (int64_t k1 = 0; k1 < dk1; ++k1)
-        for (int64_t k2 = 0; k2 < dk2; ++k2) {
-          const double kr = Kq[2 * (k1 * dk2 + k2)], ki = Kq[2 * (k1 * dk2 + k2) + 1];
-          const int64_t r0 = ko + k2, r1 = kt + ko + k2;
-          kb[(size_t)(r0 * ncol + k1)] = kr;
-          kb[(size_t)(r0 * ncol + dk1 + k1)] = ki;
-          kb[(size_t)(r1 * ncol + k1)] = -ki;
-          kb[(size_t)(r1 * ncol + dk1 + k1)] = kr;
-        }
-    }
-    std::vector<float> kf(kb.begin(), kb.end());
-    if ((rc = upload(&p->kbig64[a], kb.data(), (int64_t)kb.size())) ||
-        (rc = upload(&p->kbig32[a], kf.data(), (int64_t)kf.size()))) {
-      kplan_free(p);
-      return rc;
-    }
-  }
+  p->h_koff.assign(k_off, k_off + (nblk ? nblk + 1 : 0));
+  if (nblk) p->h_K.assign(K, K + 2 * k_off[nblk]);
   // fused form: padded stacked columns (groups of FGK, the total a multiple
   // of FBK / 2), interleaved group rows, output columns padded to FBN
   p->kpad.assign(nJ, 0);
@@ -1126,46 +1112,8 @@ extern "C" int rm_kplan_create(int32_t nJ, const int32_t* Js, int32_t nslot, int
     kfpos += 2 * kp * p->npad[a];
     cmpos += kp;
   }
-  {
-    std::vector<double> kf((size_t)std::max<int64_t>(kfpos, 1), 0.0);
-    std::vector<int32_t> cm((size_t)std::max<int64_t>(cmpos, 1), -1);
-    for (int a = 0; a < nJ; ++a) {
-      const int64_t dk1 = jdim(Js[a]), np = p->npad[a];
-      double* kb = kf.data() + p->kf_off[a];
-      int64_t c0 = 0;
-      for (size_t li = 0; li < p->src[a].size(); ++li) {
-        const int q = p->src[a][li];
-        const int64_t dk2 = jdim(J2[q]);
-        const double* Kq = K + 2 * k_off[q];
-        for (int64_t k2 = 0; k2 < dk2; ++k2) {
-          const int64_t col = c0 + k2, g = col / FGK, i = col % FGK;
-          cm[(size_t)(p->cm_off[a] + col)] = (int32_t)((li << 16) | k2);
-          double* rre = kb + (2 * FGK * g + i) * np;
-          double* rim = kb + (2 * FGK * g + FGK + i) * np;
-          for (int64_t k1 = 0; k1 < dk1; ++k1) {
-            const double kr = Kq[2 * (k1 * dk2 + k2)], ki = Kq[2 * (k1 * dk2 + k2) + 1];
-            rre[k1] = kr;
-            rre[dk1 + k1] = ki;
-            rim[k1] = -ki;
-            rim[dk1 + k1] = kr;
-          }
-        }
-        c0 += (dk2 + FGK - 1) / FGK * FGK;
-      }
-    }
-    std::vector<float> kf32(kf.begin(), kf.end());
-    if ((rc = upload(&p->d_kf64, kf.data(), (int64_t)kf.size())) ||
-        (rc = upload(&p->d_kf32, kf32.data(), (int64_t)kf32.size())) ||
-        (rc = upload(&p->d_colmap, cm.data(), (int64_t)cm.size()))) {
-      kplan_free(p);
-      return rc;
-    }
-  }
-  if (rocblas_create_handle(&p->rb) != rocblas_status_success) {
-    p->rb = nullptr;
-    kplan_free(p);
-    return fail(RM_ERR_HIP, "rm_kplan_create: rocblas_create_handle failed");
-  }
+  p->kf_count = kfpos;
+  p->cm_count = cmpos;
   p->ev.assign(KCHUNK + 1, nullptr);
   if (hipStreamCreateWithFlags(&p->gs, hipStreamNonBlocking) != hipSuccess) {
     p->gs = nullptr;
@@ -1178,10 +1126,6 @@ extern "C" int rm_kplan_create(int32_t nJ, const int32_t* Js, int32_t nslot, int
       kplan_free(p);
       return fail(RM_ERR_HIP, "rm_kplan_create: event creation failed");
     }
-  if (rocblas_set_stream(p->rb, p->gs) != rocblas_status_success) {
-    kplan_free(p);
-    return fail(RM_ERR_HIP, "rm_kplan_create: rocblas_set_stream failed");
-  }
   *out = p;
   return RM_OK;
 }
@@ -1269,8 +1213,92 @@ int kwork(rm_kplan* p, int32_t ncols, int32_t m, bool f32, KWork* w, bool adapti
   return RM_OK;
 }
 
+// The K stacks of the stored forms (with rocBLAS its handle), on first use:
+// per J1 the real form of the stacked K, [[Kr^T, Ki^T], [-Ki^T, Kr^T]] (2 Ktot x 2 dk1).
+int kbig_build(rm_kplan* p) {
+  if (p->kernel != RM_KKERNEL_MFMA && !p->rb) {
+    if (rocblas_create_handle(&p->rb) != rocblas_status_success) {
+      p->rb = nullptr;
+      return fail(RM_ERR_HIP, "Kronecker-block plan: rocblas_create_handle failed");
+    }
+    if (rocblas_set_stream(p->rb, p->gs) != rocblas_status_success) {
+      (void)rocblas_destroy_handle(p->rb);
+      p->rb = nullptr;
+      return fail(RM_ERR_HIP, "Kronecker-block plan: rocblas_set_stream failed");
+    }
+  }
+  if (p->kbig_ready) return RM_OK;
+  int rc = RM_OK;
+  for (int a = 0; a < p->nJ; ++a) {
+    if (p->src[a].empty() || p->kbig32[a]) continue;
+    const int64_t dk1 = jdim(p->Js[a]), kt = p->ktot[a], ncol = 2 * dk1;
+    std::vector<double> kb((size_t)(2 * kt * ncol), 0.0);
+    for (int q : p->src[a]) {
+      const int64_t dk2 = jdim(p->h_J2[q]), ko = p->kq_off[q];
+      const double* Kq = p->h_K.data() + 2 * p->h_koff[q];   // complex (dk1 x dk2) row-major
+      for (int64_t k1 = 0; k1 < dk1; ++k1)
+        for (int64_t k2 = 0; k2 < dk2; ++k2) {
+          const double kr = Kq[2 * (k1 * dk2 + k2)], ki = Kq[2 * (k1 * dk2 + k2) + 1];
+          const int64_t r0 = ko + k2, r1 = kt + ko + k2;
+          kb[(size_t)(r0 * ncol + k1)] = kr;
+          kb[(size_t)(r0 * ncol + dk1 + k1)] = ki;
+          kb[(size_t)(r1 * ncol + k1)] = -ki;
+          kb[(size_t)(r1 * ncol + dk1 + k1)] = kr;
+        }
+    }
+    std::vector<float> kf(kb.begin(), kb.end());
+    if ((!p->kbig64[a] && (rc = upload(&p->kbig64[a], kb.data(), (int64_t)kb.size()))) ||
+        (rc = upload(&p->kbig32[a], kf.data(), (int64_t)kf.size())))
+      return rc;
+  }
+  p->kbig_ready = true;
+  return RM_OK;
+}
+
+// The fused form's interleaved K stacks and column map, on first use.
+int kf_build(rm_kplan* p) {
+  if (p->d_colmap) return RM_OK;
+  int rc = RM_OK;
+  {
+    std::vector<double> kf((size_t)std::max<int64_t>(p->kf_count, 1), 0.0);
+    std::vector<int32_t> cm((size_t)std::max<int64_t>(p->cm_count, 1), -1);
+    for (int a = 0; a < p->nJ; ++a) {
+      const int64_t dk1 = jdim(p->Js[a]), np = p->npad[a];
+      double* kb = kf.data() + p->kf_off[a];
+      int64_t c0 = 0;
+      for (size_t li = 0; li < p->src[a].size(); ++li) {
+        const int q = p->src[a][li];
+        const int64_t dk2 = jdim(p->h_J2[q]);
+        const double* Kq = p->h_K.data() + 2 * p->h_koff[q];
+        for (int64_t k2 = 0; k2 < dk2; ++k2) {
+          const int64_t col = c0 + k2, g = col / FGK, i = col % FGK;
+          cm[(size_t)(p->cm_off[a] + col)] = (int32_t)((li << 16) | k2);
+          double* rre = kb + (2 * FGK * g + i) * np;
+          double* rim = kb + (2 * FGK * g + FGK + i) * np;
+          for (int64_t k1 = 0; k1 < dk1; ++k1) {
+            const double kr = Kq[2 * (k1 * dk2 + k2)], ki = Kq[2 * (k1 * dk2 + k2) + 1];
+            rre[k1] = kr;
+            rre[dk1 + k1] = ki;
+            rim[k1] = -ki;
+            rim[dk1 + k1] = kr;
+          }
+        }
+        c0 += (dk2 + FGK - 1) / FGK * FGK;
+      }
+    }
+    std::vector<float> kf32(kf.begin(), kf.end());
+    if ((!p->d_kf64 && (rc = upload(&p->d_kf64, kf.data(), (int64_t)kf.size()))) ||
+        (!p->d_kf32 && (rc = upload(&p->d_kf32, kf32.data(), (int64_t)kf32.size()))) ||
+        (rc = upload(&p->d_colmap, cm.data(), (int64_t)cm.size())))
+      return rc;
+  }
+  return RM_OK;
+}
+
 // The (output J1, source block) tasks for ncols wavepackets, uploaded once per call.
 int ktasks(rm_kplan* p, int32_t ncols, int64_t* ntask, std::vector<int64_t>& zoff_J, hipStream_t s) {
+  const int rb = p->kernel == RM_KKERNEL_FUSED ? kf_build(p) : kbig_build(p);
+  if (rb) return rb;
   std::vector<KTask>& h = p->h_tasks;
   h.clear();
   zoff_J.assign(p->nJ, 0);
@@ -1527,6 +1555,8 @@ extern "C" int rm_kplan_matvec(rm_kplan* p, const void* x, void* y, int64_t ld, 
     return fail(RM_ERR_ARG, "rm_kplan_matvec: unknown precision %d", precision);
   hipStream_t s = (hipStream_t)stream;
   const bool f32 = precision == RM_PREC_FP32;
+  if (p->kernel == RM_KKERNEL_PRIM)
+    return kprim_matvec(p->prim, (const double2*)x, (double2*)y, ld, ncols, (const double2*)fprod_dev, f32, s);
   KWork w;
   int rc = kwork(p, ncols, 0, f32, &w);
   if (rc) return rc;
@@ -1604,17 +1634,36 @@ static int kplan_propagate(rm_kplan* p, void* psi, int64_t ld, int32_t ncols, in
   if (status)
     hipLaunchKernelGGL(k_kp_izero, dim3(grid_for(ncols, 256)), dim3(256), 0, s, status, ncols);
   if (nsteps == 0) return RM_OK;
-  KWork w;
-  int rc = kwork(p, ncols, m, f32, &w, adaptive);
-  if (rc) return rc;
-  int64_t ntask = 0;
-  std::vector<int64_t> zoff_J;
-  if ((rc = ktasks(p, ncols, &ntask, zoff_J, s))) return rc;
   // the field products of every step, uploaded once
   const int64_t nf = std::max<int32_t>(p->nslot, 1);
+  int rc;
   if ((rc = grow(&p->d_fp, &p->fp_cap, nsteps * nf))) return rc;
   if (p->nslot)
     HIPCHK(hipMemcpyAsync(p->d_fp, fprod, sizeof(double2) * nsteps * p->nslot, hipMemcpyHostToDevice, s));
+  if (p->kernel == RM_KKERNEL_PRIM &&
+      (!obs || (obs->kernel == RM_KKERNEL_PRIM && kprim_same_basis(p->prim, obs->prim)))) {
+    double2* ex = expect;
+    if (obs) {
+      if (!ex) {
+        if ((rc = grow(&obs->d_ex, &obs->ex_cap, nsteps * ncols))) return rc;
+        ex = obs->d_ex;
+      }
+      if ((rc = grow(&obs->d_fp, &obs->fp_cap, std::max<int32_t>(obs->nslot, 1)))) return rc;
+      if (obs->nslot)
+        HIPCHK(hipMemcpyAsync(obs->d_fp, obs_fprod, sizeof(double2) * obs->nslot, hipMemcpyHostToDevice, s));
+    }
+    if ((rc = kprim_propagate(p->prim, (double2*)psi, ld, ncols, nsteps, p->nslot, fprod, p->d_fp,
+                              make_double2(f_re, f_im), (const double2*)phase, krylov_fixed, maxorder, tol, kused,
+                              status, f32, obs ? obs->prim : nullptr, obs ? obs->d_fp : nullptr, ex, s)))
+      return rc;
+    if (obs && expect_sum) return launch_expect_sum(nsteps, ncols, ex, expect_sum, s);
+    return RM_OK;
+  }
+  KWork w;
+  if ((rc = kwork(p, ncols, m, f32, &w, adaptive))) return rc;
+  int64_t ntask = 0;
+  std::vector<int64_t> zoff_J;
+  if ((rc = ktasks(p, ncols, &ntask, zoff_J, s))) return rc;
   const double2* ph = (const double2*)phase;
   const double2 f = make_double2(f_re, f_im);
   const dim3 cg = chunk_grid(p, ncols), cb(256);
@@ -1736,8 +1785,34 @@ static int kplan_propagate(rm_kplan* p, void* psi, int64_t ld, int32_t ncols, in
 
 extern "C" int rm_kplan_set_kernel(rm_kplan* p, int32_t kernel) {
   if (!p) return fail(RM_ERR_ARG, "rm_kplan_set_kernel: NULL plan");
-  if (kernel != RM_KKERNEL_FUSED && kernel != RM_KKERNEL_GEMM && kernel != RM_KKERNEL_MFMA)
+  if (kernel != RM_KKERNEL_FUSED && kernel != RM_KKERNEL_GEMM && kernel != RM_KKERNEL_MFMA &&
+      kernel != RM_KKERNEL_PRIM)
     return fail(RM_ERR_ARG, "rm_kplan_set_kernel: unknown kernel %d", kernel);
+  if (kernel == RM_KKERNEL_PRIM && !p->prim)
+    return fail(RM_ERR_ARG, "rm_kplan_set_kernel: the plan has no K factors (rm_kplan_set_factors)");
   p->kernel = kernel;
+  return RM_OK;
+}
+
+extern "C" int rm_kplan_set_factors(rm_kplan* p, const double* C, const double* P) {
+  if (!p || !C || (p->nblk > 0 && !P)) return fail(RM_ERR_ARG, "rm_kplan_set_factors: NULL argument");
+  if (p->prim) return fail(RM_ERR_ARG, "rm_kplan_set_factors: the plan has its factors already");
+  std::vector<KPrimBlock> blk((size_t)p->nblk);
+  for (int q = 0; q < p->nblk; ++q) {
+    KPrimBlock& b = blk[(size_t)q];
+    const KBlk& k = p->h_blk[(size_t)q];
+    b.J1 = p->h_J1[q];
+    b.J2 = p->h_J2[q];
+    b.ncart = k.ncart;
+    b.slot0 = k.slot0;
+    b.nsig = k.nsig;
+    b.d_off = k.d_off;
+    if (k.nsig > 5 || std::abs(b.J1 - b.J2) > 2)
+      return fail(RM_ERR_ARG, "rm_kplan_set_factors: block %d is not of rank <= 2", q);
+    for (int t = 0; t < 5; ++t) b.sig[t] = t < k.nsig ? p->h_sig[(size_t)(p->h_sig_off[q] + t)] : 0;
+  }
+  int rc = kprim_create(&p->prim, p->Js, p->h_voff, p->n, blk, p->d_mdiag, C, P);
+  if (rc) return rc;
+  p->kernel = RM_KKERNEL_PRIM;
   return RM_OK;
 }

@@ -76,6 +76,18 @@ def _kprim(comps_w, w, J1, J2):
     return P
 
 
+def _kdiag(P, J1, J2):
+    """The diagonals k1 - k2 = s = -2..2 of a primitive-k matrix as a
+    (5, 2J1+1) array: row s + 2 the elements (k1, k1 - s), 0 where |k1 - s| >
+    J2."""
+    out = np.zeros((5, 2 * J1 + 1), dtype=np.complex128)
+    k1 = np.arange(-J1, J1 + 1)
+    for s in range(-2, 3):
+        ok = np.abs(k1 - s) <= J2
+        out[s + 2, ok] = P[k1[ok] + J1, k1[ok] - s + J2]
+    return out
+
+
 def _mdiag(ucols_w, w, J1, J2, ncart):
     """Diagonals of M_w,cart (rot._m_block with all m): for every sigma,
     the (ncart, 2J1+1) values at m2 = m1 - sigma (0 where m2 is out of
@@ -105,7 +117,13 @@ class KronOperator:
     labels of the leaf's M components; layout: Jlist, per-J state offsets
     (internal order: m-major, species-concatenated k) and the permutation
     `perm` with internal index i = perm[full-form index].
+
+    factors: (C, P) with K = C[J1]^H P C[J2]: per J the coefficient matrix C
+    (primitive k, state) and per block the diagonals of P (_kdiag), which the
+    device plan's primitive-basis form works on; None when the K blocks'
+    primitive basis is not known.
     """
+    factors = None
 
     def __init__(self, basis, tensors, scales=None):
         self.Jlist = list(basis.Jlist)
@@ -119,6 +137,7 @@ class KronOperator:
         for J in self.Jlist:
             if C[J].shape != (2 * J + 1, 2 * J + 1):
                 raise ValueError("KronOperator needs the full k space of every J")
+        Pd = []
         for li, (tens, scale) in enumerate(zip(tensors, scales)):
             rank, comps, ucols = rot.spherical_components(tens)
             carts = rot.CART[rank]
@@ -132,7 +151,8 @@ class KronOperator:
                     for w in sorted(comps):
                         if abs(J1 - J2) > w:
                             continue
-                        K = C[J1].conj().T @ _kprim(comps[w], w, J1, J2) @ C[J2]
+                        P = _kprim(comps[w], w, J1, J2)
+                        K = C[J1].conj().T @ P @ C[J2]
                         K[np.abs(K) < rot._EPS] = 0
                         if not np.any(K):
                             continue
@@ -140,6 +160,8 @@ class KronOperator:
                         if not md:
                             continue
                         self.blocks.append((li, J1, J2, w, K * scale, md))
+                        Pd.append(_kdiag(P, J1, J2) * scale)
+        self.factors = (C, Pd)
         # internal layout and the permutation from the reference's full-form order
         off, pos = {}, 0
         for J in self.Jlist:
@@ -243,7 +265,33 @@ class KronOperator:
                 full += dm * dks
         self.perm = perm
         self.energies = None
+        self._find_factors(leaf0.__dict__.get("_kcoef"))
         return self, fprods
+
+    def _find_factors(self, coef):
+        """The primitive-basis factors of blocks read from a CarTens, when its
+        builder left the coefficients: P = C1 K C2^H must be banded and give K
+        back to rounding (a tensor changed since does not, and keeps the
+        dense form)."""
+        if coef is None or any(J not in coef or coef[J].shape != (2 * J + 1, 2 * J + 1) for J in self.Jlist):
+            return
+        for J in self.Jlist:
+            if np.abs(coef[J].conj().T @ coef[J] - np.eye(2 * J + 1)).max() > 1e-12:
+                return
+        Pd = []
+        for _, J1, J2, _, K, _ in self.blocks:
+            P = coef[J1] @ K @ coef[J2].conj().T
+            d = _kdiag(P, J1, J2)
+            tol = 1e-13 * np.abs(K).max()
+            d[np.abs(d) < 1e-2 * tol] = 0
+            k1 = np.arange(-J1, J1 + 1)
+            for s in range(-2, 3):
+                ok = np.abs(k1 - s) <= J2
+                P[k1[ok] + J1, k1[ok] - s + J2] -= d[s + 2, ok]
+            if np.abs(P).max() > tol:
+                return
+            Pd.append(d)
+        self.factors = (coef, Pd)
 
     def slot_row(self, fprods):
         """Field products of one step in slot order from per-leaf dicts
@@ -351,6 +399,13 @@ class DeviceKronPlan:
         self.n = int(n.value)
         self.gemm_flops_per_col = float(fl.value)
         self.kernel = "gemm"
+        if kop.factors is not None:
+            C, Pd = kop.factors
+            Ca = np.concatenate([np.ascontiguousarray(C[J], dtype=np.complex128).ravel() for J in kop.Jlist])
+            Pa = np.concatenate([np.zeros(0, np.complex128)] + [np.ascontiguousarray(d).ravel() for d in Pd])
+            _lib.check(lib.rm_kplan_set_factors(h, P(Ca.view(np.float64), ctypes.c_double),
+                                                P(Pa.view(np.float64), ctypes.c_double)), "rm_kplan_set_factors")
+            self.kernel = "prim"
 
     def close(self):
         """Destroy the device plan (idempotent)."""
@@ -365,10 +420,13 @@ class DeviceKronPlan:
         except Exception:
             pass
 
-    KERNELS = {"fused": 0, "gemm": 1, "mfma": 2}
+    KERNELS = {"fused": 0, "gemm": 1, "mfma": 2, "prim": 3}
 
     def set_kernel(self, kernel):
-        """'gemm' (default): the m-mixed input stored, rocBLAS per output J;
+        """'prim' (default with kop.factors): a stencil in the primitive
+        symmetric-top basis, the wavepackets transformed once before and
+        after each step's Krylov recurrence;
+        'gemm' (default without): the m-mixed input stored, rocBLAS per output J;
         'mfma': the m-mixed input stored, the library's own matrix-core
         product per J chunk; 'fused': one MFMA launch per matvec, the m-mixed
         input built in LDS."""

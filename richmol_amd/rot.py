@@ -430,6 +430,9 @@ def _build(basis, rank, carts, comps, ucols):
     T.kmat, T.mmat = {}, {}
     dJ = max(comps.keys()) if comps else 0
     kcache, mcache = {}, {}
+    # the states' coefficients over primitive k, species concatenated: the
+    # factored operator (kron) works in the primitive basis with them
+    T._kcoef = {J: np.concatenate([basis.kfun[J][s][1] for s in basis.symlist[J]], axis=1) for J in basis.Jlist}
     for J2 in basis.Jlist:
         for J1 in basis.Jlist:
             if abs(J1 - J2) > dJ:

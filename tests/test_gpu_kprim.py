@@ -1,0 +1,150 @@
+"""The Kronecker-block operator's primitive-basis form (the stencil over
+(m, k) and the transforms around it): matvecs against the host factorisation
+(KronOperator.matvec, 1e-13 relative in FP64, 2e-6 with FP32 products) at the
+sizes where its tiling changes, for every field pattern that selects another
+stencil, and propagation against the dense form (rocBLAS products, 1e-11).
+"""
+import numpy as np
+import pytest
+
+from _fixtures import LARGE_B, large_top_tensors
+from richmol_amd import rot
+from richmol_amd.kron import DeviceKronPlan, KronOperator, slot_products
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = {"z": [0.0, 0.0, 1.3e8], "x": [1.1e8, 0.0, 0.0], "xy": [7e7, -9e7, 0.0], "xyz": [7e7, 5e7, -9e7]}
+
+
+def _basis(jmin, jmax, cplx):
+    bas = rot.asymtop_basis(*LARGE_B, jmax, Jmin=jmin)
+    if cplx:   # states with arbitrary phases: complex coefficients
+        rng = np.random.default_rng(5)
+        for J in bas.Jlist:
+            for s, (kp, c) in bas.kfun[J].items():
+                bas.kfun[J][s] = (kp, c * np.exp(2j * np.pi * rng.random(c.shape[1]))[None, :])
+    return bas
+
+
+def _rows(n, ncols, seed):
+    rng = np.random.default_rng(seed)
+    return rng.normal(size=(ncols, n)) + 1j * rng.normal(size=(ncols, n))
+
+
+def _tensors(kind):
+    tens, scales = large_top_tensors()
+    if kind == "diag":      # s = 0, +-2 only
+        return [np.diag([24.0, 25.5, 24.7])], [scales[1]]
+    if kind == "dipole":    # s = 0, +-1
+        return [np.array([0.2, 0.3, -0.1])], [scales[0]]
+    return tens, scales
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 2e-6)])
+@pytest.mark.parametrize("jmin,jmax,ncols,kind,field,cplx", [
+    (0, 0, 1, "full", "xyz", False), (0, 3, 1, "full", "z", False), (0, 9, 13, "full", "xy", False),
+    (0, 9, 3, "dipole", "xyz", True), (0, 12, 5, "diag", "x", False), (28, 33, 2, "full", "xyz", False),
+    (29, 31, 3, "diag", "z", True), (60, 62, 1, "full", "xy", False), (0, 6, 70, "full", "xyz", False)])
+def test_matvec(device, jmin, jmax, ncols, kind, field, cplx, precision, tol):
+    import torch
+    kop = KronOperator(_basis(jmin, jmax, cplx), *_tensors(kind))
+    dp = DeviceKronPlan(kop)
+    assert dp.kernel == "prim"
+    fields = [np.array([FIELDS[field]])] * len(kop.carts)
+    X = _rows(kop.n, ncols, 1)
+    ref = kop.matvec(X, kop.field_products([F[0] for F in fields]))
+    # rows with a longer stride, NaN between them
+    x = torch.full((ncols, kop.n + 3), float("nan"), dtype=torch.complex128, device=device)
+    y = torch.full_like(x, 7.0)
+    x[:, :kop.n] = torch.from_numpy(X).to(device)
+    fp = torch.from_numpy(slot_products(kop, fields)[0]).to(device)
+    dp.matvec(x[:, :kop.n], y[:, :kop.n], fp, precision=precision)
+    got = y.cpu().numpy()
+    assert np.abs(got[:, :kop.n] - ref).max() <= tol * np.abs(ref).max()
+    assert np.all(got[:, kop.n:] == 7.0)
+
+
+@pytest.mark.parametrize("krylov", [0, 1, 5, 12])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_propagation_equals_dense_form(device, krylov, precision):
+    """Six steps with a zero-field step and another field pattern in each,
+    an unnormalised row and a basis state, <cos^2> after every step: amplitudes,
+    observables and (adaptive) Krylov dimensions of the two forms."""
+    import torch
+    bas = _basis(0, 7, False)
+    kop = KronOperator(bas, *large_top_tensors())
+    kc = KronOperator(bas, [np.diag([0.0, 0.0, 1.0])], [1.0])
+    E = 3e9 * np.array([[1, 0, 0], [0.6, 0.8, 0], [0, 0, 0], [0, 0, 1.0], [0.3, -0.4, 0.5], [0, 1, 0]])
+    fp = slot_products(kop, [E, E])
+    ofp = slot_products(kc, [np.array([[0.0, 0.0, 1.0]])])[0]
+    X = _rows(kop.n, 4, 2)
+    X /= np.linalg.norm(X, axis=1)[:, None]
+    X[1] *= 2.5
+    X[2] = 0
+    X[2, 7] = 1.0
+    f = -0.002j
+    out = {}
+    for kern in ("prim", "gemm"):
+        dp, dc = DeviceKronPlan(kop), DeviceKronPlan(kc)
+        dp.set_kernel(kern)
+        dc.set_kernel(kern)
+        psi = torch.from_numpy(X).to(device)
+        ex = torch.empty((6, 4), dtype=torch.complex128, device=device)
+        es = torch.empty(6, dtype=torch.complex128, device=device)
+        ku = torch.full((6, 4), -1, dtype=torch.int32, device=device)
+        st = torch.full((4,), -1, dtype=torch.int32, device=device)
+        for a in (0, 3):   # two calls: the second starts from the first one's lists and workspace
+            dp.propagate(psi, fp[a:a + 3], f, phase=dp.phases(f), krylov_fixed=krylov, precision=precision, obs=dc,
+                         obs_fprod=ofp, expect=ex[a:a + 3], expect_sum=es[a:a + 3], kused=ku[a:a + 3], status=st)
+        out[kern] = [t.cpu().numpy() for t in (psi, ex, es, ku, st)]
+    a, b = out["prim"], out["gemm"]
+    tol = 1e-11 if precision == "fp64" else 4e-6
+    for i in range(3):
+        assert np.abs(a[i] - b[i]).max() <= tol * max(1.0, np.abs(b[i]).max())
+    if precision == "fp64":
+        assert np.array_equal(a[3], b[3])
+    assert np.array_equal(a[3] == 0, b[3] == 0) and np.array_equal(a[4], b[4])
+
+
+def test_wavepacket_independent_of_batch(device):
+    """A wavepacket's amplitudes do not depend on the others: alone and among
+    nine, bit for bit."""
+    import torch
+    kop = KronOperator(_basis(0, 8, False), *large_top_tensors())
+    fp = slot_products(kop, [np.array([[3e9, 1e9, -2e9]] * 2)] * 2)
+    X = _rows(kop.n, 9, 3)
+    X /= np.linalg.norm(X, axis=1)[:, None]
+    dp = DeviceKronPlan(kop)
+
+    def run(rows):
+        psi = torch.from_numpy(np.ascontiguousarray(rows)).to(device)
+        dp.propagate(psi, fp, -0.002j, phase=dp.phases(-0.002j), krylov_fixed=12)
+        return psi.cpu().numpy()
+
+    full = run(X)
+    for i in (0, 4, 8):
+        assert np.array_equal(run(X[i:i + 1])[0], full[i])
+
+
+def test_factors_from_cartens(device):
+    """A sum of tensors built on a rotor basis keeps the primitive-basis form
+    through KronOperator.from_cartens; a tensor whose K blocks were changed
+    afterwards falls back to the dense form."""
+    from richmol_amd.molecules import large_top_tensors as lt
+    bas = _basis(0, 4, False)
+    tens, scales = lt()
+    T = [rot.tensor(t, bas) * s for t, s in zip(tens, scales)]
+    for t in T:
+        t.field([1e8, 2e8, -3e8])
+    kop, fprods = KronOperator.from_cartens(T[0] + T[1])
+    assert kop.factors is not None
+    X = _rows(kop.n, 2, 4)
+    import torch
+    x = torch.from_numpy(X).to(device)
+    y = torch.empty_like(x)
+    DeviceKronPlan(kop).matvec(x, y, torch.from_numpy(kop.slot_row(fprods)).to(device))
+    ref = kop.matvec(X, fprods)
+    assert np.abs(y.cpu().numpy() - ref).max() <= 1e-13 * np.abs(ref).max()
+    T[1].kmat[(4, 4)][("A", "A")][2] = T[1].kmat[(4, 4)][("A", "A")][2] * 0.5
+    kop2, _ = KronOperator.from_cartens(T[0] + T[1])
+    assert kop2.factors is None
