@@ -9,6 +9,7 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = [os.path.join(PKG_DIR, "csrc", "rm_tdse.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_subspace.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_coop.hip"),
+           os.path.join(PKG_DIR, "csrc", "rm_block.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_kron.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_kprim.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_expokit.hip"),

@@ -164,6 +164,21 @@ struct rm_plan {
   double2* sub_cval = nullptr;   // [nfield][nnz]
   float2* sub_cval32 = nullptr;  // [nfield][nnz] the same in FP32 (FP32-mode matvecs read it)
   std::vector<int64_t> h_sub_rp;
+  // the same entries in slices of up to 64 permuted rows (rm_block.hip): a
+  // slice holds whole subspaces, or 64 rows of one; (first row, rows, pairs of
+  // entries per row, row its columns count from).  Entries in pairs, pair p
+  // of lane l at soff + 64 p + l: columns 16 bits each in units of 16 bytes
+  // of a vector, values real (sreal: every B_s entry real to 1e-14) or complex
+  int4* sslice = nullptr;
+  int64_t* soff = nullptr;
+  int32_t* srow = nullptr;       // [n] slice of each permuted row
+  uint32_t* scol = nullptr;      // [spairs]
+  double* sval = nullptr;        // [nfield][spairs] pairs
+  float* sval32 = nullptr;
+  int64_t spairs = 0;
+  bool sreal = false;
+  std::vector<int32_t> h_srow;
+  std::vector<int64_t> h_soff;   // [slices + 1]
   // per-call scratch of the subspace path
   int32_t* dom = nullptr;        // 2 per column: domain lo, hi
   int64_t dom_cap = 0;
@@ -230,6 +245,13 @@ struct SubOp {
   const double2* cval;     //   values [nslot][nnz]
   const float2* cval32;    //   and their FP32 rounding
   int64_t nnz;
+  const int4* sslice;      // the same in slices (rm_plan::sslice ...)
+  const int64_t* soff;
+  const int32_t* srow;
+  const uint32_t* scol;
+  const void* sval;
+  const void* sval32;
+  int64_t npairs;
   const int32_t* perm;     // permuted row -> original row
   const double2* phase;    // original order, or NULL
   const double2* table;    // [nsteps][nslot] field products of the launch's steps
@@ -325,6 +347,9 @@ struct LongItem {
   int4 item;
   int64_t nent;
   int32_t maxrow, nslot;
+  int32_t variant;   // blk_variant of its slices (0: the kernels of rm_coop.hip)
+  int64_t npairs;    // pairs of its slices
+  int32_t ppairs;    // and of one lane (blk_part_pairs)
 };
 // Long-domain wavepackets (rm_coop.hip): blk one workgroup each in one launch,
 // coop the whole device each (one cooperative launch each).  d_ops, d_blk,

@@ -3,7 +3,8 @@
 //
 // Two launch forms share one kernel body:
 //  * block: one workgroup per wavepacket, many wavepackets per launch, the
-//    workgroup's barriers between the Lanczos reductions;
+//    workgroup's barriers between the Lanczos reductions -- for domains that
+//    k_blk (rm_block.hip) does not take;
 //  * cooperative: every workgroup of the device on one wavepacket (one
 //    cooperative launch per wavepacket, all workgroups resident), grid
 //    barriers between the reductions -- for a few wavepackets on long domains.
@@ -51,7 +52,6 @@ constexpr int mg_of() { return F32 ? 4 : 2; }
 template <bool F32>
 constexpr int umg_of() { return F32 ? 4 : 8; }
 constexpr int GL = 32;           // Gram matrix order held in LDS (adaptive)
-constexpr int XL_ROWS = 2048;    // block form: matvec input staged in LDS up to this many rows
 constexpr unsigned SPIN_LIMIT = 1u << 22;   // polls of a grid barrier before the launch gives up
 constexpr int BAR_LINES = 8;                // arrival counters of a grid barrier
 constexpr int BAR_STRIDE = 32;              // u64 between counters (one 256-byte line each)
@@ -291,26 +291,9 @@ __device__ __forceinline__ double inv_beta(double beta) {
   return ib;
 }
 
-// Dynamic LDS of the XL stage (matvec input and row offsets), rounded up to
-// 256 bytes: the LV vectors follow it.
-template <bool F32>
-constexpr size_t xl_bytes() {
-  return ((F32 ? sizeof(float2) : sizeof(double2)) * XL_ROWS + sizeof(int) * (XL_ROWS + 1) + 255) & ~(size_t)255;
-}
-
-// XL (block form, domains of at most XL_ROWS rows): the matvec input is
-// staged in LDS by the threads that write it, and gathered from there.
-// LV (with XL): the Krylov basis and the step's vectors (V, W, Y, S, P) sit
-// in LDS after the stage instead of the workgroup's global region (the host
-// takes it when they fit); the step's operator array stays global.
-template <int MODE, bool FIXED, bool F32, bool XL = false, bool LV = false>
+template <int MODE, bool FIXED, bool F32>
 __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
   using XT = typename XType<F32>::T;
-  static_assert(!XL || MODE == BLOCK, "LDS-staged input is for the block form");
-  static_assert(!LV || XL, "LDS vectors come with the LDS-staged input");
-  extern __shared__ char s_dyn[];
-  XT* s_x = (XT*)s_dyn;                                   // [XL_ROWS] matvec input
-  int* s_rp = (int*)(s_dyn + sizeof(XT) * XL_ROWS);       // [XL_ROWS + 1] row offsets from e_lo
   constexpr int CT = ct_of<MODE>();
   constexpr int CWV = CT / 64;
   constexpr bool REG = MODE == GRID_REG;
@@ -333,18 +316,15 @@ __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
   const int sub = lane % LPR, rw = lane / LPR;
   const int kc = a.kcap;
   char* base = a.ws + (MODE == BLOCK ? (int64_t)blockIdx.x * a.wg_bytes : 0);
-  char* vbase = LV ? s_dyn + xl_bytes<F32>() : base;      // the vectors' region (offsets below offA)
-  double2* V = (double2*)(vbase + a.offV);
-  double2* Wb = (double2*)(vbase + a.offWb);
-  float2* Wf = (float2*)(vbase + a.offWf);
-  double2* Y = (double2*)(vbase + a.offY);
-  double2* S = (double2*)(vbase + a.offS);
-  double2* P = (double2*)(vbase + a.offP);
+  double2* V = (double2*)(base + a.offV);
+  double2* Wb = (double2*)(base + a.offWb);
+  float2* Wf = (float2*)(base + a.offWf);
+  double2* Y = (double2*)(base + a.offY);
+  double2* S = (double2*)(base + a.offS);
+  double2* P = (double2*)(base + a.offP);
   XT* Ast = (XT*)(base + a.offA);
   const XT* Xin;
-  if constexpr (XL)
-    Xin = s_x;
-  else if constexpr (F32)
+  if constexpr (F32)
     Xin = Wf;
   else
     Xin = Wb;
@@ -377,15 +357,8 @@ __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
       S[i] = op.psi[(int64_t)b * op.ld + orig];
       P[i] = op.phase ? op.phase[orig] : make_double2(1.0, 0.0);
     }
-    if constexpr (XL)
-      for (int64_t i = t0; i <= len; i += nthr) s_rp[i] = (int)(op.rp[lo + i] - e_lo);
-    // first entry of domain row r (XL: from LDS, published by the first barrier of a step)
-    auto row_start = [&](int r) __attribute__((always_inline)) -> int64_t {
-      if constexpr (XL)
-        return e_lo + s_rp[r];
-      else
-        return op.rp[lo + r];
-    };
+    // first entry of domain row r
+    auto row_start = [&](int r) __attribute__((always_inline)) -> int64_t { return op.rp[lo + r]; };
     // this lane's row in the matvec (REG: the wave's only row group) and its entries
     const int rreg = gw * RPW + rw;
     int64_t ebeg = 0, eend = 0;
@@ -477,7 +450,6 @@ __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
         V[i] = v;
         Wb[i] = v;
         if constexpr (F32) Wf[i] = to_x<true>(v);
-        if constexpr (XL) s_x[i] = to_x<F32>(v);
       }
       sync_all<MODE>(a, ss, &s_ab);
 
@@ -498,11 +470,7 @@ __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
           w.y = row_sum16(w.y);
           if (sub == 0 && r < len) {
             w = cscale(ib, w);
-            double2 wr;
-            if constexpr (XL && !F32)
-              wr = s_x[r];   // W itself
-            else
-              wr = Wb[r];
+            const double2 wr = Wb[r];
             const double2 v = cscale(ib, wr);
             Vit[r] = v;
             Y[r] = w;
@@ -602,7 +570,6 @@ __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
           if (it > 0) wn = csub(wn, cscale(beta, Vprev[i]));
           Wb[i] = wn;
           if constexpr (F32) Wf[i] = to_x<true>(wn);
-          if constexpr (XL) s_x[i] = to_x<F32>(wn);
           bs += wn.x * wn.x + wn.y * wn.y;
         }
         k = it + 1;
@@ -675,7 +642,6 @@ __global__ __launch_bounds__(ct_of<MODE>()) void k_long(LongArgs a) {
           Wb[i] = v;
           Vk[i] = v;
           if constexpr (F32) Wf[i] = to_x<true>(v);
-          if constexpr (XL) s_x[i] = to_x<F32>(v);
         }
         if (!FIXED) {
           // Gram column of the restart vector, explicit dots
@@ -744,50 +710,39 @@ struct LongScratch {
   size_t bytes = 0;
 };
 
-template <int MODE, bool FIXED, bool F32, bool XL, bool LV = false>
-hipError_t launch_r(LongArgs& a, int grid, size_t lds, hipStream_t s) {
+template <int MODE, bool FIXED, bool F32>
+hipError_t launch_r(LongArgs& a, int grid, hipStream_t s) {
   if (MODE == BLOCK) {
-    hipLaunchKernelGGL((k_long<MODE, FIXED, F32, XL, LV>), dim3(grid), dim3(ct_of<MODE>()), lds, s, a);
+    hipLaunchKernelGGL((k_long<MODE, FIXED, F32>), dim3(grid), dim3(ct_of<MODE>()), 0, s, a);
     return hipGetLastError();
   }
   void* args[] = {&a};
-  return hipLaunchCooperativeKernel((const void*)k_long<MODE, FIXED, F32, XL>, dim3(grid), dim3(ct_of<MODE>()),
-                                    args, lds, s);
+  return hipLaunchCooperativeKernel((const void*)k_long<MODE, FIXED, F32>, dim3(grid), dim3(ct_of<MODE>()), args, 0,
+                                    s);
 }
 
-template <int MODE, bool XL = false, bool LV = false>
-hipError_t launch_m(LongArgs& a, int grid, bool f32, size_t lds, hipStream_t s) {
+template <int MODE>
+hipError_t launch_m(LongArgs& a, int grid, bool f32, hipStream_t s) {
   const bool fixed = a.fixed_m > 0;
-  if (fixed)
-    return f32 ? launch_r<MODE, true, true, XL, LV>(a, grid, lds, s)
-               : launch_r<MODE, true, false, XL, LV>(a, grid, lds, s);
-  return f32 ? launch_r<MODE, false, true, XL, LV>(a, grid, lds, s)
-             : launch_r<MODE, false, false, XL, LV>(a, grid, lds, s);
+  if (fixed) return f32 ? launch_r<MODE, true, true>(a, grid, s) : launch_r<MODE, true, false>(a, grid, s);
+  return f32 ? launch_r<MODE, false, true>(a, grid, s) : launch_r<MODE, false, false>(a, grid, s);
 }
 
 // Workgroups of one form the device holds at once (the smallest over its
-// instantiations) with lds bytes of dynamic LDS each; 0 when one of them
-// cannot run with that much.
-template <int MODE, bool XL = false, bool LV = false>
-hipError_t resident(int n_cu, size_t lds, int* grid) {
-  const void* ks[] = {(const void*)k_long<MODE, true, true, XL, LV>, (const void*)k_long<MODE, true, false, XL, LV>,
-                      (const void*)k_long<MODE, false, true, XL, LV>, (const void*)k_long<MODE, false, false, XL, LV>};
+// instantiations), at least one per CU.
+template <int MODE>
+hipError_t max_resident(int n_cu, int* grid) {
+  const void* ks[] = {(const void*)k_long<MODE, true, true>, (const void*)k_long<MODE, true, false>,
+                      (const void*)k_long<MODE, false, true>, (const void*)k_long<MODE, false, false>};
   int occ = INT32_MAX;
   for (const void* k : ks) {
     int o = 0;
-    hipError_t e = occupancy(k, ct_of<MODE>(), lds, &o);
+    hipError_t e = occupancy(k, ct_of<MODE>(), 0, &o);
     if (e != hipSuccess) return e;
     occ = std::min(occ, o);
   }
-  *grid = occ * n_cu;
+  *grid = std::max(occ, 1) * n_cu;
   return hipSuccess;
-}
-
-template <int MODE, bool XL = false>
-hipError_t max_resident(int n_cu, size_t lds, int* grid) {
-  hipError_t e = resident<MODE, XL>(n_cu, lds, grid);
-  *grid = std::max(*grid, n_cu);
-  return e;
 }
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -825,15 +780,10 @@ int long_run(void** scratch, const SubOp* d_ops, const int4* d_blk, const std::v
              int32_t maxorder, double tol, bool f32, int n_cu, hipStream_t s, int32_t abort_preset,
              const SubOp* op0, int32_t coop_grid) {
   if (blk.empty() && coop.empty()) return RM_OK;
-  int gres_r = 1, gres_m = 1, gres_b = 1, gres_x = 1;
-  HIPCHK((max_resident<GRID_REG>(n_cu, 0, &gres_r)));
-  HIPCHK((max_resident<GRID_MEM>(n_cu, 0, &gres_m)));
-  HIPCHK((max_resident<BLOCK>(n_cu, 0, &gres_b)));
-  // block items on domains of at most XL_ROWS rows come first (staged in LDS)
-  size_t nx = 0;
-  while (nx < blk.size() && blk[nx].item.z <= XL_ROWS) ++nx;
-  const size_t lds_x = (f32 ? sizeof(float2) : sizeof(double2)) * XL_ROWS + sizeof(int) * (XL_ROWS + 1);
-  if (nx) HIPCHK((max_resident<BLOCK, true>(n_cu, lds_x, &gres_x)));
+  int gres_r = 1, gres_m = 1, gres_b = 1;
+  HIPCHK(max_resident<GRID_REG>(n_cu, &gres_r));
+  HIPCHK(max_resident<GRID_MEM>(n_cu, &gres_m));
+  HIPCHK(max_resident<BLOCK>(n_cu, &gres_b));
   gres_r = std::min(gres_r, n_cu);
   gres_m = std::min(gres_m, n_cu);
   const bool fixed = fixed_m > 0;
@@ -851,7 +801,7 @@ int long_run(void** scratch, const SubOp* d_ops, const int4* d_blk, const std::v
       need_A |= it.nslot > 1;
     }
     const size_t region = region_layout(ab, lmax, emax, kcap, f32, need_A);
-    nwg = (int)std::max(std::min<int64_t>((int64_t)nx, gres_x), std::min<int64_t>((int64_t)(blk.size() - nx), gres_b));
+    nwg = (int)std::min<int64_t>((int64_t)blk.size(), gres_b);
     ab.wg_bytes = (int64_t)region;
     ab.lmax = lmax;
     b_bytes = region * (size_t)nwg;
@@ -915,36 +865,11 @@ int long_run(void** scratch, const SubOp* d_ops, const int4* d_blk, const std::v
     a->maxorder = maxorder;
     a->tol = tol;
   }
-  if (nx) {
+  if (!blk.empty()) {
     ab.ws = wb;
     ab.items = d_blk;
-    ab.nitems = (int32_t)nx;
-    // the vectors of the longest of these domains in LDS beside the stage,
-    // when the kernel still fits a CU with them (fixed Krylov dimensions and
-    // domains of up to ~500 rows); the region layout's vector part ends at offA
-    int64_t lx = 0;
-    for (size_t i = 0; i < nx; ++i) lx = std::max<int64_t>(lx, blk[i].item.z);
-    LongArgs lv = ab;
-    const size_t vbytes = region_layout(lv, lx, 1, kcap, f32, false);
-    const size_t lds_v = (f32 ? xl_bytes<true>() : xl_bytes<false>()) + vbytes;
-    int gres_v = 0;
-    if (lds_v <= LDS_BYTES) HIPCHK((resident<BLOCK, true, true>(n_cu, lds_v, &gres_v)));
-    if (gres_v > 0) {
-      // same offsets as the global region's vectors (lmax differs: a layout of their own)
-      lv.ws = wb;
-      lv.offA = ab.offA;
-      lv.wg_bytes = ab.wg_bytes;
-      lv.lmax = lx;
-      HIPCHK((launch_m<BLOCK, true, true>(lv, (int)std::min<int64_t>((int64_t)nx, gres_v), f32, lds_v, s)));
-    } else {
-      HIPCHK((launch_m<BLOCK, true>(ab, (int)std::min<int64_t>((int64_t)nx, gres_x), f32, lds_x, s)));
-    }
-  }
-  if (blk.size() > nx) {
-    ab.ws = wb;
-    ab.items = d_blk + nx;
-    ab.nitems = (int32_t)(blk.size() - nx);
-    HIPCHK((launch_m<BLOCK>(ab, (int)std::min<int64_t>((int64_t)ab.nitems, gres_b), f32, 0, s)));
+    ab.nitems = (int32_t)blk.size();
+    HIPCHK(launch_m<BLOCK>(ab, (int)std::min<int64_t>((int64_t)ab.nitems, gres_b), f32, s));
   }
   ac.ws = wc;
   ac.wg_bytes = 0;
@@ -966,9 +891,9 @@ int long_run(void** scratch, const SubOp* d_ops, const int4* d_blk, const std::v
                        LRING * 4 * gmax, abort_preset);
     HIPCHK(hipGetLastError());
     if (reg)
-      HIPCHK((launch_m<GRID_REG>(ac, grid, f32, 0, s)));
+      HIPCHK(launch_m<GRID_REG>(ac, grid, f32, s));
     else
-      HIPCHK((launch_m<GRID_MEM>(ac, grid, f32, 0, s)));
+      HIPCHK(launch_m<GRID_MEM>(ac, grid, f32, s));
   }
   return RM_OK;
 }

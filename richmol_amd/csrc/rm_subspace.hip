@@ -24,7 +24,7 @@
 #include <mutex>
 #include <numeric>
 
-#include "rm_common.h"
+#include "rm_block.h"
 
 namespace {
 
@@ -971,6 +971,74 @@ std::vector<double2> entry_values(const rm_plan* p) {
   return B;
 }
 
+// The sliced form of the permuted CSR arrays (rm_block.hip).
+int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
+                const std::vector<double2>& cval) {
+  const int64_t n = p->n, nnz = p->nnz;
+  const int32_t nf = std::max(p->nfield, 1);
+  p->sreal = true;
+  for (const double2& v : cval)
+    if (std::fabs(v.y) > 1e-14 * std::fabs(v.x)) {
+      p->sreal = false;
+      break;
+    }
+  std::vector<int4> sl;
+  for (int32_t c = 0; c < p->nsub; ++c) {
+    const int32_t lo = p->h_sub_start[c], len = p->h_sub_end[c] - lo;
+    if (len <= 64 && !sl.empty() && sl.back().w == sl.back().x && sl.back().y + len <= 64 &&
+        sl.back().x + sl.back().y == lo && p->h_sub_end[p->h_sub_label_perm[sl.back().x]] <= lo) {
+      sl.back().y += len;   // with the small subspaces before it
+      continue;
+    }
+    for (int32_t r = 0; r < len; r += 64) sl.push_back(make_int4(lo + r, std::min(64, len - r), 0, lo));
+  }
+  std::vector<int64_t> off(1, 0);
+  p->h_srow.assign((size_t)n, 0);
+  for (size_t i = 0; i < sl.size(); ++i) {
+    int64_t w = 0;
+    for (int32_t r = sl[i].x; r < sl[i].x + sl[i].y; ++r) {
+      w = std::max(w, rp[r + 1] - rp[r]);
+      p->h_srow[r] = (int32_t)i;
+    }
+    // a subspace longer than the block kernel takes: no entries
+    const int32_t c = p->h_sub_label_perm[sl[i].x];
+    sl[i].z = p->h_sub_end[c] - p->h_sub_start[c] <= BLK_MAX_ROWS ? (int32_t)((w + 1) / 2) : 0;
+    off.push_back(off.back() + 64 * (int64_t)sl[i].z);
+  }
+  const int64_t np = off.back();
+  const int q = p->sreal ? 2 : 4;   // values of a pair
+  std::vector<uint32_t> col((size_t)std::max<int64_t>(np, 1), 0);
+  std::vector<double> val((size_t)(nf * np * q), 0.0);
+  for (size_t i = 0; i < sl.size(); ++i)
+    for (int32_t l = 0; l < sl[i].y && sl[i].z > 0; ++l) {
+      const int64_t e0 = rp[sl[i].x + l], len = rp[sl[i].x + l + 1] - e0;
+      for (int64_t j = 0; j < len; ++j) {
+        const int64_t at = off[i] + 64 * (j / 2) + l;
+        col[(size_t)at] |= (uint32_t)((ccol[e0 + j] - sl[i].w) * 16) << (16 * (j & 1));
+        for (int32_t s = 0; s < nf; ++s) {
+          const double2 v = cval[(size_t)s * nnz + e0 + j];
+          double* d = val.data() + (size_t)((s * np + at) * q);
+          if (p->sreal) {
+            d[j & 1] = v.x;
+          } else {
+            d[2 * (j & 1)] = v.x;
+            d[2 * (j & 1) + 1] = v.y;
+          }
+        }
+      }
+    }
+  const std::vector<float> val32(val.begin(), val.end());
+  int rc = RM_OK;
+  if ((rc = upload(&p->sslice, sl.data(), (int64_t)sl.size())) || (rc = upload(&p->soff, off.data(), (int64_t)off.size())) ||
+      (rc = upload(&p->srow, p->h_srow.data(), n)) || (rc = upload(&p->scol, col.data(), (int64_t)col.size())) ||
+      (rc = upload(&p->sval, val.data(), (int64_t)val.size())) ||
+      (rc = upload(&p->sval32, val32.data(), (int64_t)val32.size())))
+    return rc;
+  p->spairs = np;
+  p->h_soff.swap(off);
+  return RM_OK;
+}
+
 // The B_s as CSR in permuted row and column order (the cooperative kernel's
 // operator); rows keep the order of their entries.
 int csr_build(rm_plan* p, const std::vector<double2>& B) {
@@ -1003,6 +1071,7 @@ int csr_build(rm_plan* p, const std::vector<double2>& B) {
       (rc = upload(&p->sub_cval, cval.data(), (int64_t)nf * nnz)) ||
       (rc = upload(&p->sub_cval32, cval32.data(), (int64_t)nf * nnz)))
     return rc;
+  if ((rc = slice_build(p, rp, ccol, cval))) return rc;
   p->h_sub_rp.swap(rp);
   return RM_OK;
 }
@@ -1226,6 +1295,8 @@ struct SubScratch {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   void* long_ws = nullptr;   // the long-domain kernels' workspace (rm_coop.hip)
+  void* blk_ws = nullptr;    // the block kernel's (rm_block.hip)
+  size_t blk_ws_bytes = 0;
   // launch classes run concurrently on auxiliary streams (default priority)
   hipStream_t aux[NCLASS + 1] = {};
   hipEvent_t fork = nullptr;
@@ -1253,6 +1324,7 @@ void scratch_release(SubScratch* sc) {
   if (sc->ws) (void)hipFree(sc->ws);
   if (sc->kept_dev) (void)hipFree(sc->kept_dev);
   coop_scratch_release(sc->long_ws);
+  if (sc->blk_ws) (void)hipFree(sc->blk_ws);
   for (int i = 0; i <= NCLASS; ++i) {
     if (sc->aux[i]) {
       (void)hipStreamSynchronize(sc->aux[i]);
@@ -1371,7 +1443,18 @@ int launch_all(SubScratch* sc, const SubArgs& a0, const int4* const (&items)[NCL
   }
   hipStream_t bs = s;
   if (!blk.empty() && (rc = next_stream(&bs))) return rc;
-  rc = long_run(&sc->long_ws, a0.ops, d_blk, blk, d_coop, coop, kcap, fixed_m, maxorder, tol, f32, n_cu, bs,
+  // the block kernel's items by variant, then those of the long-domain kernels
+  size_t nb = 0;
+  while (nb < blk.size() && blk[nb].variant != 0) {
+    size_t e = nb;
+    while (e < blk.size() && blk[e].variant == blk[nb].variant) ++e;
+    rc = blk_run(&sc->blk_ws, &sc->blk_ws_bytes, a0.ops, a0.ops ? nullptr : &a0.op0, d_blk, blk, nb, e - nb,
+                 blk[nb].variant, kcap, fixed_m, maxorder, tol, f32, n_cu, bs);
+    if (rc) return rc;
+    nb = e;
+  }
+  const std::vector<LongItem> rest(blk.begin() + nb, blk.end());
+  rc = long_run(&sc->long_ws, a0.ops, d_blk + nb, rest, d_coop, coop, kcap, fixed_m, maxorder, tol, f32, n_cu, bs,
                 abort_preset, a0.ops ? nullptr : &a0.op0, tn.coop_grid);
   if (rc) return rc;
   if (fork && !blk.empty()) HIPCHK(hipEventRecord(sc->join[nused - 1], bs));
@@ -1503,6 +1586,13 @@ SubOp plan_op(const rm_plan* p) {
   op.ccol = p->sub_ccol;
   op.cval = p->sub_cval;
   op.cval32 = p->sub_cval32;
+  op.sslice = p->sslice;
+  op.soff = p->soff;
+  op.srow = p->srow;
+  op.scol = p->scol;
+  op.sval = p->sval;
+  op.sval32 = p->sval32;
+  op.npairs = p->spairs;
   op.nnz = p->nnz;
   op.perm = p->sub_perm;
   op.n = (int32_t)p->n;
@@ -1596,16 +1686,20 @@ LongItem long_item(const rm_plan* p, int col, int lo, int len, int op) {
   for (int64_t r = lo; r < (int64_t)lo + len; ++r) mr = std::max(mr, p->h_sub_rp[r + 1] - p->h_sub_rp[r]);
   it.maxrow = (int32_t)std::min<int64_t>(mr, INT32_MAX);
   it.nslot = p->nfield;
+  const int32_t s0 = p->h_srow[lo], s1 = p->h_srow[lo + len - 1];
+  it.npairs = p->h_soff[s1 + 1] - p->h_soff[s0];
+  int64_t mp = 0;
+  for (int32_t i = s0; i <= s1; ++i) mp = std::max<int64_t>(mp, (p->h_soff[i + 1] - p->h_soff[i]) / 64);
+  it.ppairs = blk_part_pairs(s1 - s0 + 1, mp);
+  it.variant = len <= BLK_MAX_ROWS ? blk_variant(s1 - s0 + 1, p->sreal) : 0;
   return it;
 }
 
-// Most work first, with the domains the block kernel stages in LDS
-// (RM_XL_ROWS rows at most) ahead of the longer ones.
-constexpr int RM_XL_ROWS = 2048;
+// By launch variant and pairs per lane, most work first.
 void sort_long(std::vector<LongItem>& v) {
   std::stable_sort(v.begin(), v.end(), [](const LongItem& x, const LongItem& y) {
-    const bool lx = x.item.z <= RM_XL_ROWS, ly = y.item.z <= RM_XL_ROWS;
-    if (lx != ly) return lx;
+    if (x.variant != y.variant) return x.variant > y.variant;
+    if (x.variant != 0 && x.ppairs != y.ppairs) return x.ppairs > y.ppairs;
     return x.nent > y.nent;
   });
 }
@@ -2043,13 +2137,12 @@ static int collect_jobs(const char* who, const rm_job* jobs, int32_t njobs, int3
     for (size_t t = 0; t < ix.size(); ++t) sorted[t] = cls[c][ix[t]];
     cls[c].swap(sorted);
   }
-  // long domains: one workgroup each (block kernel), LDS-staged domains
-  // first, most work first
+  // long domains: one workgroup each, by launch variant, most work first
   std::vector<size_t> ix(blk.size());
   std::iota(ix.begin(), ix.end(), 0);
   std::stable_sort(ix.begin(), ix.end(), [&](size_t x, size_t y) {
-    const bool lx = blk[x].item.z <= RM_XL_ROWS, ly = blk[y].item.z <= RM_XL_ROWS;
-    if (lx != ly) return lx;
+    if (blk[x].variant != blk[y].variant) return blk[x].variant > blk[y].variant;
+    if (blk[x].variant != 0 && blk[x].ppairs != blk[y].ppairs) return blk[x].ppairs > blk[y].ppairs;
     return blk_work[x] > blk_work[y];
   });
   std::vector<LongItem> sorted(ix.size());
