@@ -176,7 +176,7 @@ struct rm_plan {
   double* sval = nullptr;        // [nfield][spairs] pairs
   float* sval32 = nullptr;
   int64_t spairs = 0;
-  bool sreal = false;
+  bool sreal = false, ssym = false;   // ssym: real and symmetric
   std::vector<int32_t> h_srow;
   std::vector<int64_t> h_soff;   // [slices + 1]
   // per-call scratch of the subspace path
@@ -252,6 +252,7 @@ struct SubOp {
   const void* sval;
   const void* sval32;
   int64_t npairs;
+  int32_t sflags;          // bit 0: every B_s real and symmetric
   const int32_t* perm;     // permuted row -> original row
   const double2* phase;    // original order, or NULL
   const double2* table;    // [nsteps][nslot] field products of the launch's steps

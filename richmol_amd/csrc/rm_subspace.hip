@@ -25,25 +25,12 @@
 #include <numeric>
 
 #include "rm_block.h"
+#include "rm_wave.h"
 
 namespace {
 
 constexpr int NSR = 2;                         // field slots held in registers
 constexpr size_t SUB_LDS_BASIS = 32 * 1024;    // LDS budget of a wave's Krylov basis
-
-struct SubArgs {
-  const SubOp* ops;        // the jobs, or NULL: the one job is op0
-  SubOp op0;               // the job of a single-job launch, by value (no staging)
-  const int4* items;       // (column, lo, len, op), one wavepacket each
-  int32_t nitems;
-  double2* basis;          // per wave kcap * 64R (global-basis variant)
-  double2* gram;           // per wave kcap * kcap (adaptive)
-  double2* cscr;           // per wave 2 * kcap (adaptive)
-  int32_t kcap, fixed_m, maxorder;
-  double tol;
-  int32_t max_waves;       // > 0: at most this many waves (the launch's workspace holds no more)
-  int32_t obs;             // 1: some job reads an observable (k_sub_prop: LDS for the state)
-};
 
 // One wave per wavepacket, R rows per lane (domain <= 64 R rows).  WM > 0:
 // the ELL entries of the lane's rows (width <= WM) are held in registers
@@ -982,6 +969,20 @@ int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<in
       p->sreal = false;
       break;
     }
+  // symmetric to 1e-14 (rows keep the ascending column order of the original within a subspace)
+  p->ssym = p->sreal;
+  for (int64_t r = 0; r < n && p->ssym; ++r)
+    for (int64_t e = rp[r]; e < rp[r + 1] && p->ssym; ++e) {
+      const int64_t c = ccol[e];
+      const int32_t* b = ccol.data() + rp[c];
+      const int32_t* t = ccol.data() + rp[c + 1];
+      const int32_t* f = std::lower_bound(b, t, (int32_t)r);
+      const int64_t e2 = f != t && *f == r ? f - ccol.data() : -1;
+      for (int32_t s = 0; s < nf; ++s) {
+        const double x = cval[(size_t)s * nnz + e].x, y = e2 >= 0 ? cval[(size_t)s * nnz + e2].x : 0.0;
+        if (std::fabs(x - y) > 1e-14 * std::max(std::fabs(x), std::fabs(y))) p->ssym = false;
+      }
+    }
   std::vector<int4> sl;
   for (int32_t c = 0; c < p->nsub; ++c) {
     const int32_t lo = p->h_sub_start[c], len = p->h_sub_end[c] - lo;
@@ -1012,9 +1013,11 @@ int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<in
   for (size_t i = 0; i < sl.size(); ++i)
     for (int32_t l = 0; l < sl[i].y && sl[i].z > 0; ++l) {
       const int64_t e0 = rp[sl[i].x + l], len = rp[sl[i].x + l + 1] - e0;
-      for (int64_t j = 0; j < len; ++j) {
+      const uint32_t self = (uint32_t)((sl[i].x + l - sl[i].w) * 16);   // padding: the row's own column
+      for (int64_t j = 0; j < 2 * (int64_t)sl[i].z; ++j) {
         const int64_t at = off[i] + 64 * (j / 2) + l;
-        col[(size_t)at] |= (uint32_t)((ccol[e0 + j] - sl[i].w) * 16) << (16 * (j & 1));
+        col[(size_t)at] |= (j < len ? (uint32_t)((ccol[e0 + j] - sl[i].w) * 16) : self) << (16 * (j & 1));
+        if (j >= len) continue;
         for (int32_t s = 0; s < nf; ++s) {
           const double2 v = cval[(size_t)s * nnz + e0 + j];
           double* d = val.data() + (size_t)((s * np + at) * q);
@@ -1041,20 +1044,20 @@ int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<in
 
 // The B_s as CSR in permuted row and column order (the cooperative kernel's
 // operator); rows keep the order of their entries.
-int csr_build(rm_plan* p, const std::vector<double2>& B) {
-  if (p->sub_rp) return RM_OK;
+void csr_host(const rm_plan* p, const std::vector<double2>& B, std::vector<int64_t>& rp, std::vector<int32_t>& ccol,
+              std::vector<double2>& cval) {
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   const std::vector<int32_t>& perm = p->h_sub_perm;
   std::vector<int32_t> iperm((size_t)n);
   for (int64_t ip = 0; ip < n; ++ip) iperm[perm[ip]] = (int32_t)ip;
-  std::vector<int64_t> rp((size_t)n + 1, 0);
+  rp.assign((size_t)n + 1, 0);
   for (int64_t ip = 0; ip < n; ++ip) {
     const int32_t i = perm[ip];
     rp[ip + 1] = rp[ip] + (p->h_row_ptr[i + 1] - p->h_row_ptr[i]);
   }
-  std::vector<int32_t> ccol((size_t)nnz);
-  std::vector<double2> cval((size_t)nf * (size_t)nnz);
+  ccol.resize((size_t)nnz);
+  cval.resize((size_t)nf * (size_t)nnz);
   for (int64_t ip = 0; ip < n; ++ip) {
     const int32_t i = perm[ip];
     const int64_t r0 = p->h_row_ptr[i], len = p->h_row_ptr[i + 1] - r0;
@@ -1064,6 +1067,12 @@ int csr_build(rm_plan* p, const std::vector<double2>& B) {
         cval[(size_t)s * nnz + (size_t)(rp[ip] + j)] = B[(size_t)s * nnz + (size_t)(r0 + j)];
     }
   }
+}
+
+int csr_upload(rm_plan* p, std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
+               const std::vector<double2>& cval) {
+  const int64_t n = p->n, nnz = p->nnz;
+  const int32_t nf = std::max(p->nfield, 1);
   std::vector<float2> cval32(cval.size());
   for (size_t q = 0; q < cval.size(); ++q) cval32[q] = make_float2((float)cval[q].x, (float)cval[q].y);
   int rc = RM_OK;
@@ -1071,9 +1080,17 @@ int csr_build(rm_plan* p, const std::vector<double2>& B) {
       (rc = upload(&p->sub_cval, cval.data(), (int64_t)nf * nnz)) ||
       (rc = upload(&p->sub_cval32, cval32.data(), (int64_t)nf * nnz)))
     return rc;
-  if ((rc = slice_build(p, rp, ccol, cval))) return rc;
   p->h_sub_rp.swap(rp);
   return RM_OK;
+}
+
+int csr_build(rm_plan* p, const std::vector<double2>& B) {
+  if (p->sub_rp) return RM_OK;
+  std::vector<int64_t> rp;
+  std::vector<int32_t> ccol;
+  std::vector<double2> cval;
+  csr_host(p, B, rp, ccol, cval);
+  return csr_upload(p, rp, ccol, cval);
 }
 
 // Connected components of the sparsity graph (host union-find), the row
@@ -1157,48 +1174,78 @@ int sub_build(rm_plan* p) {
       return rc;
   }
   p->h_sub_perm.swap(perm);
+  std::vector<int64_t> rp;
+  std::vector<int32_t> ccol;
+  std::vector<double2> cval;
+  csr_host(p, B, rp, ccol, cval);
+  if ((rc = slice_build(p, rp, ccol, cval))) return rc;
   // CSR (row-major, permuted) for the cooperative kernel: if some subspace does not fit
-  if (mx > RM_SUBSPACE_MAX_ROWS && (rc = csr_build(p, B))) return rc;
+  if (mx > RM_SUBSPACE_MAX_ROWS && (rc = csr_upload(p, rp, ccol, cval))) return rc;
   p->sub_w = W;
   p->sub_ready = 1;
   return RM_OK;
 }
 
-// Launch classes (one kernel instantiation each): rows per lane R and where
-// the operator entries live.  A wavepacket's class depends only on its own
-// domain and operator width, so its arithmetic -- and its result, bit for bit
-// -- does not depend on the other wavepackets of the launch.
-//   0: R=1, 1: R=2, 2: R=4 with the operator in registers (ELL width <= 4)
-//   3: R=4, 4: R=8, 5: R=16 reading the operator at every matvec
+// Launch classes (one kernel instantiation each).  A wavepacket's class
+// depends only on its own domain and operator, so its arithmetic -- and its
+// result, bit for bit -- does not depend on the other wavepackets of the launch.
+// One wave per wavepacket, R rows per lane (k_sub_prop):
+//   1: R=2, 2: R=4 with the operator in registers (ELL width <= 4)
+//   9: R=2, 3: R=4, 4: R=8, 5: R=16 reading the operator at every matvec
+// Domains of at most 64 rows (within one slice):
 //   6: two wavepackets per wave (k_sub_pair): fixed Krylov dimension <= 16,
-//      domains <= 32 rows, ELL width <= 4 -- the class-0 items that qualify,
-//      paired with an item of the same operator or with an empty half
+//      domains <= 32 rows, ELL width <= 4, paired with an item of the same
+//      operator or with an empty half
 //   7: the same with a banded domain (every entry within one row of the
 //      diagonal, <= 2 field slots): neighbours by DPP shifts (k_sub_pair BAND)
-//   8: R=1, 9: R=2 reading the operator at every matvec (ELL width > 4)
-constexpr int NCLASS = 10;
+//   0, 8, 12: k_wav, one wavepacket per wave: ELL width <= 4, wider, complex
+//   10, 11, 13: the same, two wavepackets per wave (<= 32 rows)
+//   14: complex, ELL width <= 4: before group_pairs only (goes to 6, 12 or 13)
+constexpr int NCLASS = 15;
 constexpr int PAIR_CLASS = 6;
 constexpr int PAIR_BAND_CLASS = 7;
+constexpr int COMPLEX4_CLASS = 14;
 constexpr int PAIR_MAX_M = 16;
-constexpr int CLASS_R[NCLASS] = {1, 2, 4, 4, 8, 16, 1, 1, 1, 2};
+constexpr int CLASS_R[NCLASS] = {1, 2, 4, 4, 8, 16, 1, 1, 1, 2, 1, 1, 1, 1, 1};
 
-int sub_class(int w, int len) {
-  if (w <= 4) {
-    if (len <= 64) return 0;
-    if (len <= 128) return 1;
-    if (len <= 256) return 2;
-  } else {
-    if (len <= 64) return 8;
-    if (len <= 128) return 9;
-    if (len <= 256) return 3;
-  }
+int sub_class(const rm_plan* p, int lo, int len) {
+  const bool narrow = p->sub_w <= 4;
+  if (len <= 64 && p->h_srow[lo] == p->h_srow[lo + len - 1])
+    return p->sreal ? (narrow ? 0 : 8) : (narrow ? COMPLEX4_CLASS : 12);
+  if (len <= 128) return narrow ? 1 : 9;
+  if (len <= 256) return narrow ? 2 : 3;
   return len <= 512 ? 4 : 5;
+}
+
+// the k_wav launch kind of a class, -1 for the other kernels
+int wav_kind(int c) {
+  switch (c) {
+    case 0: return WAV_S2;
+    case 8: return WAV_S32;
+    case 10: return WAV_P2;
+    case 11: return WAV_P16;
+    case 12: return WAV_SC;
+    case 13: return WAV_PC;
+    default: return -1;
+  }
 }
 
 // Krylov basis in LDS: register classes whose basis fits.
 bool class_basis_lds(int c, int kcap) {
   if (c == PAIR_CLASS || c == PAIR_BAND_CLASS) return true;   // static LDS of k_sub_pair
-  return (c <= 2 || c >= 8) && (size_t)kcap * 64 * CLASS_R[c] * sizeof(double2) <= SUB_LDS_BASIS;
+  return (c <= 2 || c == 9) && (size_t)kcap * 64 * CLASS_R[c] * sizeof(double2) <= SUB_LDS_BASIS;
+}
+
+// Elements (double2) of a class's workspace per wave: basis, Gram matrices, coefficients.
+struct ClassWs {
+  size_t basis, gram, cscr;
+  size_t total() const { return basis + gram + cscr; }
+};
+ClassWs class_ws(int c, int kcap, bool fixed) {
+  const int k = wav_kind(c);
+  if (k >= 0) return {wav_basis(kcap), wav_gram(k, kcap, fixed), wav_cscr(k, kcap)};
+  return {class_basis_lds(c, kcap) ? 0 : (size_t)kcap * 64 * CLASS_R[c], fixed ? 0 : (size_t)kcap * kcap,
+          fixed ? 0 : 2 * (size_t)kcap};
 }
 
 template <bool F32, bool BAND, bool OBS>
@@ -1251,18 +1298,17 @@ hipError_t launch_sub_b(int c, const SubArgs& a, int n_cu, hipStream_t s, int* w
 template <bool FIXED, bool F32>
 hipError_t launch_class_p(int c, const SubArgs& a, int n_cu, hipStream_t s, int* waves, bool dry) {
   switch (c) {
-    case 0: return launch_sub_b<1, 4, FIXED, F32>(c, a, n_cu, s, waves, dry);
     case 1: return launch_sub_b<2, 4, FIXED, F32>(c, a, n_cu, s, waves, dry);
     case 2: return launch_sub_b<4, 4, FIXED, F32>(c, a, n_cu, s, waves, dry);
     case 3: return launch_sub_k<4, 0, FIXED, F32, false>(a, n_cu, s, waves, dry);
     case 4: return launch_sub_k<8, 0, FIXED, F32, false>(a, n_cu, s, waves, dry);
-    case 8: return launch_sub_b<1, 0, FIXED, F32>(c, a, n_cu, s, waves, dry);
     case 9: return launch_sub_b<2, 0, FIXED, F32>(c, a, n_cu, s, waves, dry);
     default: return launch_sub_k<16, 0, FIXED, F32, false>(a, n_cu, s, waves, dry);
   }
 }
 
 hipError_t launch_class(int c, const SubArgs& a, bool f32, int n_cu, hipStream_t s, int* waves, bool dry) {
+  if (wav_kind(c) >= 0) return launch_wav(wav_kind(c), a, f32, n_cu, s, waves, dry);
   if (c == PAIR_CLASS || c == PAIR_BAND_CLASS) {
     const bool band = c == PAIR_BAND_CLASS, obs = a.obs != 0;
     if (f32)
@@ -1336,14 +1382,16 @@ void scratch_release(SubScratch* sc) {
   delete sc;
 }
 
-// The pair classes: class-0 items of <= 32 rows under a fixed Krylov
-// dimension <= 16 (the banded ones, placed in PAIR_BAND_CLASS by the caller,
-// keep their own class), grouped by operator, each group padded to an even
-// count; other Krylov settings send the banded items back to class 0.
-void group_pairs(std::vector<int4> (&cls)[NCLASS], int32_t fixed_m, bool allow = true) {
+// The pair classes: narrow items (ELL width <= 4) of <= 32 rows under a fixed
+// Krylov dimension <= 16 go to k_sub_pair (the banded ones, placed in
+// PAIR_BAND_CLASS by the caller, keep their own class; other Krylov settings
+// send them back to the narrow class `narrow`), all other items of <= 32
+// rows to k_wav's pair classes; grouped by operator, each group padded to an
+// even count.  allow: two wavepackets per wave at all.
+void group_pairs(std::vector<int4> (&cls)[NCLASS], int32_t fixed_m, bool allow = true, int narrow = 0) {
   const bool pairs = allow && fixed_m >= 1 && fixed_m <= PAIR_MAX_M;
   if (!pairs && !cls[PAIR_BAND_CLASS].empty()) {
-    cls[0].insert(cls[0].end(), cls[PAIR_BAND_CLASS].begin(), cls[PAIR_BAND_CLASS].end());
+    cls[narrow].insert(cls[narrow].end(), cls[PAIR_BAND_CLASS].begin(), cls[PAIR_BAND_CLASS].end());
     cls[PAIR_BAND_CLASS].clear();
   }
   auto pair_up = [](std::vector<int4>& v) {
@@ -1358,13 +1406,22 @@ void group_pairs(std::vector<int4> (&cls)[NCLASS], int32_t fixed_m, bool allow =
     }
     v.swap(out);
   };
-  if (pairs && cls[PAIR_CLASS].empty()) {
+  auto move_short = [&](int from, int to, int rest) {
     std::vector<int4> keep;
-    for (const int4& it : cls[0]) (it.z <= 32 ? cls[PAIR_CLASS] : keep).push_back(it);
-    cls[0].swap(keep);
-    pair_up(cls[PAIR_CLASS]);
-    pair_up(cls[PAIR_BAND_CLASS]);
+    for (const int4& it : cls[from]) (it.z <= 32 ? cls[to] : keep).push_back(it);
+    cls[from].clear();
+    cls[rest].insert(cls[rest].end(), keep.begin(), keep.end());
+  };
+  // (a list grouped already, kept from an earlier call, is left as it is)
+  for (int c : {PAIR_CLASS, 10, 11, 13})
+    if (!cls[c].empty()) return;
+  if (allow) {
+    move_short(0, pairs ? PAIR_CLASS : 10, 0);
+    move_short(8, 11, 8);
+    move_short(12, 13, 12);
   }
+  move_short(COMPLEX4_CLASS, pairs ? PAIR_CLASS : allow ? 13 : 12, 12);
+  for (int c : {PAIR_CLASS, PAIR_BAND_CLASS, 10, 11, 13}) pair_up(cls[c]);
 }
 
 // Stage ops and items (the wave classes, then the block and cooperative
@@ -1391,8 +1448,7 @@ int launch_all(SubScratch* sc, const SubArgs& a0, const int4* const (&items)[NCL
     a.nitems = (int32_t)cls[c].size();
     int waves = 0;
     HIPCHK(launch_class(c, a, f32, n_cu, s, &waves, true));
-    const size_t per_wave = (class_basis_lds(c, kcap) ? 0 : (size_t)kcap * 64 * CLASS_R[c]) +
-                            (fixed_m > 0 ? 0 : (size_t)kcap * kcap + 2 * (size_t)kcap);
+    const size_t per_wave = class_ws(c, kcap, fixed_m > 0).total();
     wsoff[c] = need;
     need += (sizeof(double2) * std::max<size_t>(per_wave, 1) * (size_t)waves + 255) & ~(size_t)255;
   }
@@ -1432,10 +1488,10 @@ int launch_all(SubScratch* sc, const SubArgs& a0, const int4* const (&items)[NCL
     a.nitems = (int32_t)cls[c].size();
     int waves = 0;
     HIPCHK(launch_class(c, a, f32, n_cu, s, &waves, true));
-    const bool bl = class_basis_lds(c, kcap);
+    const ClassWs w = class_ws(c, kcap, fixed_m > 0);
     a.basis = (double2*)((char*)sc->ws + wsoff[c]);
-    a.gram = a.basis + (bl ? 0 : (size_t)waves * kcap * 64 * CLASS_R[c]);
-    a.cscr = a.gram + (fixed_m > 0 ? 0 : (size_t)waves * kcap * kcap);
+    a.gram = a.basis + (size_t)waves * w.basis;
+    a.cscr = a.gram + (size_t)waves * w.gram;
     hipStream_t cs;
     if ((rc = next_stream(&cs))) return rc;
     HIPCHK(launch_class(c, a, f32, n_cu, cs, &waves, false));
@@ -1593,6 +1649,7 @@ SubOp plan_op(const rm_plan* p) {
   op.sval = p->sval;
   op.sval32 = p->sval32;
   op.npairs = p->spairs;
+  op.sflags = p->ssym ? 1 : 0;
   op.nnz = p->nnz;
   op.perm = p->sub_perm;
   op.n = (int32_t)p->n;
@@ -1890,8 +1947,8 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
       if (force || hi - lo > std::min<int32_t>(p->tune.wave_max_rows, RM_SUBSPACE_MAX_ROWS) || !p->sub_col) {
         big.push_back(make_int4((int)b, lo, hi - lo, 0));
       } else {
-        const int c = sub_class(p->sub_w, hi - lo);
-        sc->kept_cls[c == 0 && hi - lo <= 32 && p->nfield <= NSR && sub_banded(p, lo, hi) ? PAIR_BAND_CLASS : c]
+        const int c = sub_class(p, lo, hi - lo);
+        sc->kept_cls[(c == 0 || c == COMPLEX4_CLASS) && hi - lo <= 32 && p->nfield <= NSR && sub_banded(p, lo, hi) ? PAIR_BAND_CLASS : c]
             .push_back(make_int4((int)b, lo, hi - lo, 0));
       }
     }
@@ -1914,7 +1971,7 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
     sort_long(sc->kept_blk);
     for (auto& v : sc->kept_cls)
       std::stable_sort(v.begin(), v.end(), [](const int4& x, const int4& y) { return x.z > y.z; });
-    group_pairs(sc->kept_cls, krylov_fixed, p->tune.pair != 0);
+    group_pairs(sc->kept_cls, krylov_fixed, p->tune.pair != 0, p->sreal ? 0 : COMPLEX4_CLASS);
     sc->kept_pairs = pairs;
     if (p->dom_reuse) {
       // a copy of their own: rm_plan_domains rewrites p->dom
@@ -2122,7 +2179,7 @@ static int collect_jobs(const char* who, const rm_job* jobs, int32_t njobs, int3
       blk.push_back(long_item(p, jb.col, lo, len, (int)ops.size()));
       blk_work.push_back((int64_t)jb.nsteps * blk.back().nent);
     } else {
-      const int c = sub_class(p->sub_w, len);
+      const int c = sub_class(p, lo, len);
       cls[c].push_back(make_int4(jb.col, lo, len, (int)ops.size()));
       work[c].push_back((int64_t)jb.nsteps * len);
     }
@@ -2249,9 +2306,8 @@ static int sub_run_static(char* dev, size_t bytes, const std::vector<SubOp>& ops
     if (cls[c].empty()) continue;
     a.items = (const int4*)(dev + off[c]);
     a.nitems = (int32_t)cls[c].size();
-    const bool bl = class_basis_lds(c, kcap);
-    const size_t per_wave = sizeof(double2) * ((bl ? 0 : (size_t)kcap * 64 * CLASS_R[c]) +
-                                               (fixed_m > 0 ? 0 : (size_t)kcap * kcap + 2 * (size_t)kcap));
+    const ClassWs w = class_ws(c, kcap, fixed_m > 0);
+    const size_t per_wave = sizeof(double2) * w.total();
     a.max_waves = 0;
     if (per_wave > 0) {
       const size_t cap = ws_bytes / per_wave;
@@ -2263,8 +2319,8 @@ static int sub_run_static(char* dev, size_t bytes, const std::vector<SubOp>& ops
     int waves = 0;
     HIPCHK(launch_class(c, a, f32, n_cu, s, &waves, true));
     a.basis = (double2*)ws;
-    a.gram = a.basis + (bl ? 0 : (size_t)waves * kcap * 64 * CLASS_R[c]);
-    a.cscr = a.gram + (fixed_m > 0 ? 0 : (size_t)waves * kcap * kcap);
+    a.gram = a.basis + (size_t)waves * w.basis;
+    a.cscr = a.gram + (size_t)waves * w.gram;
     HIPCHK(launch_class(c, a, f32, n_cu, s, &waves, false));
   }
   return RM_OK;
