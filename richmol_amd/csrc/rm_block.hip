@@ -86,7 +86,7 @@ struct BlkShared {
 // of the quadratic form; c and c_prev also go to cv (c, then c_prev) as the
 // general form keeps them.
 __device__ __forceinline__ double metric16(int k, bool breakdown, double2* G, int ld, const double2* alpha,
-                                           const double* beta, double2 f, double2* cv) {
+                                           const double* beta, double2 f, bool herm, double2* cv, double2* tmp) {
   const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
   if (!breakdown && i < k && q == 0) {
     double2 hv;
@@ -106,7 +106,7 @@ __device__ __forceinline__ double metric16(int k, bool breakdown, double2* G, in
     G[k * ld + i] = cconj(t);
   }
   if (lane == 0) G[k * ld + k] = make_double2(1.0, 0.0);
-  const double2 c = expm_row16(k + 1, alpha, beta, f);
+  const double2 c = herm ? expm_row16_herm<false>(k + 1, alpha, beta, f.y, tmp) : expm_row16(k + 1, alpha, beta, f);
   double2 d = make_double2(0.0, 0.0);
   if (i <= k) d = csub(c, i < k ? cv[ld + i] : make_double2(0.0, 0.0));
   if (q == 0) cv[i] = d;
@@ -148,6 +148,10 @@ __device__ __forceinline__ void blk_control(const BlkArgs& a, const SubOp& op, i
       observe(step);
       continue;
     }
+    // a real symmetric operator under real field products: alpha is real, and
+    // with a real-time exponent the exponentials take the real recursion
+    bool herm = (op.sflags & 1) && op.f.x == 0.0;
+    for (int s = 0; s < op.nslot; ++s) herm = herm && op.table[(int64_t)step * op.nslot + s].y == 0.0;
     __syncthreads();
     double2* Gm = sh.gram;
     double2* cv = sh.cv;
@@ -164,7 +168,7 @@ __device__ __forceinline__ void blk_control(const BlkArgs& a, const SubOp& op, i
         red[1] = r2[1];
       }
       k = it + 1;
-      if (lane == 0) sh.alpha[it] = make_double2(red[0], red[1]);
+      if (lane == 0) sh.alpha[it] = make_double2(red[0], herm ? 0.0 : red[1]);
       if (FIXED && k >= a.fixed_m) break;
       if (!FIXED) {
         if (it == 0) {
@@ -175,7 +179,7 @@ __device__ __forceinline__ void blk_control(const BlkArgs& a, const SubOp& op, i
           }
         } else {
           wave_sync();
-          const double c = it < 16 ? metric16(it, brk, Gm, g_ld, sh.alpha, sh.beta, op.f, cv)
+          const double c = it < 16 ? metric16(it, brk, Gm, g_ld, sh.alpha, sh.beta, op.f, herm, cv, sh.cf)
                                    : adaptive_metric<false>(it, brk, Gm, g_ld, sh.alpha, sh.beta, op.f, cv, cv + g_ld);
           if (lane == 0) sh.conv = c;
         }
@@ -226,7 +230,9 @@ __device__ __forceinline__ void blk_control(const BlkArgs& a, const SubOp& op, i
       if (k == 1) {
         if (lane == 0) sh.cf[0] = make_double2(1.0, 0.0);
       } else if (k <= 16) {
-        const double2 c = expm_row16(k, sh.alpha, sh.beta, op.f);
+        const double2 c = herm ? expm_row16_herm<false>(k, sh.alpha, sh.beta, op.f.y, sh.cf)
+                               : expm_row16(k, sh.alpha, sh.beta, op.f);
+        wave_sync();
         if (lane < k) sh.cf[lane] = c;
       } else {
         expm_e0(k, sh.alpha, sh.beta, op.f, sh.cf);
@@ -309,7 +315,7 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
   auto row_sum = [&](int r, const PT* __restrict__ q) __attribute__((always_inline)) -> XT {
     XT acc = to_x<F32>(zero), acc2 = to_x<F32>(zero);
     const uint32_t* __restrict__ qc = op.scol;
-    constexpr int U = 4;   // pairs loaded together
+    constexpr int U = 4;   // pairs loaded together (8: more spilled registers, 7 % slower)
     int p = 0;
     const int n = np[r];
     if (!ok[r]) return acc;
@@ -407,6 +413,7 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
       }
     }
     const double2 f0 = nslot == 1 ? fp[0] : make_double2(1.0, 0.0);
+    const bool realal = (op.sflags & 1) && op.f.x == 0.0 && !imag && f0.y == 0.0;
     // V_0 = phi = P psi (unnormalised, tdse.py:443-446), the first matvec input
 #pragma unroll
     for (int r = 0; r < RS; ++r) {
@@ -485,7 +492,7 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
         red[0] = r2[0];
         red[1] = r2[1];
       }
-      const double2 al = make_double2(red[0], red[1]);
+      const double2 al = make_double2(red[0], realal ? 0.0 : red[1]);
       k = it + 1;
       if (FIXED && k >= a.fixed_m) break;
       // W = w - alpha V_it - beta V_{it-1}, and |W|^2

@@ -92,4 +92,23 @@ __device__ __forceinline__ double2 expm_row16(int s, const double2* alpha, const
   return y;
 }
 
+// exp(f T) e0, s <= 16, per lane (expm_row16), for a real T and f = i phi: the
+// real recursion of expm_e0_16_herm_row.  Each half's own 1-norm decides.
+template <bool PAIR>
+__device__ __forceinline__ double2 expm_row16_herm(int s, const double2* alpha, const double* beta, double phi,
+                                                   double2* tmp) {
+  const int i = threadIdx.x & 15;
+  double a = 0.0, bl = 0.0, bu = 0.0, col1 = 0.0;
+  if (i < s) {
+    a = phi * alpha[i].x;
+    if (i >= 1) bl = phi * beta[i];
+    if (i + 1 < s) bu = phi * beta[i + 1];
+    col1 = fabs(a) + fabs(bl) + fabs(bu);
+  }
+  expm_e0_16_herm_row<PAIR>(s, a, bl, bu, row_max16(col1), tmp);
+  wave_sync();
+  const double2 c = tmp[i];
+  return i < s ? c : make_double2(0.0, 0.0);
+}
+
 }  // namespace

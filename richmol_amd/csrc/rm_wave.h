@@ -26,7 +26,8 @@ inline bool wav_pair(int kind) { return kind == WAV_P2 || kind == WAV_P16 || kin
 // coefficients beyond what LDS holds
 inline size_t wav_basis(int kcap) { return (size_t)kcap * 64; }
 inline size_t wav_gram(int kind, int kcap, bool fixed) { return fixed ? 0 : (size_t)kcap * kcap * (wav_pair(kind) ? 2 : 1); }
-inline size_t wav_cscr(int kind, int kcap) { return 2 * (size_t)kcap * (wav_pair(kind) ? 2 : 1); }
+// (c, c_prev, alpha, and beta as reals)
+inline size_t wav_cscr(int kind, int kcap) { return (4 * (size_t)kcap + 1) * (wav_pair(kind) ? 2 : 1); }
 // Launches a.items (column, lo, len, op; a pair's items adjacent, column -1: an
 // empty half) or, dry, only tells the number of waves.
 hipError_t launch_wav(int kind, const SubArgs& a, bool f32, int n_cu, hipStream_t s, int* waves, bool dry);

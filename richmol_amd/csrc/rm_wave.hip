@@ -25,27 +25,12 @@ namespace {
 constexpr int GO = 16, GLD = 17;   // Gram matrix order in LDS and its row length
 constexpr int LB_FIX = 20, LB_AD = 8;   // Krylov vectors in LDS, fixed and adaptive
 
+// alpha and beta held in LDS: all of a fixed dimension, 16 under the adaptive
+// rule (8 waves of a CU then fit its LDS; longer recurrences move to global memory)
+__host__ __device__ constexpr int lds_orders(int kcap, bool fixed) { return fixed || kcap < GO + 1 ? kcap : GO + 1; }
+
 __host__ __device__ constexpr int lds_vectors(int kcap, bool fixed) {
   return kcap < (fixed ? LB_FIX : LB_AD) ? kcap : (fixed ? LB_FIX : LB_AD);
-}
-
-// exp(f T) e0, s <= 16, per lane (expm_row16), for a real T and f = i phi: the
-// real recursion of expm_e0_16_herm_row.  Each half's own 1-norm decides.
-template <bool PAIR>
-__device__ __forceinline__ double2 expm_row16_herm(int s, const double2* alpha, const double* beta, double phi,
-                                                   double2* tmp) {
-  const int i = threadIdx.x & 15;
-  double a = 0.0, bl = 0.0, bu = 0.0, col1 = 0.0;
-  if (i < s) {
-    a = phi * alpha[i].x;
-    if (i >= 1) bl = phi * beta[i];
-    if (i + 1 < s) bu = phi * beta[i + 1];
-    col1 = fabs(a) + fabs(bl) + fabs(bu);
-  }
-  expm_e0_16_herm_row<PAIR>(s, a, bl, bu, row_max16(col1), tmp);
-  wave_sync();
-  const double2 c = tmp[i];
-  return i < s ? c : make_double2(0.0, 0.0);
 }
 
 // Orders beyond 16, as calls: they are rare and would set the registers of the
@@ -60,7 +45,7 @@ __device__ __attribute__((noinline)) void long_expm(int k, const double2* alpha,
 }
 
 template <bool FIXED, bool F32, bool REAL, bool PAIR, int NP>
-__global__ __launch_bounds__(64) void k_wav(SubArgs a) {
+__global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
   using XT = typename XType<F32>::T;
   using PT = typename PairT<F32, REAL>::T;
   constexpr int H = PAIR ? 2 : 1;         // wavepackets per wave
@@ -68,24 +53,27 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
   extern __shared__ char s_dyn[];
   const int kc = a.kcap;
   const int lb = lds_vectors(kc, FIXED);
-  // LDS: matvec input, basis [lb][64], alpha and beta per half, coefficients
+  // LDS: matvec input, basis [lb][64] (between steps the observable's state),
+  // alpha and beta per half (kl of them), coefficients
+  const int kl = lds_orders(kc, FIXED);
   XT* s_x = (XT*)s_dyn;
   double2* s_V = (double2*)(s_dyn + 64 * sizeof(XT));
-  double2* s_al = s_V + (size_t)lb * 64;                   // [H][kc]
-  double* s_be = (double*)(s_al + (size_t)H * kc);         // [H][kc + 1]
+  double2* s_o = s_V;
+  double2* s_al = s_V + (size_t)lb * 64;                   // [H][kl]
+  double* s_be = (double*)(s_al + (size_t)H * kl);         // [H][kl + 1]
   __shared__ double2 s_c[H][GO];                           // coefficients of the combination (orders <= 16)
   __shared__ double2 s_d[FIXED ? 1 : H][FIXED ? 1 : GO];
   __shared__ double2 s_g[FIXED ? 1 : H][FIXED ? 1 : GO * GLD];
-  __shared__ double2 s_o[64];
   const int l = threadIdx.x;
   const int h = PAIR ? l >> 5 : 0, i = PAIR ? l & 31 : l;
   const int i16 = l & 15;
   const double2 zero = make_double2(0.0, 0.0);
   double2* Vg = a.basis + (int64_t)blockIdx.x * kc * 64;
   double2* Gg = a.gram + (int64_t)blockIdx.x * kc * kc * H;
-  double2* Cg = a.cscr + (int64_t)blockIdx.x * 2 * kc * H;
-  double2* al_ = s_al + (size_t)h * kc;
-  double* be_ = s_be + (size_t)h * (kc + 1);
+  const int cs = 4 * kc + 1;              // c, c_prev, alpha, beta (as reals) of a half in global memory
+  double2* Cg = a.cscr + (int64_t)blockIdx.x * cs * H;
+  double2* al_ = s_al + (size_t)h * kl;
+  double* be_ = s_be + (size_t)h * (kl + 1);
   auto hsum = [&](double v) __attribute__((always_inline)) -> double {
     if constexpr (PAIR)
       return half_allsum32(v);
@@ -155,6 +143,7 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
     }
     auto observe = [&](int step) __attribute__((always_inline)) {
       if (!(a.obs && op.ow > 0)) return;
+      wave_sync();   // the basis' readers are done
       s_o[l] = st;
       wave_sync();
       double2 y = zero;
@@ -273,7 +262,12 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
         if (!realal) al.y = hsum(Wr.x * vk.y - Wr.y * vk.x);
         Wr = csub(Wr, cscale(beta, vp));
         Wr = realal ? csub(Wr, cscale(al.x, vk)) : csub(Wr, cmul(al, vk));
-        if (i == 0) al_[it] = al;
+        if (i == 0) {
+          if (FIXED || it < GO)
+            al_[it] = al;
+          else
+            Cg[(int64_t)h * cs + 2 * kc + it] = al;
+        }
         if (live) vl = vk;
         const int k = it + 1;
         if (FIXED) {
@@ -334,7 +328,12 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
                   double2* G = Gg + (int64_t)q * kc * kc;
                   for (int e = l; e < GO * GO; e += 64) G[(e / GO) * kc + e % GO] = s_g[q][(e / GO) * GLD + e % GO];
                 }
-                if (live && i < 16) Cg[(int64_t)h * 2 * kc + kc + i] = cprev;
+                if (live && i < 16) Cg[(int64_t)h * cs + kc + i] = cprev;
+                if (i < 16) {
+                  Cg[(int64_t)h * cs + 2 * kc + i] = al_[i];
+                  ((double*)(Cg + (int64_t)h * cs + 3 * kc))[i] = be_[i];
+                }
+                if (i == 0) ((double*)(Cg + (int64_t)h * cs + 3 * kc))[it] = be_[it];
                 __threadfence_block();
                 wave_sync();
               }
@@ -345,8 +344,9 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
                 const bool lq = __any(live && h == q);
                 if (!lq) continue;
                 const double bq = __shfl(beta, LP * q);
-                const double cq = long_metric(it, !(bq != 0.0), Gg + (int64_t)q * kc * kc, kc, s_al + (size_t)q * kc,
-                                              s_be + (size_t)q * (kc + 1), op.f, Cg + (int64_t)q * 2 * kc);
+                double2* c = Cg + (int64_t)q * cs;
+                const double cq = long_metric(it, !(bq != 0.0), Gg + (int64_t)q * kc * kc, kc, c + 2 * kc,
+                                              (const double*)(c + 3 * kc), op.f, c);
                 if (h == q) conv = cq;
               }
               if (live) {
@@ -364,7 +364,12 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
         beta = 0.0;
         if (ww != 0.0) sqrt_rcp_nb(ww, &beta, &ib);
         brk = !(ww != 0.0);
-        if (i == 0) be_[k] = beta;
+        if (i == 0) {
+          if (FIXED || k <= GO)
+            be_[k] = beta;
+          else
+            ((double*)(Cg + (int64_t)h * cs + 3 * kc))[k] = beta;
+        }
         vp = vk;
         if (!brk) {
           vk = cscale(ib, Wr);
@@ -390,7 +395,7 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
         if (kk > 16) {
 #pragma unroll
           for (int q = 0; q < H; ++q)
-            long_expm(kk, s_al + (size_t)q * kc, s_be + (size_t)q * (kc + 1), op.f, Cg + (int64_t)q * 2 * kc);
+            long_expm(kk, s_al + (size_t)q * kl, s_be + (size_t)q * (kl + 1), op.f, Cg + (int64_t)q * cs);
           big = true;
           __threadfence_block();
         } else if (kk > 1) {
@@ -400,7 +405,7 @@ __global__ __launch_bounds__(64) void k_wav(SubArgs a) {
       wave_sync();
       if (i < 16) s_c[h][i] = cprev;
       wave_sync();
-      const double2* cf = big ? Cg + (int64_t)h * 2 * kc + (FIXED ? 0 : kc) : s_c[h];
+      const double2* cf = big ? Cg + (int64_t)h * cs + (FIXED ? 0 : kc) : s_c[h];
       double2 u0 = zero, u1 = zero;
       const int kmax = PAIR ? max(kk, __shfl_xor(kk, 32)) : kk;
       for (int j = 0; j < kmax - 1; ++j) {
@@ -430,8 +435,8 @@ hipError_t launch_k(const SubArgs& a0, int n_cu, hipStream_t s, int* waves_out, 
   auto kern = k_wav<FIXED, F32, REAL, PAIR, NP>;
   constexpr int H = PAIR ? 2 : 1;
   const size_t lds = 64 * (F32 ? sizeof(float2) : sizeof(double2)) +
-                     sizeof(double2) * (size_t)(lds_vectors(a0.kcap, FIXED) * 64 + H * a0.kcap) +
-                     sizeof(double) * (size_t)(H * (a0.kcap + 1));
+                     sizeof(double2) * (size_t)(lds_vectors(a0.kcap, FIXED) * 64 + H * lds_orders(a0.kcap, FIXED)) +
+                     sizeof(double) * (size_t)(H * (lds_orders(a0.kcap, FIXED) + 1));
   int occ = 0;
   hipError_t e = occupancy((const void*)kern, 64, lds, &occ);
   if (e != hipSuccess) return e;
