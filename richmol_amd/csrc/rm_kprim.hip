@@ -168,9 +168,12 @@ __global__ __launch_bounds__(256) void k_pr_mf(const PMf* __restrict__ d, const 
   }
 }
 
-// One source block's contribution to the SR output rows of a wave: per
-// source row the k mixing U = sum_s P_s x(k1 - s) -- the neighbours in k are the
-// neighbouring lanes -- then acc[m1] += MF_sigma(m1) U on the rows it reaches.
+// One source block's contribution to the SR output rows of a wave: per output
+// row the m mixing z = sum_sigma MF_sigma(m1) x(m1 - sigma), then the k mixing
+// acc += sum_s P_s z(k1 - s) -- the neighbours in k are the neighbouring lanes.
+// (The k mixing first, on the SR + 4 source rows, costs 37 % more operations
+// for a full rank-2 tensor: 0.97 against 0.89 ms per matvec.  Loading the
+// rows once for all blocks of one J2 took 1.00 ms: more registers, fewer waves.)
 // xp: this lane's element of source row m2 = 0; row r of the window is
 // m2 = m0 + r - (largest sigma).
 template <typename T, int SP, int GP>
@@ -196,31 +199,26 @@ __device__ __forceinline__ void sten_task(const double2* __restrict__ xp, int m2
       p[i] = P[(int64_t)i * d1];
   }
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    V u;
-    {
-      const V c = p[2];
-      u.x = c.x * x[r].x - c.y * x[r].y;
-      u.y = c.x * x[r].y + c.y * x[r].x;
-    }
-    if constexpr (SP != S_0) {
-      const V dn = shc(x[r], false), up = shc(x[r], true);   // x(k1 - 1), x(k1 + 1)
-      if constexpr (SP == S_1 || SP == S_2) {
-        u = mac(p[3], dn, u);
-        u = mac(p[1], up, u);
-      }
-      if constexpr (SP == S_02 || SP == S_2) {
-        u = mac(p[4], shc(dn, false), u);
-        u = mac(p[0], shc(up, true), u);
-      }
-    }
+  for (int o = 0; o < SR; ++o) {
+    V z{0, 0};
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
       const int sg = i - 2;
       const bool use = GP == G_0 ? sg == 0 : GP == G_PM1 ? (sg == 1 || sg == -1) : GP == G_1 ? (sg >= -1 && sg <= 1)
                        : GP == G_02 ? (sg == 0 || sg == 2 || sg == -2) : true;
-      const int o = r - GM + sg;   // output row: m1 = m2 + sigma
-      if (use && o >= 0 && o < SR) acc[o] = mac(mf[(int64_t)i * dpad + o], u, acc[o]);
+      if (use) z = mac(mf[(int64_t)i * dpad + o], x[o + GM - sg < 0 || o + GM - sg >= NR ? 0 : o + GM - sg], z);
+    }
+    acc[o] = mac(p[2], z, acc[o]);
+    if constexpr (SP != S_0) {
+      const V dn = shc(z, false), up = shc(z, true);   // k1 - 1, k1 + 1
+      if constexpr (SP == S_1 || SP == S_2) {
+        acc[o] = mac(p[3], dn, acc[o]);
+        acc[o] = mac(p[1], up, acc[o]);
+      }
+      if constexpr (SP == S_02 || SP == S_2) {
+        acc[o] = mac(p[4], shc(dn, false), acc[o]);
+        acc[o] = mac(p[0], shc(up, true), acc[o]);
+      }
     }
   }
 }
