@@ -209,7 +209,7 @@ int rm_plan_kernel_time(rm_plan* plan, double* total_ms, int64_t* launches);
  * RM_SUBSPACE_MAX_ROWS) are advanced by a cooperative launch (many
  * workgroups on one wavepacket, grid barriers between the Lanczos
  * reductions) when there are at most 8 of them and each holds at least
- * their count x 6400 stored entries (RM_TUNE_COOP_MAX,
+ * their count x 40000 stored entries (RM_TUNE_COOP_MAX,
  * RM_TUNE_COOP_MIN_ENTRIES), otherwise by the block kernel (one workgroup
  * per wavepacket, all in one launch).
  *
@@ -247,7 +247,7 @@ int rm_plan_set_kernel(rm_plan* plan, int32_t variant);
  *                    RM_SUBSPACE_MAX_ROWS) take the long-domain forms;
  *  RM_TUNE_COOP_MIN_ENTRIES  the cooperative form only while every long
  *                    domain holds at least (their count) x this many stored
- *                    entries (default 6400: it runs them one at a time).
+ *                    entries (default 40000: it runs them one at a time).
  * Results do not depend on these choices beyond summation order.  A change
  * drops the launch lists kept for domain reuse. */
 #define RM_TUNE_PAIR       0
