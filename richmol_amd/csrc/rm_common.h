@@ -176,6 +176,7 @@ struct rm_plan {
   double* sval = nullptr;        // [nfield][spairs] pairs
   float* sval32 = nullptr;
   int64_t spairs = 0;
+  int32_t slice_rows = 0;        // subspaces of at most this many rows have their entries in slices
   bool sreal = false, ssym = false;   // ssym: real and symmetric
   std::vector<int32_t> h_srow;
   std::vector<int64_t> h_soff;   // [slices + 1]
@@ -229,6 +230,7 @@ struct rm_plan {
   int64_t expo_anorm_cap = 0;
   int4* expo_items = nullptr;
   int64_t expo_items_cap = 0;
+  std::vector<void*> arenas;     // the plan's arrays (Uploader)
   // optional HIP-event timing of the Krylov step launches
   int timing = 0;
   int nrec = 0;
@@ -286,6 +288,57 @@ static int upload(T** dst, const T* src, int64_t count) {
   if (count > 0 && src) HIPCHK(hipMemcpy(*dst, src, sizeof(T) * (size_t)count, hipMemcpyHostToDevice));
   return RM_OK;
 }
+
+// Several arrays in one allocation and (short ones) one copy: add() each, then
+// commit().  fill: the byte of arrays without a source.
+struct Uploader {
+  struct Item {
+    void** dst;
+    const void* src;
+    size_t bytes, off;
+    int fill;
+  };
+  std::vector<Item> items;
+  size_t total = 0;
+  template <typename T>
+  void add(T** dst, const T* src, int64_t count, int fill = 0) {
+    const size_t bytes = sizeof(T) * (size_t)(count > 0 ? count : 1);
+    items.push_back({(void**)dst, count > 0 ? src : nullptr, bytes, total, fill});
+    total += (bytes + 255) & ~(size_t)255;
+  }
+  int commit(std::vector<void*>& arenas) {
+    char* d = nullptr;
+    HIPCHK(hipMalloc((void**)&d, total ? total : 1));
+    arenas.push_back(d);
+    constexpr size_t BIG = 4 << 20;   // copied from where they are
+    std::vector<char> h;
+    size_t run = 0;                   // start of the staged run of short arrays
+    auto flush = [&]() -> int {
+      if (!h.empty()) HIPCHK(hipMemcpy(d + run, h.data(), h.size(), hipMemcpyHostToDevice));
+      h.clear();
+      return RM_OK;
+    };
+    for (const Item& it : items) {
+      if (it.bytes > BIG) {
+        const int rc = flush();
+        if (rc) return rc;
+        if (it.src)
+          HIPCHK(hipMemcpy(d + it.off, it.src, it.bytes, hipMemcpyHostToDevice));
+        else
+          HIPCHK(hipMemset(d + it.off, it.fill, it.bytes));
+      } else {
+        if (h.empty()) run = it.off;
+        h.resize(it.off - run, 0);
+        if (it.src)
+          h.insert(h.end(), (const char*)it.src, (const char*)it.src + it.bytes);
+        else
+          h.resize(h.size() + it.bytes, (char)it.fill);
+      }
+      *it.dst = d + it.off;
+    }
+    return flush();
+  }
+};
 
 // Grow a device scratch array to hold at least count elements (synchronises
 // the device before freeing a smaller one).

@@ -958,9 +958,10 @@ std::vector<double2> entry_values(const rm_plan* p) {
   return B;
 }
 
-// The sliced form of the permuted CSR arrays (rm_block.hip).
-int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
-                const std::vector<double2>& cval) {
+// All values real; and symmetric to 1e-14 (rows hold their columns ascending;
+// next[c]: the first entry of row c that no row above has passed).
+void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
+                    const std::vector<double2>& cval) {
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   p->sreal = true;
@@ -969,20 +970,31 @@ int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<in
       p->sreal = false;
       break;
     }
-  // symmetric to 1e-14 (rows keep the ascending column order of the original within a subspace)
   p->ssym = p->sreal;
+  std::vector<int64_t> next(rp.begin(), rp.end() - 1);
   for (int64_t r = 0; r < n && p->ssym; ++r)
     for (int64_t e = rp[r]; e < rp[r + 1] && p->ssym; ++e) {
       const int64_t c = ccol[e];
-      const int32_t* b = ccol.data() + rp[c];
-      const int32_t* t = ccol.data() + rp[c + 1];
-      const int32_t* f = std::lower_bound(b, t, (int32_t)r);
-      const int64_t e2 = f != t && *f == r ? f - ccol.data() : -1;
+      int64_t& q = next[(size_t)c];
+      while (q < rp[c + 1] && ccol[q] < r) ++q;
+      const int64_t e2 = q < rp[c + 1] && ccol[q] == r ? q : -1;
       for (int32_t s = 0; s < nf; ++s) {
         const double x = cval[(size_t)s * nnz + e].x, y = e2 >= 0 ? cval[(size_t)s * nnz + e2].x : 0.0;
         if (std::fabs(x - y) > 1e-14 * std::max(std::fabs(x), std::fabs(y))) p->ssym = false;
       }
     }
+}
+
+// The sliced form of the permuted CSR arrays (rm_block.hip), with the entries
+// of subspaces of at most max_rows rows.  Built again with all that the block
+// kernel takes when it is first given a longer one (the arrays before stay
+// with the plan: launches may still read them): the cooperative form does not
+// read them, and packing and copying took 17 of 87 ms of a first call on
+// 4 subspaces of 3 000 rows.
+int slice_build(rm_plan* p, Uploader& up, int32_t max_rows, const std::vector<int64_t>& rp,
+                const std::vector<int32_t>& ccol, const std::vector<double2>& cval) {
+  const int64_t n = p->n, nnz = p->nnz;
+  const int32_t nf = std::max(p->nfield, 1);
   std::vector<int4> sl;
   for (int32_t c = 0; c < p->nsub; ++c) {
     const int32_t lo = p->h_sub_start[c], len = p->h_sub_end[c] - lo;
@@ -1001,9 +1013,8 @@ int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<in
       w = std::max(w, rp[r + 1] - rp[r]);
       p->h_srow[r] = (int32_t)i;
     }
-    // a subspace longer than the block kernel takes: no entries
     const int32_t c = p->h_sub_label_perm[sl[i].x];
-    sl[i].z = p->h_sub_end[c] - p->h_sub_start[c] <= BLK_MAX_ROWS ? (int32_t)((w + 1) / 2) : 0;
+    sl[i].z = p->h_sub_end[c] - p->h_sub_start[c] <= max_rows ? (int32_t)((w + 1) / 2) : 0;
     off.push_back(off.back() + 64 * (int64_t)sl[i].z);
   }
   const int64_t np = off.back();
@@ -1031,13 +1042,16 @@ int slice_build(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<in
       }
     }
   const std::vector<float> val32(val.begin(), val.end());
-  int rc = RM_OK;
-  if ((rc = upload(&p->sslice, sl.data(), (int64_t)sl.size())) || (rc = upload(&p->soff, off.data(), (int64_t)off.size())) ||
-      (rc = upload(&p->srow, p->h_srow.data(), n)) || (rc = upload(&p->scol, col.data(), (int64_t)col.size())) ||
-      (rc = upload(&p->sval, val.data(), (int64_t)val.size())) ||
-      (rc = upload(&p->sval32, val32.data(), (int64_t)val32.size())))
-    return rc;
+  up.add(&p->sslice, sl.data(), (int64_t)sl.size());
+  up.add(&p->soff, off.data(), (int64_t)off.size());
+  up.add(&p->srow, p->h_srow.data(), n);
+  up.add(&p->scol, col.data(), (int64_t)col.size());
+  up.add(&p->sval, val.data(), (int64_t)val.size());
+  up.add(&p->sval32, val32.data(), (int64_t)val32.size());
+  const int rc = up.commit(p->arenas);
+  if (rc) return rc;
   p->spairs = np;
+  p->slice_rows = max_rows;
   p->h_soff.swap(off);
   return RM_OK;
 }
@@ -1075,11 +1089,13 @@ int csr_upload(rm_plan* p, std::vector<int64_t>& rp, const std::vector<int32_t>&
   const int32_t nf = std::max(p->nfield, 1);
   std::vector<float2> cval32(cval.size());
   for (size_t q = 0; q < cval.size(); ++q) cval32[q] = make_float2((float)cval[q].x, (float)cval[q].y);
-  int rc = RM_OK;
-  if ((rc = upload(&p->sub_rp, rp.data(), n + 1)) || (rc = upload(&p->sub_ccol, ccol.data(), nnz)) ||
-      (rc = upload(&p->sub_cval, cval.data(), (int64_t)nf * nnz)) ||
-      (rc = upload(&p->sub_cval32, cval32.data(), (int64_t)nf * nnz)))
-    return rc;
+  Uploader up;
+  up.add(&p->sub_rp, rp.data(), n + 1);
+  up.add(&p->sub_ccol, ccol.data(), nnz);
+  up.add(&p->sub_cval, cval.data(), (int64_t)nf * nnz);
+  up.add(&p->sub_cval32, cval32.data(), (int64_t)nf * nnz);
+  const int rc = up.commit(p->arenas);
+  if (rc) return rc;
   p->h_sub_rp.swap(rp);
   return RM_OK;
 }
@@ -1091,6 +1107,17 @@ int csr_build(rm_plan* p, const std::vector<double2>& B) {
   std::vector<double2> cval;
   csr_host(p, B, rp, ccol, cval);
   return csr_upload(p, rp, ccol, cval);
+}
+
+// Slices for a long domain of len rows.
+int slice_need(rm_plan* p, int32_t len) {
+  if (len <= p->slice_rows || len > BLK_MAX_ROWS) return RM_OK;
+  std::vector<int64_t> rp;
+  std::vector<int32_t> ccol;
+  std::vector<double2> cval;
+  csr_host(p, entry_values(p), rp, ccol, cval);
+  Uploader up;
+  return slice_build(p, up, BLK_MAX_ROWS, rp, ccol, cval);
 }
 
 // Connected components of the sparsity graph (host union-find), the row
@@ -1145,16 +1172,20 @@ int sub_build(rm_plan* p) {
   p->h_sub_label_perm.resize((size_t)n);
   for (int64_t ip = 0; ip < n; ++ip) p->h_sub_label_perm[ip] = label[perm[ip]];
   int rc = RM_OK;
-  if ((rc = upload(&p->sub_perm, perm.data(), n)) || (rc = upload(&p->sub_label, label.data(), n)) ||
-      (rc = upload(&p->sub_iperm, iperm.data(), n)) || (rc = upload(&p->sub_lo, lo.data(), nc)) ||
-      (rc = upload(&p->sub_hi, hi.data(), nc)))
-    return rc;
+  Uploader up;
+  up.add(&p->sub_perm, perm.data(), n);
+  up.add(&p->sub_label, label.data(), n);
+  up.add(&p->sub_iperm, iperm.data(), n);
+  up.add(&p->sub_lo, lo.data(), nc);
+  up.add(&p->sub_hi, hi.data(), nc);
   // ELL (column-major) for the one-wave kernel: only if some subspace fits a wave
   const int32_t W = p->ell_w;
+  std::vector<int32_t> hcol;
+  std::vector<double2> hval;
   if (mn <= RM_SUBSPACE_MAX_ROWS) {
     const size_t ne = (size_t)W * (size_t)n;
-    std::vector<int32_t> hcol(ne);
-    std::vector<double2> hval((size_t)nf * ne, make_double2(0.0, 0.0));
+    hcol.resize(ne);
+    hval.assign((size_t)nf * ne, make_double2(0.0, 0.0));
     for (int64_t ip = 0; ip < n; ++ip) {
       const int32_t i = perm[ip];
       const int64_t r0 = p->h_row_ptr[i], len = p->h_row_ptr[i + 1] - r0;
@@ -1169,16 +1200,16 @@ int sub_build(rm_plan* p) {
       }
     }
     p->h_sub_col = hcol;
-    if ((rc = upload(&p->sub_col, hcol.data(), (int64_t)ne)) ||
-        (rc = upload(&p->sub_val, hval.data(), (int64_t)((size_t)nf * ne))))
-      return rc;
+    up.add(&p->sub_col, (const int32_t*)hcol.data(), (int64_t)ne);
+    up.add(&p->sub_val, (const double2*)hval.data(), (int64_t)((size_t)nf * ne));
   }
-  p->h_sub_perm.swap(perm);
+  p->h_sub_perm = perm;
   std::vector<int64_t> rp;
   std::vector<int32_t> ccol;
   std::vector<double2> cval;
   csr_host(p, B, rp, ccol, cval);
-  if ((rc = slice_build(p, rp, ccol, cval))) return rc;
+  operator_flags(p, rp, ccol, cval);
+  if ((rc = slice_build(p, up, RM_SUBSPACE_MAX_ROWS, rp, ccol, cval))) return rc;
   // CSR (row-major, permuted) for the cooperative kernel: if some subspace does not fit
   if (mx > RM_SUBSPACE_MAX_ROWS && (rc = csr_upload(p, rp, ccol, cval))) return rc;
   p->sub_w = W;
@@ -1357,6 +1388,9 @@ struct SubScratch {
   std::vector<LongItem> kept_blk, kept_coop;
   int4* kept_dev = nullptr;            // the kept lists' items on the device (classes, block, cooperative)
   size_t kept_dev_cap = 0;             // in items
+  int4* kept_host = nullptr;           // pinned staging of their upload, and its end
+  size_t kept_host_cap = 0;
+  hipEvent_t kept_up = nullptr;
 };
 
 void scratch_release(SubScratch* sc) {
@@ -1369,6 +1403,8 @@ void scratch_release(SubScratch* sc) {
   }
   if (sc->ws) (void)hipFree(sc->ws);
   if (sc->kept_dev) (void)hipFree(sc->kept_dev);
+  if (sc->kept_up) (void)hipEventDestroy(sc->kept_up);
+  if (sc->kept_host) (void)hipHostFree(sc->kept_host);
   coop_scratch_release(sc->long_ws);
   if (sc->blk_ws) (void)hipFree(sc->blk_ws);
   for (int i = 0; i <= NCLASS; ++i) {
@@ -1380,6 +1416,17 @@ void scratch_release(SubScratch* sc) {
   }
   if (sc->fork) (void)hipEventDestroy(sc->fork);
   delete sc;
+}
+
+// Stable sort by falling length (lengths of the wave classes: counting sort).
+void longest_first(std::vector<int4>& v) {
+  if (v.size() < 2) return;
+  std::vector<int32_t> at(RM_SUBSPACE_MAX_ROWS + 2, 0);
+  for (const int4& it : v) ++at[(size_t)(RM_SUBSPACE_MAX_ROWS - it.z + 1)];
+  for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
+  std::vector<int4> out(v.size());
+  for (const int4& it : v) out[(size_t)at[(size_t)(RM_SUBSPACE_MAX_ROWS - it.z)]++] = it;
+  v.swap(out);
 }
 
 // The pair classes: narrow items (ELL width <= 4) of <= 32 rows under a fixed
@@ -1396,7 +1443,8 @@ void group_pairs(std::vector<int4> (&cls)[NCLASS], int32_t fixed_m, bool allow =
   }
   auto pair_up = [](std::vector<int4>& v) {
     if (v.empty()) return;
-    std::stable_sort(v.begin(), v.end(), [](const int4& x, const int4& y) { return x.w < y.w; });
+    const auto by_op = [](const int4& x, const int4& y) { return x.w < y.w; };
+    if (!std::is_sorted(v.begin(), v.end(), by_op)) std::stable_sort(v.begin(), v.end(), by_op);
     std::vector<int4> out;
     for (size_t i = 0; i < v.size();) {
       size_t j = i;
@@ -1941,15 +1989,26 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
     sc->kept_blk.clear();
     sc->kept_coop.clear();
     std::vector<int4> big;
+    // the class of a domain that is one subspace, found once per subspace and call
+    std::vector<int8_t> sub_cls((size_t)p->nsub, (int8_t)-1);
     for (int64_t b = 0; b < ncols; ++b) {
       const int32_t lo = p->h_dom[2 * b], hi = p->h_dom[2 * b + 1];
       if (hi <= lo) continue;   // zero column: stays zero (kused 0)
+      const int32_t sub = p->h_sub_label_perm[lo];
+      int8_t* known = p->h_sub_end[sub] == hi ? &sub_cls[(size_t)sub] : nullptr;
+      if (known && *known >= 0) {
+        sc->kept_cls[*known].push_back(make_int4((int)b, lo, hi - lo, 0));
+        continue;
+      }
       if (force || hi - lo > std::min<int32_t>(p->tune.wave_max_rows, RM_SUBSPACE_MAX_ROWS) || !p->sub_col) {
         big.push_back(make_int4((int)b, lo, hi - lo, 0));
       } else {
         const int c = sub_class(p, lo, hi - lo);
-        sc->kept_cls[(c == 0 || c == COMPLEX4_CLASS) && hi - lo <= 32 && p->nfield <= NSR && sub_banded(p, lo, hi) ? PAIR_BAND_CLASS : c]
-            .push_back(make_int4((int)b, lo, hi - lo, 0));
+        const int cl = (c == 0 || c == COMPLEX4_CLASS) && hi - lo <= 32 && p->nfield <= NSR && sub_banded(p, lo, hi)
+                           ? PAIR_BAND_CLASS
+                           : c;
+        sc->kept_cls[cl].push_back(make_int4((int)b, lo, hi - lo, 0));
+        if (known) *known = (int8_t)cl;
       }
     }
     if (!big.empty() && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
@@ -1962,19 +2021,21 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
     // 1 wavepacket of 24 046 entries 61 / 57, 49 218: 77 / 61, 370 802: 501 / 79;
     // 4 of 88 706: 136 / 224, of 151 010: 213 / 236, of 241 442: 348 / 258;
     // 8 of 367 402: 532 / 551.
-    std::vector<LongItem> lbig;
     int64_t emin = INT64_MAX;
+    int32_t longest = 0;
     for (const int4& it : big) {
-      lbig.push_back(long_item(p, it.x, it.y, it.z, 0));
-      emin = std::min<int64_t>(emin, lbig.back().nent);
+      emin = std::min<int64_t>(emin, p->h_sub_rp[it.y + it.z] - p->h_sub_rp[it.y]);
+      longest = std::max(longest, std::min<int32_t>(it.z, BLK_MAX_ROWS));
     }
     const bool to_coop = force == RM_KERNEL_COOP ||
                          (force == 0 && (int64_t)big.size() <= p->tune.coop_max &&
                           (int64_t)big.size() * p->tune.coop_min_entries <= emin);
-    for (const LongItem& it : lbig) (to_coop ? sc->kept_coop : sc->kept_blk).push_back(it);
+    // before the items: they hold their domains' slice widths
+    if (!to_coop && (rc = slice_need(p, longest))) return rc;
+    for (const int4& it : big)
+      (to_coop ? sc->kept_coop : sc->kept_blk).push_back(long_item(p, it.x, it.y, it.z, 0));
     sort_long(sc->kept_blk);
-    for (auto& v : sc->kept_cls)
-      std::stable_sort(v.begin(), v.end(), [](const int4& x, const int4& y) { return x.z > y.z; });
+    for (auto& v : sc->kept_cls) longest_first(v);
     group_pairs(sc->kept_cls, krylov_fixed, p->tune.pair != 0, p->sreal ? 0 : COMPLEX4_CLASS);
     sc->kept_pairs = pairs;
     if (p->dom_reuse) {
@@ -1997,8 +2058,18 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
         HIPCHK(hipMalloc((void**)&sc->kept_dev, sizeof(int4) * sc->kept_dev_cap));
       }
       if (!all.empty()) {
-        HIPCHK(hipMemcpyAsync(sc->kept_dev, all.data(), sizeof(int4) * all.size(), hipMemcpyHostToDevice, s));
-        HIPCHK(hipStreamSynchronize(s));   // `all` is released at the end of this block
+        // through pinned memory, rewritten only after its previous copy has run
+        if (sc->kept_up) HIPCHK(hipEventSynchronize(sc->kept_up));
+        if (sc->kept_host_cap < all.size()) {
+          if (sc->kept_host) HIPCHK(hipHostFree(sc->kept_host));
+          sc->kept_host = nullptr;
+          sc->kept_host_cap = std::max<size_t>(all.size(), 4096);
+          HIPCHK(hipHostMalloc((void**)&sc->kept_host, sizeof(int4) * sc->kept_host_cap, hipHostMallocDefault));
+        }
+        memcpy(sc->kept_host, all.data(), sizeof(int4) * all.size());
+        HIPCHK(hipMemcpyAsync(sc->kept_dev, sc->kept_host, sizeof(int4) * all.size(), hipMemcpyHostToDevice, s));
+        if (!sc->kept_up) HIPCHK(hipEventCreateWithFlags(&sc->kept_up, hipEventDisableTiming));
+        HIPCHK(hipEventRecord(sc->kept_up, s));
       }
       sc->kept = true;
       sc->kept_psi = psi;
@@ -2167,6 +2238,7 @@ static int collect_jobs(const char* who, const rm_job* jobs, int32_t njobs, int3
                   "entry point does not hold (at most %d rows; use rm_batch_propagate)", who, j, len,
                   RM_SUBSPACE_MAX_ROWS);
     if (longdom && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
+    if (longdom && (rc = slice_need(p, len))) return rc;
     SubOp op = plan_op(p);
     op.phase = (const double2*)jb.phase;
     op.table = (const double2*)jb.fprod_dev;

@@ -37,13 +37,9 @@ extern "C" int rm_version(void) { return RM_ABI_VERSION; }
 // plan
 
 static void plan_free(rm_plan* p) {
-  void* bufs[] = {p->row_ptr, p->col, p->pair_ptr, p->pair_term, p->pair_kval, p->term_ptr,
-                  p->term_field, p->term_mval, p->term_leaf, p->mf, p->aval, p->flag, p->ws,
-                  p->ell_col, p->ell_val, p->ell_pos, p->sub_perm, p->sub_label, p->sub_lo,
-                  p->sub_hi, p->sub_col, p->sub_val, p->sub_rp, p->sub_ccol, p->sub_cval, p->sub_cval32, p->sslice, p->soff, p->srow, p->scol, p->sval, p->sval32, p->dom,
-                  p->sflag, p->sflag_part, p->sflag_arrive, p->dom_keep, p->stale, p->int_status,
-                  p->sub_iperm, p->obs_col, p->obs_val, p->ex_buf, p->expo_ws, p->expo_anorm,
-                  p->expo_items};
+  void* bufs[] = {p->ws, p->dom, p->sflag, p->sflag_part, p->sflag_arrive, p->dom_keep, p->stale, p->int_status,
+                  p->obs_col, p->obs_val, p->ex_buf, p->expo_ws, p->expo_anorm, p->expo_items};
+  for (void* b : p->arenas) (void)hipFree(b);
   sub_scratch_release(p->sub_scratch);
   if (p->h_dom_pin) (void)hipHostFree(p->h_dom_pin);
   if (p->h_status_pin) (void)hipHostFree(p->h_status_pin);
@@ -105,26 +101,19 @@ extern "C" int rm_plan_create(int64_t n, int64_t nnz, const int64_t* row_ptr, co
   p->h_term_mval.assign((const double2*)term_mval, (const double2*)term_mval + nq);
   if (hipGetDevice(&p->device) != hipSuccess) { plan_free(p); return fail(RM_ERR_HIP, "hipGetDevice failed"); }
   int rc = RM_OK;
-  if ((rc = upload(&p->row_ptr, row_ptr, n + 1)) ||
-      (rc = upload(&p->col, col_idx, nnz)) ||
-      (rc = upload(&p->pair_ptr, pair_ptr, nnz + 1)) ||
-      (rc = upload(&p->pair_term, pair_term, npair)) ||
-      (rc = upload(&p->pair_kval, (const double2*)pair_kval, npair)) ||
-      (rc = upload(&p->term_ptr, term_ptr, nterm + 1)) ||
-      (rc = upload(&p->term_field, term_field, nq)) ||
-      (rc = upload(&p->term_mval, (const double2*)term_mval, nq)) ||
-      (rc = upload(&p->term_leaf, term_leaf, nterm)) ||
-      (rc = upload<double2>(&p->mf, nullptr, nterm)) ||
-      (rc = upload<double2>(&p->aval, nullptr, nnz)) ||
-      (rc = upload<int32_t>(&p->flag, nullptr, 1))) {
-    plan_free(p);
-    return rc;
-  }
-  if (hipMemset(p->aval, 0, sizeof(double2) * (size_t)(nnz > 0 ? nnz : 1)) != hipSuccess ||
-      hipMemset(p->flag, 0xff, sizeof(int32_t)) != hipSuccess) {
-    plan_free(p);
-    return fail(RM_ERR_HIP, "rm_plan_create: hipMemset failed");
-  }
+  Uploader up;
+  up.add(&p->row_ptr, row_ptr, n + 1);
+  up.add(&p->col, col_idx, nnz);
+  up.add(&p->pair_ptr, pair_ptr, nnz + 1);
+  up.add(&p->pair_term, pair_term, npair);
+  up.add(&p->pair_kval, (const double2*)pair_kval, npair);
+  up.add(&p->term_ptr, term_ptr, nterm + 1);
+  up.add(&p->term_field, term_field, nq);
+  up.add(&p->term_mval, (const double2*)term_mval, nq);
+  up.add(&p->term_leaf, term_leaf, nterm);
+  up.add<double2>(&p->mf, nullptr, nterm);
+  up.add<double2>(&p->aval, nullptr, nnz);
+  up.add<int32_t>(&p->flag, nullptr, 1, 0xff);
   // ELL layout
   int64_t w = 0;
   for (int64_t i = 0; i < n; ++i) w = row_ptr[i + 1] - row_ptr[i] > w ? row_ptr[i + 1] - row_ptr[i] : w;
@@ -154,18 +143,15 @@ extern "C" int rm_plan_create(int64_t n, int64_t nnz, const int64_t* row_ptr, co
         }
       }
     }
-    rc = upload(&p->ell_col, hcol, ne);
-    if (!rc) rc = upload(&p->ell_pos, hpos, nnz);
-    if (!rc) rc = upload<double2>(&p->ell_val, nullptr, ne);
+    up.add(&p->ell_col, (const int32_t*)hcol, ne);
+    up.add(&p->ell_pos, (const int32_t*)hpos, nnz);
+    up.add<double2>(&p->ell_val, nullptr, ne);
+    rc = up.commit(p->arenas);
     free(hcol);
     free(hpos);
     if (rc) {
       plan_free(p);
       return rc;
-    }
-    if (hipMemset(p->ell_val, 0, sizeof(double2) * (size_t)(ne > 0 ? ne : 1)) != hipSuccess) {
-      plan_free(p);
-      return fail(RM_ERR_HIP, "rm_plan_create: hipMemset failed");
     }
   }
   if (hipDeviceGetAttribute(&p->n_cu, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess ||

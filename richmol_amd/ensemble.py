@@ -188,11 +188,12 @@ class Ensemble:
             if not check:
                 return (expect, expect_sum) if obs is not None else None
             from . import _lib
-            if attempt == 0 and np.any(self.status.cpu().numpy() & _lib.RM_STALE_DOMAIN):
+            st = self.status.cpu().numpy()
+            if attempt == 0 and np.any(st & _lib.RM_STALE_DOMAIN):
                 self.plan.set_domain_reuse(True, owner=id(self))   # forget the kept domains
                 continue
             break
-        self.check()
+        self._raise_status(st)
         if obs is not None:
             return expect, expect_sum
 
@@ -238,8 +239,12 @@ class Ensemble:
         """Raise on the status bits of the last call: a cooperative timeout,
         rows rewritten since the domains were kept, or (adaptive rule) a row
         that reached maxorder."""
+        self._raise_status(self.status.cpu().numpy())
+
+    def _raise_status(self, st):
         from . import _lib
-        st = self.status.cpu().numpy()
+        if not st.any():
+            return
         if np.any(st & _lib.RM_DEVICE_TIMEOUT):
             raise RuntimeError("a cooperative propagation launch timed out at a grid barrier; "
                                "its wavepackets are invalid")
