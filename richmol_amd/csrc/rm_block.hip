@@ -446,6 +446,10 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
         } else {
           XT acc;
           if constexpr (REG) {
+            // (the empty asm: without it the compiler spills 470 registers in
+            // the FP64 kernel of a fixed dimension, 50 us an iteration)
+#pragma unroll
+            for (int p = 0; p < NP; ++p) keep(A[p]);
             XT acc1 = to_x<F32>(zero);
             acc = to_x<F32>(zero);
 #pragma unroll

@@ -35,6 +35,11 @@ __device__ __forceinline__ void pair_mac(const PairT<false, false>::T& p, double
 __device__ __forceinline__ void pair_mac(float4 p, float2 x0, float2 x1, float2& acc) {
   acc = fmac(make_float2(p.z, p.w), x1, fmac(make_float2(p.x, p.y), x0, acc));
 }
+// a pair's value as the compiler must take it from here on
+__device__ __forceinline__ void keep(double2& v) { asm volatile("" : "+v"(v.x)); }
+__device__ __forceinline__ void keep(float2& v) { asm volatile("" : "+v"(v.x)); }
+__device__ __forceinline__ void keep(float4& v) { asm volatile("" : "+v"(v.x)); }
+__device__ __forceinline__ void keep(PairT<false, false>::T& v) { asm volatile("" : "+v"(v.a.x)); }
 // the FP64 pair of slot s, and its sum over the slots in FP64, rounded once
 template <bool REAL>
 __device__ __forceinline__ typename PairT<false, REAL>::T pair_load(const SubOp& op, int64_t s, int64_t q) {
