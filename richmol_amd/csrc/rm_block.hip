@@ -42,9 +42,52 @@ struct BlkArgs {
   int32_t nitems;
   char* ws;                // one region per workgroup: basis [kcap][lmax], operator pairs
   int64_t wg_bytes, offA, offG;
+  const void* pre;         // the steps' operators (k_blk_operators), entry 0 of the plan's slices; or NULL
+  int64_t pre_ld;          // pairs from one step's to the next one's
   int32_t kcap, fixed_m, maxorder, lmax;
   double tol;
 };
+
+constexpr int PRE_STEPS = 8;   // steps of one thread
+
+// The operators A(F) = sum_s F_s B_s of steps 0 .. nsteps-1 on the pairs [q0,
+// q0 + count) of the sliced form, for every wavepacket of the launch: a step
+// whose products are those of the step before is left out, as its readers
+// leave it out.  Bound by its stores; a thread loads a pair's slots once for
+// PRE_STEPS steps.
+template <bool F32, bool REAL>
+__global__ __launch_bounds__(256) void k_blk_operators(SubOp op, int64_t q0, int64_t count,
+                                                       typename PairT<F32, REAL>::T* __restrict__ out) {
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int t0 = blockIdx.y * PRE_STEPS, nt = min(PRE_STEPS, op.nsteps - t0);
+  if (q >= count) return;
+  const double2* fp = op.table + (int64_t)t0 * op.nslot;
+  bool need[PRE_STEPS];
+  typename PairT<false, REAL>::T acc[PRE_STEPS];
+#pragma unroll
+  for (int t = 0; t < PRE_STEPS; ++t) {
+    acc[t] = {};
+    need[t] = t < nt && t0 + t == 0;
+    if (t < nt && t0 + t > 0)
+      for (int s = 0; s < op.nslot; ++s) {
+        const double2 f = fp[(int64_t)t * op.nslot + s], g = fp[(int64_t)(t - 1) * op.nslot + s];
+        need[t] = need[t] || !(f.x == g.x && f.y == g.y);
+      }
+  }
+  for (int s = 0; s < op.nslot; ++s) {
+    const auto v = pair_load<REAL>(op, s, q0 + q);
+#pragma unroll
+    for (int t = 0; t < PRE_STEPS; ++t)
+      if (need[t]) pair_add(acc[t], fp[(int64_t)t * op.nslot + s], v);
+  }
+#pragma unroll
+  for (int t = 0; t < PRE_STEPS; ++t)
+    if (need[t]) {
+      typename PairT<F32, REAL>::T o;
+      pair_round(acc[t], o);
+      out[(int64_t)(t0 + t) * count + q] = o;
+    }
+}
 
 // Sum of NQ values over the workgroup, the same on every thread; one barrier.
 // red: [2][NW][4], the halves used in turn.
@@ -398,7 +441,7 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
               for (int s = 0; s < nslot; ++s) pair_add(t, fp[s], pair_load<REAL>(op, s, e0[0] + 64 * p));
             pair_round(t, A[p]);
           }
-        } else {
+        } else if (!a.pre) {
 #pragma unroll
           for (int r = 0; r < RS; ++r) {
             const int64_t ea = e0[r] - op.soff[ns0];
@@ -468,7 +511,7 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
           } else if (nslot == 1) {
             acc = row_sum(r, F32 ? (const PT*)op.sval32 : (const PT*)op.sval);
           } else {
-            acc = row_sum(r, Ast - op.soff[ns0]);
+            acc = row_sum(r, a.pre ? (const PT*)a.pre + (int64_t)built * a.pre_ld : Ast - op.soff[ns0]);
           }
           y = cmul(f0, to_d2(acc));
         }
@@ -623,6 +666,8 @@ __global__ __launch_bounds__(NT) void k_blk(BlkArgs a) {
   }
 }
 
+constexpr size_t PRE_BYTES = (size_t)256 << 20;
+
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 template <int RS, bool REG>
@@ -678,18 +723,30 @@ int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, c
     lmax = std::max<int64_t>(lmax, items[i].item.z);
     if (items[i].nslot > 1) pmax = std::max<int64_t>(pmax, items[i].npairs);
   }
+  // one job by value: its steps' operators are formed once for all its
+  // wavepackets, for as many steps as PRE_BYTES hold, and the launch is cut
+  // there (the state is in psi between launches)
+  int64_t q0 = INT64_MAX, q1 = 0;
+  for (size_t i = first; i < first + count; ++i) {
+    q0 = std::min(q0, items[i].pair0);
+    q1 = std::max(q1, items[i].pair0 + items[i].npairs);
+  }
+  const size_t b_step = (size_t)(f32 ? 8 : 16) * (real ? 1 : 2) * (size_t)std::max<int64_t>(q1 - q0, 1);
+  const bool pre = !reg && op0 && op0->nslot > 1 && op0->nsteps > 0;
+  const int chunk = !pre ? INT32_MAX : (int)std::max<int64_t>(1, std::min<int64_t>(op0->nsteps, PRE_BYTES / b_step));
+  const size_t b_pre = pre ? al256(b_step * (size_t)chunk) : 0;
   const size_t lds = lds_bytes(lmax, f32);
   int occ = 0;
   HIPCHK(occupancy(kern, NT, lds, &occ));
   if (occ < 1) return fail(RM_ERR_ARG, "block propagation: a domain of %lld rows does not fit LDS", (long long)lmax);
   const int grid = (int)std::min<int64_t>((int64_t)count, (int64_t)occ * n_cu);
   const size_t b_v = al256(sizeof(double2) * (size_t)kcap * lmax);
-  const size_t b_a = al256((f32 ? 8 : 16) * (real ? 1 : 2) * (size_t)std::max<int64_t>(pmax, 1));
+  const size_t b_a = pre ? 0 : al256((f32 ? 8 : 16) * (real ? 1 : 2) * (size_t)std::max<int64_t>(pmax, 1));
   const size_t b_g = fixed ? 0 : al256(sizeof(double2) * ((size_t)kcap * kcap + 2 * (size_t)kcap));
   a.offA = (int64_t)b_v;
   a.offG = (int64_t)(b_v + b_a);
   a.wg_bytes = (int64_t)(b_v + b_a + b_g);
-  const size_t need = (size_t)a.wg_bytes * (size_t)grid;
+  const size_t need = b_pre + (size_t)a.wg_bytes * (size_t)grid;
   if (*ws_bytes < need) {
     if (*ws) {
       HIPCHK(hipDeviceSynchronize());
@@ -704,13 +761,37 @@ int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, c
   if (op0) a.op0 = *op0;
   a.items = d_items + first;
   a.nitems = (int32_t)count;
-  a.ws = (char*)*ws;
+  a.ws = (char*)*ws + b_pre;
   a.kcap = kcap;
   a.fixed_m = fixed_m;
   a.maxorder = maxorder;
   a.lmax = (int32_t)lmax;
   a.tol = tol;
   void* args[] = {&a};
-  HIPCHK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(NT), args, lds, s));
+  const int nsteps = pre ? op0->nsteps : 1;
+  for (int c0 = 0; c0 < nsteps; c0 += chunk) {
+    if (pre) {
+      const int nc = std::min(chunk, nsteps - c0);
+      a.op0.nsteps = nc;
+      a.op0.table = op0->table + (int64_t)c0 * op0->nslot;
+      a.op0.sflag = op0->sflag + c0;
+      if (op0->kused) a.op0.kused = op0->kused + (int64_t)c0 * op0->kused_ld;
+      if (op0->expect) a.op0.expect = op0->expect + (int64_t)c0 * op0->expect_ld;
+      const dim3 g((unsigned)((q1 - q0 + 255) / 256), (unsigned)((nc + PRE_STEPS - 1) / PRE_STEPS));
+      if (f32 && real)
+        hipLaunchKernelGGL((k_blk_operators<true, true>), g, dim3(256), 0, s, a.op0, q0, q1 - q0, (float2*)*ws);
+      else if (f32)
+        hipLaunchKernelGGL((k_blk_operators<true, false>), g, dim3(256), 0, s, a.op0, q0, q1 - q0, (float4*)*ws);
+      else if (real)
+        hipLaunchKernelGGL((k_blk_operators<false, true>), g, dim3(256), 0, s, a.op0, q0, q1 - q0, (double2*)*ws);
+      else
+        hipLaunchKernelGGL((k_blk_operators<false, false>), g, dim3(256), 0, s, a.op0, q0, q1 - q0,
+                           (PairT<false, false>::T*)*ws);
+      HIPCHK(hipGetLastError());
+      a.pre = (const char*)*ws - (int64_t)(b_step / (size_t)std::max<int64_t>(q1 - q0, 1)) * q0;
+      a.pre_ld = q1 - q0;
+    }
+    HIPCHK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(NT), args, lds, s));
+  }
   return RM_OK;
 }

@@ -402,7 +402,8 @@ struct LongItem {
   int64_t nent;
   int32_t maxrow, nslot;
   int32_t variant;   // blk_variant of its slices (0: the kernels of rm_coop.hip)
-  int64_t npairs;    // pairs of its slices
+  int64_t npairs;    // pairs of its slices, and the first one's offset
+  int64_t pair0;
   int32_t ppairs;    // and of one lane (blk_part_pairs)
 };
 // Long-domain wavepackets (rm_coop.hip): blk one workgroup each in one launch,

@@ -1793,6 +1793,7 @@ LongItem long_item(const rm_plan* p, int col, int lo, int len, int op) {
   it.nslot = p->nfield;
   const int32_t s0 = p->h_srow[lo], s1 = p->h_srow[lo + len - 1];
   it.npairs = p->h_soff[s1 + 1] - p->h_soff[s0];
+  it.pair0 = p->h_soff[s0];
   int64_t mp = 0;
   for (int32_t i = s0; i <= s1; ++i) mp = std::max<int64_t>(mp, (p->h_soff[i + 1] - p->h_soff[i]) / 64);
   it.ppairs = blk_part_pairs(s1 - s0 + 1, mp);
