@@ -206,10 +206,11 @@ int rm_plan_kernel_time(rm_plan* plan, double* total_ms, int64_t* launches);
  * step from the field table.  Applies when no MF threshold is given; results
  * equal the full-vector kernels' to rounding (entries outside the domain stay
  * exactly zero).  Domains of more than 64 rows (RM_TUNE_WAVE_MAX_ROWS; at most
- * RM_SUBSPACE_MAX_ROWS) are advanced by a cooperative launch (many
- * workgroups on one wavepacket, grid barriers between the Lanczos
+ * RM_SUBSPACE_MAX_ROWS) are advanced by teams of workgroups side by side (a
+ * few wavepackets with real operators in FP64, 961 to 3840 rows each), by a
+ * cooperative launch (many workgroups on one wavepacket, grid barriers between the Lanczos
  * reductions) when there are at most 8 of them and each holds at least
- * their count x 40000 stored entries (RM_TUNE_COOP_MAX,
+ * their count x 100000 stored entries (RM_TUNE_COOP_MAX,
  * RM_TUNE_COOP_MIN_ENTRIES), otherwise by the block kernel (one workgroup
  * per wavepacket, all in one launch).
  *
@@ -247,7 +248,7 @@ int rm_plan_set_kernel(rm_plan* plan, int32_t variant);
  *                    RM_SUBSPACE_MAX_ROWS) take the long-domain forms;
  *  RM_TUNE_COOP_MIN_ENTRIES  the cooperative form only while every long
  *                    domain holds at least (their count) x this many stored
- *                    entries (default 40000: it runs them one at a time).
+ *                    entries (default 100000: it runs them one at a time).
  * Results do not depend on these choices beyond summation order.  A change
  * drops the launch lists kept for domain reuse. */
 #define RM_TUNE_PAIR       0

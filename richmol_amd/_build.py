@@ -10,6 +10,7 @@ SOURCES = [os.path.join(PKG_DIR, "csrc", "rm_tdse.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_subspace.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_coop.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_block.hip"),
+           os.path.join(PKG_DIR, "csrc", "rm_team.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_wave.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_kron.hip"),
            os.path.join(PKG_DIR, "csrc", "rm_kprim.hip"),

@@ -5,7 +5,7 @@
 #include "rm_common.h"
 
 // pairs of entries a lane holds in registers (1024 threads leave 128 vector
-// registers: 5 each in FP64, 3 in FP32, 9 and 5 for complex operators)
+// registers; a pair takes 5 in FP64, 3 in FP32, 9 and 5 for complex operators)
 constexpr int BLK_PAIRS(bool f32, bool real) { return real ? (f32 ? 20 : 12) : (f32 ? 12 : 6); }
 constexpr int BLK_MAX_ROWS = 4096;
 

@@ -99,7 +99,7 @@ struct RmTuning {
   int32_t coop_grid = 0;   // workgroups of a cooperative launch at most (0: the domain's row groups, one per CU)
   int32_t fork = 1;        // launch classes of a call side by side on auxiliary streams
   int32_t wave_max_rows = 64;       // domains longer than this leave the one-wave kernels
-  int32_t coop_min_entries = 40000;  // stored entries per cooperative wavepacket at least
+  int32_t coop_min_entries = 100000;  // stored entries per cooperative wavepacket at least
 };
 
 struct rm_plan {
@@ -405,6 +405,9 @@ struct LongItem {
   int64_t npairs;    // pairs of its slices, and the first one's offset
   int64_t pair0;
   int32_t ppairs;    // and of one lane (blk_part_pairs)
+  int32_t nslices, maxpairs;   // its slices, the pairs of its longest row
+  bool real;         // real operator
+  int32_t team;      // workgroups of the team kernel (rm_team.hip) on it, 0: not for that kernel
 };
 // Long-domain wavepackets (rm_coop.hip): blk one workgroup each in one launch,
 // coop the whole device each (one cooperative launch each).  d_ops, d_blk,

@@ -21,11 +21,11 @@
 // 16 n bytes per wavepacket.
 //
 // Measured (MI355X, J <= 80 all m: 708 561 states, 64 wavepackets, Krylov
-// dimension 12, dipole + full polarizability in an XY field): 22.3 ms per step
-// FP64, 18.3 ms with FP32 products, where the dense form (m-mixed input stored,
+// dimension 12, dipole + full polarizability in an XY field): 20.5 ms per step
+// FP64, 17.7 ms with FP32 products, where the dense form (m-mixed input stored,
 // rocBLAS products) takes 157.5 and 112.2 ms; J <= 31, 16 wavepackets, adaptive,
-// <cos^2> read: 0.37 ms per step against 4.8.  Of the 22.3 ms the stencils take
-// 11.7 (0.97 each), the vector updates 6.1 (0.55 each: 2.9 GB at 5.3 TB/s), the
+// <cos^2> read: 0.37 ms per step against 4.8.  Of the 20.5 ms the stencils take
+// 10.7 (0.89 each), the vector updates 6.1 (0.55 each: 2.9 GB at 5.3 TB/s), the
 // final combination 1.9 (9.4 GB at 5.1 TB/s), the transforms 1.6.  Error
 // against 64-bit dense products 1e-15 (FP64); FP32 2.3e-9 (dense form 3.2e-9).
 

@@ -25,6 +25,7 @@
 #include <numeric>
 
 #include "rm_block.h"
+#include "rm_team.h"
 #include "rm_wave.h"
 
 namespace {
@@ -985,17 +986,10 @@ void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vecto
     }
 }
 
-// The sliced form of the permuted CSR arrays (rm_block.hip), with the entries
-// of subspaces of at most max_rows rows.  Built again with all that the block
-// kernel takes when it is first given a longer one (the arrays before stay
-// with the plan: launches may still read them): the cooperative form does not
-// read them, and packing and copying took 17 of 87 ms of a first call on
-// 4 subspaces of 3 000 rows.
-int slice_build(rm_plan* p, Uploader& up, int32_t max_rows, const std::vector<int64_t>& rp,
-                const std::vector<int32_t>& ccol, const std::vector<double2>& cval) {
-  const int64_t n = p->n, nnz = p->nnz;
-  const int32_t nf = std::max(p->nfield, 1);
-  std::vector<int4> sl;
+// Slices of the permuted rows (first row, rows, pairs per row, row that columns
+// count from), with room for the entries of subspaces of at most max_rows rows.
+void slice_shape(rm_plan* p, int32_t max_rows, const std::vector<int64_t>& rp, std::vector<int4>& sl,
+                 std::vector<int64_t>& off) {
   for (int32_t c = 0; c < p->nsub; ++c) {
     const int32_t lo = p->h_sub_start[c], len = p->h_sub_end[c] - lo;
     if (len <= 64 && !sl.empty() && sl.back().w == sl.back().x && sl.back().y + len <= 64 &&
@@ -1005,8 +999,8 @@ int slice_build(rm_plan* p, Uploader& up, int32_t max_rows, const std::vector<in
     }
     for (int32_t r = 0; r < len; r += 64) sl.push_back(make_int4(lo + r, std::min(64, len - r), 0, lo));
   }
-  std::vector<int64_t> off(1, 0);
-  p->h_srow.assign((size_t)n, 0);
+  off.assign(1, 0);
+  p->h_srow.assign((size_t)p->n, 0);
   for (size_t i = 0; i < sl.size(); ++i) {
     int64_t w = 0;
     for (int32_t r = sl[i].x; r < sl[i].x + sl[i].y; ++r) {
@@ -1017,6 +1011,17 @@ int slice_build(rm_plan* p, Uploader& up, int32_t max_rows, const std::vector<in
     sl[i].z = p->h_sub_end[c] - p->h_sub_start[c] <= max_rows ? (int32_t)((w + 1) / 2) : 0;
     off.push_back(off.back() + 64 * (int64_t)sl[i].z);
   }
+}
+
+// The sliced form of the permuted CSR arrays (rm_block.hip) of subspaces of at
+// most RM_SUBSPACE_MAX_ROWS rows, packed here with the plan.
+int slice_build(rm_plan* p, Uploader& up, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
+                const std::vector<double2>& cval) {
+  const int64_t n = p->n, nnz = p->nnz;
+  const int32_t nf = std::max(p->nfield, 1);
+  std::vector<int4> sl;
+  std::vector<int64_t> off;
+  slice_shape(p, RM_SUBSPACE_MAX_ROWS, rp, sl, off);
   const int64_t np = off.back();
   const int q = p->sreal ? 2 : 4;   // values of a pair
   std::vector<uint32_t> col((size_t)std::max<int64_t>(np, 1), 0);
@@ -1051,7 +1056,7 @@ int slice_build(rm_plan* p, Uploader& up, int32_t max_rows, const std::vector<in
   const int rc = up.commit(p->arenas);
   if (rc) return rc;
   p->spairs = np;
-  p->slice_rows = max_rows;
+  p->slice_rows = RM_SUBSPACE_MAX_ROWS;
   p->h_soff.swap(off);
   return RM_OK;
 }
@@ -1109,15 +1114,71 @@ int csr_build(rm_plan* p, const std::vector<double2>& B) {
   return csr_upload(p, rp, ccol, cval);
 }
 
-// Slices for a long domain of len rows.
+// A workgroup per slice: its entries from the CSR arrays (slice_build's packing).
+__global__ __launch_bounds__(256) void k_slice_pack(const int4* __restrict__ sslice, const int64_t* __restrict__ soff,
+                                                    const int64_t* __restrict__ rp, const int32_t* __restrict__ ccol,
+                                                    const double2* __restrict__ cval, int64_t nnz, int32_t nf,
+                                                    int64_t np, int32_t real, uint32_t* __restrict__ scol,
+                                                    double* __restrict__ sval, float* __restrict__ sval32) {
+  const int4 sl = sslice[blockIdx.x];
+  const int lane = threadIdx.x & 63, q = real ? 2 : 4;
+  const bool in = lane < sl.y;
+  const int64_t e0 = in ? rp[sl.x + lane] : 0, len = in ? rp[sl.x + lane + 1] - e0 : 0;
+  const uint32_t self = in ? (uint32_t)((sl.x + lane - sl.w) * 16) : 0u;   // padding: the row's own column
+  for (int p = threadIdx.x >> 6; p < sl.z; p += 4) {
+    const int64_t at = soff[blockIdx.x] + 64 * (int64_t)p + lane;
+    uint32_t c = 0;
+    for (int j = 0; j < 2; ++j)
+      c |= (2 * p + j < len ? (uint32_t)((ccol[e0 + 2 * p + j] - sl.w) * 16) : self) << (16 * j);
+    scol[at] = c;
+    for (int s = 0; s < nf; ++s)
+      for (int j = 0; j < 2; ++j) {
+        const double2 v = 2 * p + j < len ? cval[(int64_t)s * nnz + e0 + 2 * p + j] : make_double2(0.0, 0.0);
+        const int64_t d = (s * np + at) * q + (q / 2) * j;
+        sval[d] = v.x;
+        sval32[d] = (float)v.x;
+        if (!real) {
+          sval[d + 1] = v.y;
+          sval32[d + 1] = (float)v.y;
+        }
+      }
+  }
+}
+
+// Slices for a long domain of len rows: all that the block kernel takes, on
+// the device from the CSR arrays (a plan's first long domain for a kernel that
+// reads slices; packed on the host they took 50 of 125 ms of a first call on 4
+// subspaces of 3 000 rows).  The arrays before stay with the plan: launches may
+// still read them.
 int slice_need(rm_plan* p, int32_t len) {
   if (len <= p->slice_rows || len > BLK_MAX_ROWS) return RM_OK;
-  std::vector<int64_t> rp;
-  std::vector<int32_t> ccol;
-  std::vector<double2> cval;
-  csr_host(p, entry_values(p), rp, ccol, cval);
+  std::vector<int4> sl;
+  std::vector<int64_t> off;
+  slice_shape(p, BLK_MAX_ROWS, p->h_sub_rp, sl, off);
+  const int64_t np = off.back(), nval = (int64_t)std::max(p->nfield, 1) * np * (p->sreal ? 2 : 4);
   Uploader up;
-  return slice_build(p, up, BLK_MAX_ROWS, rp, ccol, cval);
+  up.add(&p->sslice, sl.data(), (int64_t)sl.size());
+  up.add(&p->soff, off.data(), (int64_t)off.size());
+  up.add(&p->srow, p->h_srow.data(), p->n);
+  int rc = up.commit(p->arenas);
+  if (rc) return rc;
+  char* d = nullptr;
+  const size_t b_col = (sizeof(uint32_t) * (size_t)std::max<int64_t>(np, 1) + 255) & ~(size_t)255;
+  const size_t b_val = (sizeof(double) * (size_t)std::max<int64_t>(nval, 1) + 255) & ~(size_t)255;
+  HIPCHK(hipMalloc((void**)&d, b_col + b_val + b_val / 2));
+  p->arenas.push_back(d);
+  p->scol = (uint32_t*)d;
+  p->sval = (double*)(d + b_col);
+  p->sval32 = (float*)(d + b_col + b_val);
+  hipLaunchKernelGGL(k_slice_pack, dim3((unsigned)sl.size()), dim3(256), 0, 0, p->sslice, p->soff, p->sub_rp,
+                     p->sub_ccol, p->sub_cval, p->nnz, std::max(p->nfield, 1), np, p->sreal ? 1 : 0, p->scol, p->sval,
+                     p->sval32);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(0));
+  p->spairs = np;
+  p->slice_rows = BLK_MAX_ROWS;
+  p->h_soff.swap(off);
+  return RM_OK;
 }
 
 // Connected components of the sparsity graph (host union-find), the row
@@ -1209,7 +1270,7 @@ int sub_build(rm_plan* p) {
   std::vector<double2> cval;
   csr_host(p, B, rp, ccol, cval);
   operator_flags(p, rp, ccol, cval);
-  if ((rc = slice_build(p, up, RM_SUBSPACE_MAX_ROWS, rp, ccol, cval))) return rc;
+  if ((rc = slice_build(p, up, rp, ccol, cval))) return rc;
   // CSR (row-major, permuted) for the cooperative kernel: if some subspace does not fit
   if (mx > RM_SUBSPACE_MAX_ROWS && (rc = csr_upload(p, rp, ccol, cval))) return rc;
   p->sub_w = W;
@@ -1374,6 +1435,8 @@ struct SubScratch {
   void* long_ws = nullptr;   // the long-domain kernels' workspace (rm_coop.hip)
   void* blk_ws = nullptr;    // the block kernel's (rm_block.hip)
   size_t blk_ws_bytes = 0;
+  void* team_ws = nullptr;   // the team kernel's (rm_team.hip)
+  size_t team_ws_bytes = 0;
   // launch classes run concurrently on auxiliary streams (default priority)
   hipStream_t aux[NCLASS + 1] = {};
   hipEvent_t fork = nullptr;
@@ -1407,6 +1470,7 @@ void scratch_release(SubScratch* sc) {
   if (sc->kept_host) (void)hipHostFree(sc->kept_host);
   coop_scratch_release(sc->long_ws);
   if (sc->blk_ws) (void)hipFree(sc->blk_ws);
+  if (sc->team_ws) (void)hipFree(sc->team_ws);
   for (int i = 0; i <= NCLASS; ++i) {
     if (sc->aux[i]) {
       (void)hipStreamSynchronize(sc->aux[i]);
@@ -1558,7 +1622,13 @@ int launch_all(SubScratch* sc, const SubArgs& a0, const int4* const (&items)[NCL
     nb = e;
   }
   const std::vector<LongItem> rest(blk.begin() + nb, blk.end());
-  rc = long_run(&sc->long_ws, a0.ops, d_blk + nb, rest, d_coop, coop, kcap, fixed_m, maxorder, tol, f32, n_cu, bs,
+  // the wavepackets for several workgroups each: side by side by teams, or the whole device on one after another
+  const std::vector<LongItem> none;
+  const int team = f32 || coop.empty() ? 0 : coop[0].team;
+  if (team && (rc = team_run(&sc->team_ws, &sc->team_ws_bytes, a0.ops, a0.ops ? nullptr : &a0.op0, d_coop, coop, team,
+                             kcap, fixed_m, maxorder, tol, n_cu, bs, abort_preset)))
+    return rc;
+  rc = long_run(&sc->long_ws, a0.ops, d_blk + nb, rest, d_coop, team ? none : coop, kcap, fixed_m, maxorder, tol, f32, n_cu, bs,
                 abort_preset, a0.ops ? nullptr : &a0.op0, tn.coop_grid);
   if (rc) return rc;
   if (fork && !blk.empty()) HIPCHK(hipEventRecord(sc->join[nused - 1], bs));
@@ -1779,6 +1849,8 @@ extern "C" int rm_plan_set_precision(rm_plan* p, int32_t precision) {
   if (precision != RM_PREC_FP64 && precision != RM_PREC_FP32)
     return fail(RM_ERR_ARG, "rm_plan_set_precision: unknown precision %d", precision);
   p->precision = precision;
+  // the long domains of kept launch lists were routed under the old one
+  if (p->sub_scratch) ((SubScratch*)p->sub_scratch)->kept = false;
   return RM_OK;
 }
 
@@ -1794,8 +1866,12 @@ LongItem long_item(const rm_plan* p, int col, int lo, int len, int op) {
   const int32_t s0 = p->h_srow[lo], s1 = p->h_srow[lo + len - 1];
   it.npairs = p->h_soff[s1 + 1] - p->h_soff[s0];
   it.pair0 = p->h_soff[s0];
-  int64_t mp = 0;
+  int64_t mp = (mr + 1) / 2;
   for (int32_t i = s0; i <= s1; ++i) mp = std::max<int64_t>(mp, (p->h_soff[i + 1] - p->h_soff[i]) / 64);
+  it.nslices = s1 - s0 + 1;
+  it.maxpairs = (int32_t)std::min<int64_t>(mp, INT32_MAX);
+  it.real = p->sreal;
+  it.team = 0;
   it.ppairs = blk_part_pairs(s1 - s0 + 1, mp);
   it.variant = len <= BLK_MAX_ROWS ? blk_variant(s1 - s0 + 1, p->sreal) : 0;
   return it;
@@ -2013,28 +2089,36 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
       }
     }
     if (!big.empty() && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
+    // a few real ones in FP64 go to teams of workgroups (rm_team.hip).  Else
     // the cooperative form runs its wavepackets one launch after another on
     // many workgroups, the block form all of them at once, one workgroup
-    // each: cooperative while the count times a cooperative step (~50-70 us)
-    // stays below one workgroup's on the smallest of them (~25 us + 1.35 ns
+    // each: cooperative while the count times a cooperative step (~50-65 us)
+    // stays below one workgroup's on the smallest of them (~15 us + 0.45 ns
     // per stored entry), i.e. count * coop_min_entries <= its entries.
-    // Measured (water-like top, adaptive, us per step, block / cooperative):
-    // 1 wavepacket of 24 046 entries 61 / 57, 49 218: 77 / 61, 370 802: 501 / 79;
-    // 4 of 88 706: 136 / 224, of 151 010: 213 / 236, of 241 442: 348 / 258;
-    // 8 of 367 402: 532 / 551.
+    // Measured (water-like top, FP32, adaptive, us per step, block / cooperative):
+    // 1 wavepacket of 49 218 entries 39 / 47, 90 372: 57 / 50, 153 186: 77 / 53,
+    // 370 802: 172 / 62; 2 of 151 010: 78 / 104, 241 442: 125 / 118, 367 402:
+    // 175 / 125; 4 of 367 402: 176 / 254.
     int64_t emin = INT64_MAX;
     int32_t longest = 0;
+    std::vector<LongItem> lbig;
     for (const int4& it : big) {
-      emin = std::min<int64_t>(emin, p->h_sub_rp[it.y + it.z] - p->h_sub_rp[it.y]);
+      lbig.push_back(long_item(p, it.x, it.y, it.z, 0));
+      emin = std::min<int64_t>(emin, lbig.back().nent);
       longest = std::max(longest, std::min<int32_t>(it.z, BLK_MAX_ROWS));
     }
-    const bool to_coop = force == RM_KERNEL_COOP ||
+    const int team = force == RM_KERNEL_BLOCK || p->precision != RM_PREC_FP64 || p->tune.coop_max == 0
+                         ? 0
+                         : team_size(lbig, p->n_cu, p->tune.coop_grid, force == RM_KERNEL_COOP);
+    const bool to_coop = force == RM_KERNEL_COOP || team > 0 ||
                          (force == 0 && (int64_t)big.size() <= p->tune.coop_max &&
                           (int64_t)big.size() * p->tune.coop_min_entries <= emin);
-    // before the items: they hold their domains' slice widths
-    if (!to_coop && (rc = slice_need(p, longest))) return rc;
-    for (const int4& it : big)
+    // before the items that are kept: they hold their domains' slice widths
+    if ((!to_coop || team > 0) && (rc = slice_need(p, longest))) return rc;
+    for (const int4& it : big) {
       (to_coop ? sc->kept_coop : sc->kept_blk).push_back(long_item(p, it.x, it.y, it.z, 0));
+      if (to_coop) sc->kept_coop.back().team = team;
+    }
     sort_long(sc->kept_blk);
     for (auto& v : sc->kept_cls) longest_first(v);
     group_pairs(sc->kept_cls, krylov_fixed, p->tune.pair != 0, p->sreal ? 0 : COMPLEX4_CLASS);

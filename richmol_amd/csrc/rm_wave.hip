@@ -14,6 +14,11 @@
 // recursion.  Per half of a pair every operation is lane- or row-local, so a
 // wavepacket's result does not depend on its partner; a half that has stopped
 // (adaptive rule) keeps its coefficients while its partner goes on.
+//
+// Bound by the latency of the recurrence; LDS per wave sets how many run beside
+// each other (8 per CU).  Measured: 4096 wavepackets, J <= 60, adaptive, 40 steps,
+// 477 us against 1 830 with a wave per wavepacket on entries read at every
+// matvec (776 before the real exponential and the smaller Gram block).
 
 #include <algorithm>
 
