@@ -222,12 +222,10 @@ template <bool FIXED, bool F32, bool REAL, int RS, bool REG>
 __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int b, int lo, int len, int wv,
                                          char* s_dyn, double2* s_w, double2* s_part, BlkShared<FIXED>& sh,
                                          double2* __restrict__ V, char* base, int& half) {
-  using XT = typename XType<F32>::T;
   using PT = typename PairT<F32, REAL>::T;
   constexpr int NP = REG ? BLK_PAIRS(F32, REAL) : 1;
   const int lane = threadIdx.x & 63;
   const double2 zero = make_double2(0.0, 0.0);
-  XT* s_x = (XT*)s_dyn;   // [lmax] matvec input, at the start of LDS: gathers address it by offset
   PT* Ast = (PT*)(base + a.offA);
   const int ns0 = op.srow[lo], nsl = op.srow[lo + len - 1] - ns0 + 1;   // the domain's slices
   const int G = RS == 1 ? NWORK / nsl : 1;       // parts per slice
@@ -273,16 +271,15 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
     }
   }
   int built = -1;
-  // acc += a pair's two products; c: the two columns' offsets in units of 16
-  // bytes of an FP64 vector
-  auto gather = [&](uint32_t c, const PT& v, XT& acc) __attribute__((always_inline)) {
-    constexpr int sh1 = F32 ? 1 : 0;
-    const XT x0 = *(const XT*)(s_dyn + ((c & 0xffffu) >> sh1)), x1 = *(const XT*)(s_dyn + (c >> (16 + sh1)));
+  // acc += a pair's two products; c: the two columns' offsets in
+  // bytes of the vector
+  auto gather = [&](uint32_t c, const PT& v, double2& acc) __attribute__((always_inline)) {
+    const double2 x0 = *(const double2*)(s_dyn + (c & 0xffffu)), x1 = *(const double2*)(s_dyn + (c >> 16));
     pair_mac(v, x0, x1, acc);
   };
   // the row's sum with pairs read from q
-  auto row_sum = [&](int r, const PT* __restrict__ q) __attribute__((always_inline)) -> XT {
-    XT acc = to_x<F32>(zero), acc2 = to_x<F32>(zero);
+  auto row_sum = [&](int r, const PT* __restrict__ q) __attribute__((always_inline)) -> double2 {
+    double2 acc = zero, acc2 = zero;
     const uint32_t* __restrict__ qc = op.scol;
     constexpr int U = 4;   // pairs loaded together (8: more spilled registers, 7 % slower)
     int p = 0;
@@ -303,14 +300,11 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
       }
     }
     for (; p < n; ++p) gather(qc[e0[r] + 64 * p] + cb[r], q[e0[r] + 64 * p], acc);
-    acc.x += acc2.x;
-    acc.y += acc2.y;
-    return acc;
+    return cadd(acc, acc2);
   };
   auto publish = [&](int r) __attribute__((always_inline)) {
     if (own && ok[r]) {
-      s_x[row[r]] = to_x<F32>(W[r]);
-      if (F32) s_w[row[r]] = W[r];
+      s_w[row[r]] = W[r];
     }
   };
   // <psi|O|psi> after step `step` (the state in S)
@@ -404,23 +398,23 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
           // complex field products of a real operator: slot by slot
           y = zero;
           for (int s = 0; s < nslot; ++s) {
-            XT t = to_x<F32>(zero);
+            double2 tot = zero;
             for (int p = 0; ok[r] && p < np[r]; ++p) {
               PT v;
               pair_round(pair_load<REAL>(op, s, e0[r] + 64 * p), v);
-              gather(op.scol[e0[r] + 64 * p] + cb[r], v, t);
+              gather(op.scol[e0[r] + 64 * p] + cb[r], v, tot);
             }
-            y = fmac(fp[s], to_d2(t), y);
+            y = fmac(fp[s], tot, y);
           }
         } else {
-          XT acc;
+          double2 acc;
           if constexpr (REG) {
             // (the empty asm: without it the compiler spills 470 registers in
             // the FP64 kernel of a fixed dimension, 50 us an iteration)
 #pragma unroll
             for (int p = 0; p < NP; ++p) keep(A[p]);
-            XT acc1 = to_x<F32>(zero);
-            acc = to_x<F32>(zero);
+            double2 acc1 = zero;
+            acc = zero;
 #pragma unroll
             for (int p = 0; p < NP; p += 2) {
               // (the empty asm keeps the columns packed: unpacked ahead of the
@@ -432,14 +426,13 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
                 gather(cc[p + 1], A[p + 1], acc1);
               }
             }
-            acc.x += acc1.x;
-            acc.y += acc1.y;
+            acc = cadd(acc, acc1);
           } else if (nslot == 1) {
             acc = row_sum(r, F32 ? (const PT*)op.sval32 : (const PT*)op.sval);
           } else {
             acc = row_sum(r, a.pre ? (const PT*)a.pre + (int64_t)built * a.pre_ld : Ast - op.soff[ns0]);
           }
-          y = cmul(f0, to_d2(acc));
+          y = cmul(f0, acc);
         }
         y = cscale(ib, y);
         yp[r] = ok[r] ? y : zero;
@@ -566,10 +559,8 @@ __device__ __forceinline__ void blk_work(const BlkArgs& a, const SubOp& op, int 
 
 template <bool FIXED, bool F32, bool REAL, int RS, bool REG>
 __global__ __launch_bounds__(NT) void k_blk(BlkArgs a) {
-  using XT = typename XType<F32>::T;
   extern __shared__ char s_dyn[];
-  // W in FP64: the matvec input itself, or beside it
-  double2* s_w = F32 ? (double2*)(s_dyn + sizeof(XT) * (size_t)((a.lmax + 1) & ~1)) : (double2*)s_dyn;
+  double2* s_w = (double2*)s_dyn;   // [lmax] W, the matvec input, at the start of LDS: gathers address it by offset
   __shared__ double2 s_part[RS == 1 ? NWORK * 64 : 1];   // partial sums of parts 1..
   __shared__ BlkShared<FIXED> sh;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -605,10 +596,7 @@ const void* blk_kernel(bool fixed, bool f32, bool real) {
   return k[4 * fixed + 2 * f32 + real];
 }
 
-size_t lds_bytes(int64_t lmax, bool f32) {
-  return f32 ? (size_t)((lmax + 1) & ~1ll) * sizeof(float2) + sizeof(double2) * (size_t)lmax
-             : sizeof(double2) * (size_t)lmax;
-}
+size_t lds_bytes(int64_t lmax) { return sizeof(double2) * (size_t)lmax; }
 
 }  // namespace
 
@@ -661,7 +649,7 @@ int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, c
   const bool pre = !reg && op0 && op0->nslot > 1 && op0->nsteps > 0;
   const int chunk = !pre ? INT32_MAX : (int)std::max<int64_t>(1, std::min<int64_t>(op0->nsteps, PRE_BYTES / b_step));
   const size_t b_pre = pre ? al256(b_step * (size_t)chunk) : 0;
-  const size_t lds = lds_bytes(lmax, f32);
+  const size_t lds = lds_bytes(lmax);
   int occ = 0;
   HIPCHK(occupancy(kern, NT, lds, &occ));
   if (occ < 1) return fail(RM_ERR_ARG, "block propagation: a domain of %lld rows does not fit LDS", (long long)lmax);

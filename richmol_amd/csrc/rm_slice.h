@@ -17,23 +17,22 @@ template <> struct PairT<true, false> { using T = float4; };
 __device__ __forceinline__ double2 fmac(double2 a, double2 b, double2 c) {
   return make_double2(fma(a.x, b.x, fma(-a.y, b.y, c.x)), fma(a.x, b.y, fma(a.y, b.x, c.y)));
 }
-__device__ __forceinline__ float2 fmac(float2 a, float2 b, float2 c) {
-  return make_float2(fmaf(a.x, b.x, fmaf(-a.y, b.y, c.x)), fmaf(a.x, b.y, fmaf(a.y, b.x, c.y)));
-}
 // acc += pair . (x0, x1)
 __device__ __forceinline__ void pair_mac(double2 p, double2 x0, double2 x1, double2& acc) {
   acc.x = fma(p.y, x1.x, fma(p.x, x0.x, acc.x));
   acc.y = fma(p.y, x1.y, fma(p.x, x0.y, acc.y));
 }
-__device__ __forceinline__ void pair_mac(float2 p, float2 x0, float2 x1, float2& acc) {
-  acc.x = fmaf(p.y, x1.x, fmaf(p.x, x0.x, acc.x));
-  acc.y = fmaf(p.y, x1.y, fmaf(p.x, x0.y, acc.y));
+// (FP32 entries: the vector and the sum stay FP64.  Their own loads are what
+// FP32 saves; the gathers and sums in FP32 were no faster, and added one by one
+// they lost up to 1.8 times more than the sums of 16 lanes per row did)
+__device__ __forceinline__ void pair_mac(float2 p, double2 x0, double2 x1, double2& acc) {
+  pair_mac(make_double2(p.x, p.y), x0, x1, acc);
 }
 __device__ __forceinline__ void pair_mac(const PairT<false, false>::T& p, double2 x0, double2 x1, double2& acc) {
   acc = fmac(p.b, x1, fmac(p.a, x0, acc));
 }
-__device__ __forceinline__ void pair_mac(float4 p, float2 x0, float2 x1, float2& acc) {
-  acc = fmac(make_float2(p.z, p.w), x1, fmac(make_float2(p.x, p.y), x0, acc));
+__device__ __forceinline__ void pair_mac(float4 p, double2 x0, double2 x1, double2& acc) {
+  acc = fmac(make_double2(p.z, p.w), x1, fmac(make_double2(p.x, p.y), x0, acc));
 }
 // a pair's value as the compiler must take it from here on
 __device__ __forceinline__ void keep(double2& v) { asm volatile("" : "+v"(v.x)); }

@@ -51,7 +51,6 @@ __device__ __attribute__((noinline)) void long_expm(int k, const double2* alpha,
 
 template <bool FIXED, bool F32, bool REAL, bool PAIR, int NP>
 __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
-  using XT = typename XType<F32>::T;
   using PT = typename PairT<F32, REAL>::T;
   constexpr int H = PAIR ? 2 : 1;         // wavepackets per wave
   constexpr int LP = 64 / H;              // lanes of each
@@ -61,8 +60,8 @@ __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
   // LDS: matvec input, basis [lb][64] (between steps the observable's state),
   // alpha and beta per half (kl of them), coefficients
   const int kl = lds_orders(kc, FIXED);
-  XT* s_x = (XT*)s_dyn;
-  double2* s_V = (double2*)(s_dyn + 64 * sizeof(XT));
+  double2* s_x = (double2*)s_dyn;
+  double2* s_V = (double2*)(s_dyn + 64 * sizeof(double2));
   double2* s_o = s_V;
   double2* s_al = s_V + (size_t)lb * 64;                   // [H][kl]
   double* s_be = (double*)(s_al + (size_t)H * kl);         // [H][kl + 1]
@@ -164,9 +163,8 @@ __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
       wave_sync();   // s_o is rewritten only after these reads
     };
     // acc += a pair's two products (columns as byte offsets of an FP64 vector)
-    auto gather = [&](uint32_t c, const PT& v, XT& acc) __attribute__((always_inline)) {
-      constexpr int sh = F32 ? 1 : 0;
-      const XT x0 = *(const XT*)(s_dyn + ((c & 0xffffu) >> sh)), x1 = *(const XT*)(s_dyn + (c >> (16 + sh)));
+    auto gather = [&](uint32_t c, const PT& v, double2& acc) __attribute__((always_inline)) {
+      const double2 x0 = *(const double2*)(s_dyn + (c & 0xffffu)), x1 = *(const double2*)(s_dyn + (c >> 16));
       pair_mac(v, x0, x1, acc);
     };
 
@@ -182,8 +180,10 @@ __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
       const double2* fp = op.table + (int64_t)step * nslot;
       // the step's operator from the real field products, unless it is the one
       // already built; with one slot B_0 itself is used and its sums are scaled
+      // (not in FP32: the rounding of B_0 would add up over the steps, that of
+      // F B_0 differs from step to step)
       bool imag = false;
-      if (nslot > 1) {
+      if (nslot > 1 || F32) {
         bool same = built >= 0;
         const double2* fb = op.table + (int64_t)max(built, 0) * nslot;
         for (int s = 0; s < nslot; ++s) {
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
           }
         }
       }
-      const double2 f0 = nslot == 1 ? fp[0] : make_double2(1.0, 0.0);
+      const double2 f0 = nslot == 1 && !F32 ? fp[0] : make_double2(1.0, 0.0);
       const bool realal = REAL && (op.sflags & 1) && !imag && f0.y == 0.0;
       const bool realexp = realal && op.f.x == 0.0;
       auto matvec = [&]() __attribute__((always_inline)) -> double2 {
@@ -211,25 +211,23 @@ __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
           // complex field products of a real operator: slot by slot
           y = zero;
           for (int s = 0; s < nslot; ++s) {
-            XT t = to_x<F32>(zero);
+            double2 t = zero;
             for (int p = 0; ok && p < z; ++p) {
               PT v;
               pair_round(pair_load<REAL>(op, s, e0 + 64 * p), v);
               gather(op.scol[e0 + 64 * p] + cb, v, t);
             }
-            y = fmac(fp[s], to_d2(t), y);
+            y = fmac(fp[s], t, y);
           }
         } else {
-          XT acc = to_x<F32>(zero), acc1 = to_x<F32>(zero);
+          double2 acc = zero, acc1 = zero;
 #pragma unroll
           for (int p = 0; p < NP; p += 2)
             if (p < np) {
               gather(cc[p], A[p], acc);
               gather(cc[p + 1], A[p + 1], acc1);
             }
-          acc.x += acc1.x;
-          acc.y += acc1.y;
-          const double2 t = to_d2(acc);
+          const double2 t = cadd(acc, acc1);
           y = realal ? cscale(f0.x, t) : cmul(f0, t);
         }
         return ok ? y : zero;
@@ -242,7 +240,7 @@ __global__ __launch_bounds__(64, NP == 2 ? 2 : 1) void k_wav(SubArgs a) {
       bool brk = false, big = false;   // big: order beyond 16, Gram matrix in global memory
       for (int it = 0;; ++it) {
         *vec(it) = vk;
-        s_x[l] = to_x<F32>(vk);
+        s_x[l] = vk;
         wave_sync();
         if (!FIXED && brk && live && it > 0) {
           // Gram column of the restart vector, explicit dots
@@ -439,7 +437,7 @@ template <bool FIXED, bool F32, bool REAL, bool PAIR, int NP>
 hipError_t launch_k(const SubArgs& a0, int n_cu, hipStream_t s, int* waves_out, bool dry) {
   auto kern = k_wav<FIXED, F32, REAL, PAIR, NP>;
   constexpr int H = PAIR ? 2 : 1;
-  const size_t lds = 64 * (F32 ? sizeof(float2) : sizeof(double2)) +
+  const size_t lds = 64 * sizeof(double2) +
                      sizeof(double2) * (size_t)(lds_vectors(a0.kcap, FIXED) * 64 + H * lds_orders(a0.kcap, FIXED)) +
                      sizeof(double) * (size_t)(H * (lds_orders(a0.kcap, FIXED) + 1));
   int occ = 0;
