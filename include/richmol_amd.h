@@ -307,6 +307,15 @@ int rm_plan_set_domain_reuse(rm_plan* plan, int32_t on);
  * RM_DEVICE_TIMEOUT -- the timeout path without a timeout.  Default 0. */
 int rm_plan_set_coop_abort(rm_plan* plan, int32_t preset);
 
+/* Host query (no reference counterpart): the workgroups per wavepacket that
+ * the team kernel would put on nitems wavepackets with real operators in FP64
+ * on a device of n_cu compute units, 0 when it does not take them.  Per
+ * wavepacket: the rows of its domain, the 64-row slices these lie in, the
+ * pairs of stored entries of its longest row and its stored entries.
+ * max_grid: RM_TUNE_COOP_GRID; forced: RM_KERNEL_COOP was asked for. */
+int rm_team_size(int32_t nitems, const int32_t* rows, const int32_t* slices, const int32_t* pairs,
+                 const int64_t* entries, int32_t n_cu, int32_t max_grid, int32_t forced);
+
 /* sflag[s] = 1 if step s (row s of fprod_dev, nsteps x nfield complex,
  * device) makes any MF element non-zero, else 0: the `len(H.mfmat) > 0`
  * test of tdse.py:377 without thresholds.  sflag: device int32[nsteps]. */

@@ -64,6 +64,8 @@ SIGNATURES = {
     "rm_plan_set_domain_reuse": (ctypes.c_int, [_vp, ctypes.c_int32]),
     "rm_plan_set_tuning": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32]),
     "rm_plan_set_coop_abort": (ctypes.c_int, [_vp, ctypes.c_int32]),
+    "rm_team_size": (ctypes.c_int, [ctypes.c_int32, _c_i32p, _c_i32p, _c_i32p, _c_i64p, ctypes.c_int32,
+                                    ctypes.c_int32, ctypes.c_int32]),
     "rm_plan_domains": (ctypes.c_int, [_vp, _vp, ctypes.c_int64, ctypes.c_int64, _c_i32p, _vp]),
     "rm_plan_step_flags": (ctypes.c_int, [_vp, ctypes.c_int64, _vp, _vp, _vp]),
     "rm_batch_create": (ctypes.c_int, [ctypes.POINTER(_vp)]),

@@ -561,9 +561,13 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 int team_size(const std::vector<LongItem>& items, int n_cu, int32_t max_grid, bool forced) {
   if (items.empty()) return 0;
   if (max_grid > 0) n_cu = std::min<int>(n_cu, max_grid);
-  for (const LongItem& it : items)
+  int64_t lo = 2, hi = std::min<int64_t>(TEAM_MAX, n_cu / (int64_t)items.size()), emin = INT64_MAX;
+  for (const LongItem& it : items) {
     if (it.item.z <= NVL || it.item.z > TEAM_MAX_ROWS || !it.real) return 0;
-  int64_t lo = 2, hi = std::min<int64_t>(TEAM_MAX, n_cu / (int64_t)items.size());
+    // a workgroup without a slice of every item could not take part in its exchanges
+    hi = std::min<int64_t>(hi, it.nslices);
+    emin = std::min(emin, it.nent);
+  }
   for (const LongItem& it : items) {
     int64_t need = 0;
     for (int64_t t = lo; t <= hi && !need; ++t) {
@@ -573,14 +577,22 @@ int team_size(const std::vector<LongItem>& items, int n_cu, int32_t max_grid, bo
     if (!need) return 0;
     lo = std::max(lo, need);
   }
-  // more workgroups than slices of the largest domain would idle
-  int64_t ns = 0, emin = INT64_MAX;
-  for (const LongItem& it : items) {
-    ns = std::max<int64_t>(ns, it.nslices);
-    emin = std::min(emin, it.nent);
+  return forced || hi * (int64_t)items.size() * 800 <= emin ? (int)hi : 0;
+}
+
+extern "C" int rm_team_size(int32_t nitems, const int32_t* rows, const int32_t* slices, const int32_t* pairs,
+                            const int64_t* entries, int32_t n_cu, int32_t max_grid, int32_t forced) {
+  if (nitems < 0 || n_cu < 1 || (nitems > 0 && (!rows || !slices || !pairs || !entries)))
+    return fail(RM_ERR_ARG, "rm_team_size: bad arguments");
+  std::vector<LongItem> items((size_t)nitems);
+  for (int32_t i = 0; i < nitems; ++i) {
+    items[i].item = make_int4(i, 0, rows[i], 0);
+    items[i].nslices = slices[i];
+    items[i].maxpairs = pairs[i];
+    items[i].nent = entries[i];
+    items[i].real = true;
   }
-  const int64_t team = std::max(lo, std::min(hi, ns));
-  return forced || team * (int64_t)items.size() * 800 <= emin ? (int)team : 0;
+  return team_size(items, n_cu, max_grid, forced != 0);
 }
 
 int team_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, const int4* d_items,

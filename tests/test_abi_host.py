@@ -176,3 +176,32 @@ def test_rm_job_layout_matches_header(tmp_path):
     for n in names:
         assert int(out[n]) == getattr(RmJob, n).offset, n
     assert int(out["sizeof"]) == ctypes.sizeof(RmJob)
+
+
+@pytest.mark.parametrize("forced", [0, 1])
+def test_team_rule_leaves_no_workgroup_without_rows(lib, forced):
+    """Every workgroup of a team owns a slice of every wavepacket of the
+    launch and holds its part of it, whatever the mix of domain lengths."""
+    from richmol_amd import _lib
+    rng = np.random.default_rng(3)
+    seen = 0
+    for case in range(400):
+        nitems = int(rng.integers(1, 7))
+        rows = rng.integers(961, 3841, size=nitems).astype(np.int32)
+        if case == 0:
+            rows = np.array([1135, 2270], dtype=np.int32)
+            nitems = 2
+        slices = ((rows + 63) // 64 + rng.integers(0, 2, size=nitems)).astype(np.int32)
+        pairs = rng.integers(5, 65, size=nitems).astype(np.int32)
+        entries = (rows.astype(np.int64) * pairs * 2)
+        t = lib.rm_team_size(nitems, _lib.ptr(rows, ctypes.c_int32), _lib.ptr(slices, ctypes.c_int32),
+                             _lib.ptr(pairs, ctypes.c_int32), _lib.ptr(entries, ctypes.c_int64), 256, 0, forced)
+        assert t >= 0
+        if t == 0:
+            continue
+        seen += len(set(slices.tolist())) > 1
+        assert t * nitems <= 256 and t <= slices.min()
+        for n, p in zip(slices, pairs):
+            own = [int(n) * (i + 1) // t - int(n) * i // t for i in range(t)]
+            assert min(own) >= 1 and max(own) <= 15 and -(-int(p) // (15 // max(own))) <= 8
+    assert seen > 10   # mixes of lengths among them

@@ -110,6 +110,45 @@ def test_coop_timeout_path_forced(device):
     assert np.abs(ens.psi.cpu().numpy() - _oracle_steps(h0, H, X, fields, krylov=8)).max() <= 1e-10
 
 
+def test_coop_timeout_path_of_the_team_kernel(device):
+    """The same with two wavepackets on domains the team kernel takes (1 135
+    rows): bounded waits give up, the status bit, then a normal run."""
+    import torch
+    from _fixtures import water, water_fields
+    from richmol_amd import _lib
+    from richmol_amd.ensemble import Ensemble
+    from richmol_amd.tdse import TDSE
+    h0, leaves, bas = water(14)
+    n = sum((2 * J + 1) ** 2 for J in range(15))
+    fields = water_fields(395.0 + 5.0 * np.arange(3))
+    for T, F in zip(leaves, fields):
+        T.field(list(F[0]))
+    H = leaves[0] + leaves[1] + leaves[2]
+    f = TDSE(t_end=100.0, dt=5.0, t_units="fs").exp_fac
+    X = np.zeros((2, n), dtype=np.complex128)
+    X[:, 0] = [1.0, 1j]
+    out = []
+    for kern in ("coop", "global"):
+        ens = Ensemble(H, h0, f, X, krylov_fixed=6)
+        ens.set_kernel(kern)
+        table = ens.prepare(fields, per_term=True)
+        if kern == "coop":
+            print("coop abort hook: 1135-row domains, team kernel", flush=True)
+            ens.plan.set_coop_abort(True)
+            try:
+                ens.propagate(None, table=table, check=False)
+                torch.cuda.synchronize()
+                assert np.all(ens.status.cpu().numpy() & _lib.RM_DEVICE_TIMEOUT)
+                with pytest.raises(RuntimeError, match="timed out"):
+                    ens.check()
+            finally:
+                ens.plan.set_coop_abort(False)
+            ens.load(X)
+        ens.propagate(None, table=table)
+        out.append(ens.psi.cpu().numpy())
+    assert np.abs(out[0] - out[1]).max() <= 1e-11
+
+
 def test_full_vector_kernels_refuse_fp32(device):
     import torch
     from richmol_amd import _lib

@@ -3,10 +3,13 @@ operators) against the full-vector kernel on the same field table (1e-11), at
 the sizes where its layout and the rule for it change: one or more slices per
 workgroup, few and many wavepackets, adaptive and fixed Krylov dimensions,
 complex field products, steps whose products are so small that |W|^2
-underflows (the restart after a breakdown), an observable.
+underflows (the restart after a breakdown), an observable, wavepackets on
+domains of different lengths side by side without one.
 """
 import numpy as np
 import pytest
+from scipy.sparse import csr_matrix
+from scipy.sparse.csgraph import connected_components
 
 from _fixtures import linear_rotor, water, water_fields
 from test_gpu_asymtop import DT, _summed
@@ -59,3 +62,36 @@ def test_linear_rotor_observable_and_restart(device, jmax, fixed, kernel):
     obs = ensemble.Ensemble.observable_plan(cos2)
     X = _rows((jmax + 1) ** 2, 3, jmax)
     _compare(H, h0, -0.0019j, X, lambda e: e.prepare(fields), fixed, 1.0, obs, kernel)
+
+
+@pytest.mark.parametrize("order", [1, -1])
+@pytest.mark.parametrize("fixed", [0, 9])
+@pytest.mark.parametrize("kernel", ["auto", "coop"])
+def test_unequal_domains(device, order, fixed, kernel):
+    """A basis state (18 slices) beside a superposition of two species (36), no
+    observable, many exchanges: amplitudes and Krylov dimensions."""
+    import torch
+    h0, leaves, bas = water(14)
+    n = sum((2 * J + 1) ** 2 for J in range(15))
+    fields = water_fields(395.0 + DT * np.arange(12))
+    f = TDSE(t_end=20.0, dt=DT, t_units="fs").exp_fac
+    H = _summed(leaves, fields, 0)
+    e = ensemble.Ensemble(H, h0, f, np.eye(1, n, dtype=np.complex128), krylov_fixed=fixed)
+    e.prepare(fields, per_term=True)
+    arr = e.plan._arrays
+    A = csr_matrix((np.ones(arr["nnz"]), arr["col_idx"], arr["row_ptr"]), shape=(n, n))
+    _, lab = connected_components(A)
+    X = np.zeros((2, n), dtype=np.complex128)
+    X[:, np.argmax(lab == 0)] = 1.0
+    X[1, np.argmax(lab == 1)] = 1.0
+    assert e.plan.domain_sizes(X)[0].tolist() == [1135, 2255]
+    X[1] /= np.linalg.norm(X[1])
+    out = []
+    for kern in (kernel, "global"):
+        e = ensemble.Ensemble(H, h0, f, X[::order].copy(), krylov_fixed=fixed)
+        e.set_kernel(kern)
+        ku = torch.full((12, 2), -1, dtype=torch.int32, device=device)
+        e.propagate(None, table=e.prepare(fields, per_term=True), kused=ku)
+        out.append((e.psi.cpu().numpy(), ku.cpu().numpy()))
+    assert np.abs(out[0][0] - out[1][0]).max() <= 1e-11
+    assert np.array_equal(out[0][1], out[1][1])
