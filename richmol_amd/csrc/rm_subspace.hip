@@ -1148,33 +1148,44 @@ __global__ __launch_bounds__(256) void k_slice_pack(const int4* __restrict__ ssl
 // Slices for a long domain of len rows: all that the block kernel takes, on
 // the device from the CSR arrays (a plan's first long domain for a kernel that
 // reads slices; packed on the host they took 50 of 125 ms of a first call on 4
-// subspaces of 3 000 rows).  The arrays before stay with the plan: launches may
-// still read them.
+// subspaces of 3 000 rows).  They enter the plan together once everything has
+// succeeded: after an error it holds what it held before.  The arrays before
+// stay with the plan: launches may still read them.
 int slice_need(rm_plan* p, int32_t len) {
   if (len <= p->slice_rows || len > BLK_MAX_ROWS) return RM_OK;
   std::vector<int4> sl;
   std::vector<int64_t> off;
   slice_shape(p, BLK_MAX_ROWS, p->h_sub_rp, sl, off);
   const int64_t np = off.back(), nval = (int64_t)std::max(p->nfield, 1) * np * (p->sreal ? 2 : 4);
-  Uploader up;
-  up.add(&p->sslice, sl.data(), (int64_t)sl.size());
-  up.add(&p->soff, off.data(), (int64_t)off.size());
-  up.add(&p->srow, p->h_srow.data(), p->n);
-  int rc = up.commit(p->arenas);
-  if (rc) return rc;
+  const size_t bytes[6] = {sizeof(int4) * sl.size(), sizeof(int64_t) * off.size(), sizeof(int32_t) * (size_t)p->n,
+                           sizeof(uint32_t) * (size_t)np, sizeof(double) * (size_t)nval, sizeof(float) * (size_t)nval};
+  const void* src[6] = {sl.data(), off.data(), p->h_srow.data(), nullptr, nullptr, nullptr};
+  size_t at[7] = {0};
+  for (int i = 0; i < 6; ++i) at[i + 1] = (at[i] + bytes[i] + 255) & ~(size_t)255;
   char* d = nullptr;
-  const size_t b_col = (sizeof(uint32_t) * (size_t)std::max<int64_t>(np, 1) + 255) & ~(size_t)255;
-  const size_t b_val = (sizeof(double) * (size_t)std::max<int64_t>(nval, 1) + 255) & ~(size_t)255;
-  HIPCHK(hipMalloc((void**)&d, b_col + b_val + b_val / 2));
+  HIPCHK(hipMalloc((void**)&d, std::max<size_t>(at[6], 1)));
+  auto fill = [&]() -> int {
+    for (int i = 0; i < 3; ++i) HIPCHK(hipMemcpy(d + at[i], src[i], bytes[i], hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_slice_pack, dim3((unsigned)sl.size()), dim3(256), 0, 0, (const int4*)(d + at[0]),
+                       (const int64_t*)(d + at[1]), p->sub_rp, p->sub_ccol, p->sub_cval, p->nnz,
+                       std::max(p->nfield, 1), np, p->sreal ? 1 : 0, (uint32_t*)(d + at[3]), (double*)(d + at[4]),
+                       (float*)(d + at[5]));
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(0));
+    return RM_OK;
+  };
+  const int rc = fill();
+  if (rc) {
+    (void)hipFree(d);
+    return rc;
+  }
   p->arenas.push_back(d);
-  p->scol = (uint32_t*)d;
-  p->sval = (double*)(d + b_col);
-  p->sval32 = (float*)(d + b_col + b_val);
-  hipLaunchKernelGGL(k_slice_pack, dim3((unsigned)sl.size()), dim3(256), 0, 0, p->sslice, p->soff, p->sub_rp,
-                     p->sub_ccol, p->sub_cval, p->nnz, std::max(p->nfield, 1), np, p->sreal ? 1 : 0, p->scol, p->sval,
-                     p->sval32);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(0));
+  p->sslice = (int4*)(d + at[0]);
+  p->soff = (int64_t*)(d + at[1]);
+  p->srow = (int32_t*)(d + at[2]);
+  p->scol = (uint32_t*)(d + at[3]);
+  p->sval = (double*)(d + at[4]);
+  p->sval32 = (float*)(d + at[5]);
   p->spairs = np;
   p->slice_rows = BLK_MAX_ROWS;
   p->h_soff.swap(off);

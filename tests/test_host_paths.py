@@ -1,0 +1,148 @@
+"""Host paths of the library on the CPU, in a process whose HIP runtime is
+hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
+recorded and allocations can be made to fail.  What a plan's launches read after
+an allocation failed.
+"""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+P = ctypes.c_void_p
+LONG, SHORT, BAND = 2000, 300, 60   # rows of the two subspaces, half the band
+
+
+def _matrix():
+    """A real band matrix of a long subspace (first) and a short one, two slots."""
+    rng = np.random.default_rng(0)
+    rows, cols = [], []
+    for lo, n in ((0, LONG), (LONG, SHORT)):
+        for i in range(n):
+            c = np.arange(max(0, i - BAND), min(n, i + BAND + 1))
+            rows.append(np.full(c.size, lo + i))
+            cols.append(lo + c)
+    rows, cols = np.concatenate(rows), np.concatenate(cols)
+    return rows, cols.astype(np.int32), rng.normal(size=(2, rows.size))
+
+
+class Stub:
+    def __init__(self, lib_path, stub_path):
+        from richmol_amd import _lib
+        self.lib, self.stub = ctypes.CDLL(lib_path), ctypes.CDLL(stub_path)
+        for name, (res, args) in _lib.SIGNATURES.items():
+            if hasattr(self.lib, name):
+                getattr(self.lib, name).restype, getattr(self.lib, name).argtypes = res, args
+        self.stub.stub_launch.restype = P
+        self.rows, self.cols, self.vals = _matrix()
+        self.n = n = LONG + SHORT
+        nnz = self.rows.size
+        i64, i32 = np.int64, np.int32
+        ptr = np.zeros(n + 1, i64)
+        np.add.at(ptr, self.rows + 1, 1)
+        ptr = np.cumsum(ptr).astype(i64)
+        kval = np.zeros((nnz, 2, 2))
+        kval[:, :, 0] = self.vals.T
+        a = [ptr, self.cols, np.arange(nnz + 1, dtype=i64) * 2, np.tile(np.array([0, 1], i32), nnz), kval,
+             np.array([0, 1, 2], i64), np.array([0, 1], i32), np.array([1.0, 0.0, 1.0, 0.0]), np.zeros(2, i32)]
+        q = [x.ctypes.data_as(t) for x, t in zip(a, _lib.SIGNATURES["rm_plan_create"][1][2:7])]
+        t = [x.ctypes.data_as(t) for x, t in zip(a[5:], _lib.SIGNATURES["rm_plan_create"][1][8:12])]
+        self.plan = P()
+        assert self.lib.rm_plan_create(n, nnz, *q, 2, *t, 2, 1, ctypes.byref(self.plan)) == 0
+        self.batch = P()
+        assert self.lib.rm_batch_create(ctypes.byref(self.batch)) == 0
+        assert self.lib.rm_batch_set_block_rows(self.batch, 64) == 0
+        self.table, self.flags = np.ones((3, 2), np.complex128), np.ones(3, i32)
+        self.psi, self.work = np.zeros((1, n), np.complex128), np.zeros((1, n), np.complex128)
+
+    def job(self, lo, n):
+        """A batch job on one domain; the library's status."""
+        from richmol_amd import _lib
+        j = _lib.RmJob(plan=self.plan, psi=self.psi.ctypes.data, ld=self.n, col=0, lo=lo, len=n,
+                       fprod_dev=self.table.ctypes.data, sflag_dev=self.flags.ctypes.data, nsteps=3, f_re=0.0,
+                       f_im=-0.1, phase=None, kused=None, status=None)
+        self.stub.stub_clear()
+        return self.lib.rm_batch_propagate(self.batch, ctypes.byref(j), 1, ctypes.sizeof(j), 6, 100, 1e-15, 0, None)
+
+    def launches(self, kernel):
+        """(first argument as 64-bit words, second, third) of the recorded launches of a kernel."""
+        out = []
+        for i in range(self.stub.stub_count()):
+            at = self.stub.stub_launch(i)
+            if kernel in ctypes.string_at(at).decode():
+                w = np.frombuffer(ctypes.string_at(at + 96, 66 * 8), np.uint64)
+                out.append(([int(x) for x in w[:64]], int(w[64]), int(w[65])))
+        return out
+
+    def check_operator(self, op, lo, n):
+        """The sliced operator a launch reads (a SubOp's words: sslice 7, soff 8,
+        srow 9, scol 10, sval 11, npairs 13) holds the domain's rows."""
+        def arr(word, dtype, count, off=0):
+            nb = np.dtype(dtype).itemsize
+            return np.frombuffer(ctypes.string_at(op[word] + off * nb, count * nb), dtype)
+        npairs = op[13]
+        for r in range(lo, lo + n, 7):
+            s = int(arr(9, np.int32, 1, r)[0])
+            x, rows, z, w = (int(v) for v in arr(7, np.int32, 4, 4 * s))
+            e0 = int(arr(8, np.int64, 1, s)[0]) + r - x
+            assert 0 <= r - x < rows and 0 <= e0 and e0 + 64 * (z - 1) < npairs
+            got = np.zeros((2, self.n))
+            for p in range(z):
+                c = int(arr(10, np.uint32, 1, e0 + 64 * p)[0])
+                for q in range(2):
+                    v = arr(11, np.float64, 2, 2 * (q * npairs + e0 + 64 * p))
+                    got[q, w + ((c & 0xffff) >> 4)] += v[0]
+                    got[q, w + (c >> 20)] += v[1]
+            ref = np.zeros((2, self.n))
+            sel = self.rows == r
+            ref[:, self.cols[sel]] = self.vals[:, sel]
+            assert np.array_equal(got, ref), r
+
+    def check_job(self, lo, n):
+        (words, _, _), = self.launches("k_blk")
+        self.check_operator([int(x) for x in np.frombuffer(ctypes.string_at(words[0], 8 * 14), np.uint64)], lo, n)
+
+
+def case_failed_allocation(s):
+    """Every device allocation of a plan's first long domain fails in turn;
+    short domains before, in between and after read their own entries."""
+    assert s.job(LONG, SHORT) == 0
+    s.check_job(LONG, SHORT)
+    failed = 0
+    for k in range(1, 20):
+        s.stub.stub_fail_in(k)
+        rc = s.job(0, LONG)
+        s.stub.stub_fail_in(0)
+        assert s.job(LONG, SHORT) == 0
+        s.check_job(LONG, SHORT)
+        if rc == 0:
+            break
+        failed += 1
+    assert rc == 0 and failed >= 1
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-I/opt/rocm/include", "-o", so,
+                    os.path.join(HERE, "hip_host_stub.cpp")], check=True)
+    return so
+
+
+@pytest.mark.parametrize("case", ["failed_allocation"])
+def test_host_path(stub, case):
+    from richmol_amd import _build
+    if not os.path.exists(_build.LIB_PATH):
+        _build.build()
+    env = dict(os.environ, LD_PRELOAD=":".join(filter(None, [stub, os.environ.get("LD_PRELOAD")])))
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), case, _build.LIB_PATH, stub], env=env,
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, os.path.dirname(HERE))
+    globals()["case_" + sys.argv[1]](Stub(sys.argv[2], sys.argv[3]))
