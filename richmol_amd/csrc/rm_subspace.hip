@@ -1458,6 +1458,7 @@ struct SubScratch {
   int64_t kept_ld = 0, kept_ncols = 0;
   int kept_force = 0;
   bool kept_pairs = false;             // grouped for two wavepackets per wave
+  int32_t kept_slices = 0;             // the plan's slice_rows when they were made (they hold offsets into its slices)
   std::vector<int4> kept_cls[NCLASS];
   std::vector<LongItem> kept_blk, kept_coop;
   int4* kept_dev = nullptr;            // the kept lists' items on the device (classes, block, cooperative)
@@ -1966,7 +1967,8 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
   // not kept)
   const bool expo = p->propag == RM_PROPAG_EXPOKIT;
   const bool reuse = !expo && p->dom_reuse && sc->kept && sc->kept_psi == psi && sc->kept_ld == ld &&
-                     sc->kept_ncols == ncols && sc->kept_force == force && sc->kept_pairs == pairs;
+                     sc->kept_ncols == ncols && sc->kept_force == force && sc->kept_pairs == pairs &&
+                     sc->kept_slices == p->slice_rows;
   // step flags in chunks of <= 1024 terms, at most 16 per step; from 64
   // steps on, or for up to 8192 terms, one block per step (a step with a
   // field ends its scan at the first non-zero element, in its first pass:
@@ -2172,6 +2174,7 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
       sc->kept_ld = ld;
       sc->kept_ncols = ncols;
       sc->kept_force = force;
+      sc->kept_slices = p->slice_rows;
     }
   }
   *done = true;

@@ -1,7 +1,7 @@
 """Host paths of the library on the CPU, in a process whose HIP runtime is
 hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
 recorded and allocations can be made to fail.  What a plan's launches read after
-an allocation failed.
+an allocation failed, and after its arrays were replaced.
 """
 import ctypes
 import os
@@ -67,6 +67,11 @@ class Stub:
         self.stub.stub_clear()
         return self.lib.rm_batch_propagate(self.batch, ctypes.byref(j), 1, ctypes.sizeof(j), 6, 100, 1e-15, 0, None)
 
+    def propagate(self):
+        self.stub.stub_clear()
+        return self.lib.rm_propagate(self.plan, self.psi.ctypes.data, self.work.ctypes.data, self.n, 1, 3,
+                                     self.table.ctypes.data, None, 0.0, -0.1, None, 6, 100, 1e-15, None, None, None)
+
     def launches(self, kernel):
         """(first argument as 64-bit words, second, third) of the recorded launches of a kernel."""
         out = []
@@ -124,6 +129,27 @@ def case_failed_allocation(s):
     assert rc == 0 and failed >= 1
 
 
+def case_kept_lists(s):
+    """Launch lists kept for domain reuse, then a batch job that replaces the
+    plan's slices: the next call's operators are those of its domain."""
+    s.psi[0, LONG + 5] = 1.0
+    assert s.lib.rm_plan_set_kernel(s.plan, 6) == 0
+    assert s.lib.rm_plan_set_domain_reuse(s.plan, 1) == 0
+
+    def check():
+        assert s.propagate() == 0
+        (op, q0, count), = s.launches("k_blk_operators")
+        s0, s1 = (int(np.frombuffer(ctypes.string_at(op[9] + 4 * r, 4), np.int32)[0]) for r in (LONG, s.n - 1))
+        off = np.frombuffer(ctypes.string_at(op[8] + 8 * s0, 8 * (s1 - s0 + 2)), np.int64)
+        assert (q0, count) == (off[0], off[-1] - off[0])
+
+    check()
+    check()
+    assert s.job(0, LONG) == 0
+    check()
+    check()
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
@@ -132,7 +158,7 @@ def stub(tmp_path_factory):
     return so
 
 
-@pytest.mark.parametrize("case", ["failed_allocation"])
+@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists"])
 def test_host_path(stub, case):
     from richmol_amd import _build
     if not os.path.exists(_build.LIB_PATH):
