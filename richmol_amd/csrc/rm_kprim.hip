@@ -30,6 +30,7 @@
 // against 64-bit dense products 1e-15 (FP64); FP32 2.3e-9 (dense form 3.2e-9).
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "rm_kprim.h"
@@ -63,6 +64,7 @@ struct PJ {             // one output J
 struct PMf {            // MF assembly of one block
   int32_t dm1, nsig, ncart, slot0, dpad;
   int32_t sig[5];
+  int32_t pe;           // P is kept times 2^-pe, so that its largest element is in [1, 2)
   int64_t d_off, mf_off;
 };
 
@@ -75,6 +77,7 @@ struct KPrim {
   std::vector<double> h_C;
   bool cplx = false;               // some C has an imaginary part
   int32_t nblk = 0;
+  std::vector<PMf> h_mfd;
   const double2* mdiag = nullptr;  // the plan's
   std::vector<PJ> h_pj;
   PJ* d_pj = nullptr;
@@ -138,12 +141,12 @@ __device__ __forceinline__ float2 mac(float2 a, float2 b, float2 c) {
 __device__ __forceinline__ void conv2(double2 v, double2& o) { o = v; }
 __device__ __forceinline__ void conv2(double2 v, float2& o) { o = make_float2((float)v.x, (float)v.y); }
 
-// MF_sigma(m1) of every block for the step's field products, in the padded
-// [sigma + 2][m1] tables (entries of sigmas a block lacks stay zero), and the
+// MF_sigma(m1) of every block for the step's field products, times 2^(pe + e),
+// in the padded [sigma + 2][m1] tables (entries of sigmas a block lacks stay zero), and the
 // smallest compiled sigma set that holds the non-zero ones: a field along Z
 // leaves sigma = 0, one in the XY plane +-1 (dipole) or 0, +-2 (polarizability).
 __global__ __launch_bounds__(256) void k_pr_mf(const PMf* __restrict__ d, const double2* __restrict__ mdiag,
-                                               const double2* __restrict__ fp, double2* __restrict__ mf,
+                                               const double2* __restrict__ fp, int e, double2* __restrict__ mf,
                                                float2* __restrict__ mf32, int32_t* __restrict__ gpat) {
   const PMf b = d[blockIdx.x];
   int mask = 0;
@@ -152,6 +155,7 @@ __global__ __launch_bounds__(256) void k_pr_mf(const PMf* __restrict__ d, const 
       double2 acc = make_double2(0.0, 0.0);
       for (int c = 0; c < b.ncart; ++c)
         acc = cfma(fp[b.slot0 + c], mdiag[b.d_off + ((int64_t)t * b.ncart + c) * b.dm1 + m], acc);
+      acc = make_double2(scalbn(acc.x, b.pe + e), scalbn(acc.y, b.pe + e));
       const int64_t o = b.mf_off + (int64_t)(b.sig[t] + 2) * b.dpad + m;
       mf[o] = acc;
       mf32[o] = make_float2((float)acc.x, (float)acc.y);
@@ -742,10 +746,22 @@ int prim_work(KPrim* p, int32_t ncols, int32_t m, bool f32, bool adaptive, PWork
   return RM_OK;
 }
 
-int launch_mf(KPrim* p, const double2* fp, hipStream_t s) {
+// The step's operator is taken times 2^e so that its elements are of order 1,
+// and the exponent factor f times 2^-e: exact, and in FP32 no product of the
+// unnormalised vectors leaves the range whatever the units of H and the field
+// (in joules 1e9 V/m x 1e-21 J x 1e-30 C m is not a normal number).
+int step_exponent(const KPrim* p, const double* fprod) {
+  double top = 0.0;
+  for (const PMf& b : p->h_mfd)
+    for (int c = 0; c < b.ncart; ++c)
+      for (int q = 0; q < 2; ++q) top = std::max(top, scalbn(std::fabs(fprod[2 * (b.slot0 + c) + q]), b.pe));
+  return top > 0.0 && std::isfinite(top) ? -std::ilogb(top) : 0;
+}
+
+int launch_mf(KPrim* p, const double2* fp, int e, hipStream_t s) {
   if (p->nblk)
-    hipLaunchKernelGGL(k_pr_mf, dim3((unsigned)p->nblk), dim3(256), 0, s, p->d_mfd, p->mdiag, fp, p->d_mf, p->d_mf32,
-                       p->d_gpat);
+    hipLaunchKernelGGL(k_pr_mf, dim3((unsigned)p->nblk), dim3(256), 0, s, p->d_mfd, p->mdiag, fp, e, p->d_mf,
+                       p->d_mf32, p->d_gpat);
   HIPCHK(hipGetLastError());
   return RM_OK;
 }
@@ -857,6 +873,7 @@ int kprim_create(KPrim** out, const std::vector<int32_t>& Js, const std::vector<
     m.ncart = blk[q].ncart;
     m.slot0 = blk[q].slot0;
     for (int t = 0; t < 5; ++t) m.sig[t] = t < m.nsig ? blk[q].sig[t] : 0;
+    m.pe = 0;
     m.d_off = blk[q].d_off;
     m.mf_off = mpos;
     mpos += 5 * (int64_t)m.dpad;
@@ -881,24 +898,31 @@ int kprim_create(KPrim** out, const std::vector<int32_t>& Js, const std::vector<
       t.p_off = poff[q];
       t.mf_off = mfd[q].mf_off;
       int mask = 0;
+      double top = 0.0;
       for (int s = 0; s < 5; ++s)
         for (int64_t k = 0; k < d; ++k) {
           const double* v = P + 2 * (poff[q] + s * (int64_t)d + k);
           if (v[0] != 0.0 || v[1] != 0.0) mask |= 1 << s;
+          top = std::max(top, std::max(std::fabs(v[0]), std::fabs(v[1])));
         }
+      mfd[q].pe = top > 0.0 && std::isfinite(top) ? std::ilogb(top) : 0;
       t.spat = !(mask & ~4) ? S_0 : !(mask & ~14) ? S_1 : !(mask & ~21) ? S_02 : S_2;
       tasks.push_back(t);
     }
     j.ntask = (int32_t)tasks.size() - j.task0;
     p->h_pj.push_back(j);
   }
-  std::vector<float> p32(P, P + 2 * ppos);
+  std::vector<double> ps(P, P + 2 * ppos);
+  for (size_t q = 0; q < blk.size(); ++q)
+    for (int64_t i = 2 * poff[q]; i < 2 * (poff[q] + 5 * (int64_t)mfd[q].dm1); ++i) ps[i] = scalbn(ps[i], -mfd[q].pe);
+  const std::vector<float> p32(ps.begin(), ps.end());
+  p->h_mfd = mfd;
   const std::vector<double2> zero((size_t)std::max<int64_t>(mpos, 1), make_double2(0.0, 0.0));
   int rc;
   if ((rc = upload(&p->d_T, T.data(), (int64_t)T.size())) || (rc = upload(&p->d_toff, toff.data(), nJ)) ||
       (rc = upload(&p->d_pj, p->h_pj.data(), nJ)) || (rc = upload(&p->d_task, tasks.data(), (int64_t)tasks.size())) ||
       (rc = upload(&p->d_mfd, mfd.data(), (int64_t)mfd.size())) ||
-      (rc = upload(&p->d_p, (const double2*)P, ppos)) || (rc = upload(&p->d_p32, (const float2*)p32.data(), ppos)) ||
+      (rc = upload(&p->d_p, (const double2*)ps.data(), ppos)) || (rc = upload(&p->d_p32, (const float2*)p32.data(), ppos)) ||
       (rc = upload(&p->d_mf, zero.data(), (int64_t)zero.size())) ||
       (rc = upload(&p->d_mf32, (const float2*)zero.data(), (int64_t)zero.size())) ||
       (rc = upload(&p->d_gpat, (const int32_t*)nullptr, (int64_t)blk.size()))) {
@@ -919,7 +943,7 @@ int kprim_matvec(KPrim* p, const double2* x, double2* y, int64_t ld, int32_t nco
   int rc;
   PWork w;
   if ((rc = prim_lists(p, ncols)) || (rc = prim_work(p, ncols, 1, false, false, &w))) return rc;
-  if ((rc = launch_mf(p, fprod, s)) || (rc = launch_tr(p, true, x, ld, w.W, p->n, nullptr, ncols, s))) return rc;
+  if ((rc = launch_mf(p, fprod, 0, s)) || (rc = launch_tr(p, true, x, ld, w.W, p->n, nullptr, ncols, s))) return rc;
   double2* Y = w.W + w.vs;
   rc = f32 ? launch_sten<float, double>(p, w.W, ncols, nullptr, Y, nullptr, s)
            : launch_sten<double, double>(p, w.W, ncols, nullptr, Y, nullptr, s);
@@ -936,7 +960,7 @@ int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t n
   int rc;
   PWork w;
   if ((rc = prim_lists(p, ncols)) || (rc = prim_work(p, ncols, m, f32, adaptive, &w))) return rc;
-  if (obs && ((rc = prim_lists(obs, ncols)) || (rc = launch_mf(obs, d_ofp, s)))) return rc;
+  if (obs && ((rc = prim_lists(obs, ncols)) || (rc = launch_mf(obs, d_ofp, 0, s)))) return rc;
   const unsigned ne = (unsigned)((p->n + EB - 1) / EB);
   const dim3 eg(ne, (unsigned)ncols), eb(256), cg((unsigned)ncols), cb(64);
   const bool rule = adaptive && m > 1;   // maxorder 1: V_0 itself, as a fixed dimension
@@ -951,7 +975,9 @@ int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t n
                          phase, ku);
       HIPCHK(hipGetLastError());
     } else {
-      if ((rc = launch_mf(p, d_fp + st * nslot, s))) return rc;
+      const int e = step_exponent(p, fprod + 2 * st * nslot);
+      const double2 fe = make_double2(scalbn(f.x, -e), scalbn(f.y, -e));
+      if ((rc = launch_mf(p, d_fp + st * nslot, e, s))) return rc;
       if ((rc = launch_tr(p, true, psi, ld, w.W, p->n, phase, ncols, s))) return rc;
       hipLaunchKernelGGL(k_pr_begin, bg, eb, 0, s, ncols, m, w.ibs, w.beta, rule ? w.kdone : nullptr,
                          rule ? w.running : nullptr);
@@ -970,7 +996,7 @@ int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t n
                  : launch_sten<double, double>(p, Wk, ncols, ib, last ? nullptr : Wk + w.vs, w.part, s);
         if (rc) return rc;
         hipLaunchKernelGGL(k_pr_alpha, cg, cb, 0, s, w.part, p->nslots, ncols, it, m, w.alpha, w.beta, w.ibs,
-                           rule ? 1 : 0, f, tol, maxorder, w.G, w.cb, w.kdone, w.coef, status, w.running);
+                           rule ? 1 : 0, fe, tol, maxorder, w.G, w.cb, w.kdone, w.coef, status, w.running);
         if (rule && it >= 1 && (it + 1 >= p->kpred || last)) {
           // the counts of wavepackets going on after each iteration so far: the
           // host waits for them from the previous step's dimension on
@@ -999,7 +1025,7 @@ int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t n
         hipLaunchKernelGGL(k_pr_beta, cg, cb, 0, s, w.epart, (int)ne, ncols, it, m, w.beta, w.ibs, w.G, w.cb);
       }
       if (!rule) {
-        hipLaunchKernelGGL(k_pr_expm, cg, cb, 0, s, w.alpha, w.beta, w.ibs, ncols, m, m, f, w.coef);
+        hipLaunchKernelGGL(k_pr_expm, cg, cb, 0, s, w.alpha, w.beta, w.ibs, ncols, m, m, fe, w.coef);
         if (adaptive && status)   // maxorder 1 is reached at once
           hipLaunchKernelGGL(k_pr_ifill, dim3(grid_for(ncols, 256)), dim3(256), 0, s, status, ncols,
                              RM_NOT_CONVERGED);

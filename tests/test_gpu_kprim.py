@@ -148,3 +148,26 @@ def test_factors_from_cartens(device):
     T[1].kmat[(4, 4)][("A", "A")][2] = T[1].kmat[(4, 4)][("A", "A")][2] * 0.5
     kop2, _ = KronOperator.from_cartens(T[0] + T[1])
     assert kop2.factors is None
+
+
+@pytest.mark.parametrize("field", [1e7, 3e9])
+def test_fp32_in_joules(device, field):
+    """A dipole in C m, fields in V/m, H in J and f = -i dt / hbar: FP32 products
+    are as good as in cm^-1 (4e-6 of the FP64 form), though field x dipole x H
+    is below the smallest FP32 number."""
+    import torch
+    from richmol_amd import units
+    kop = KronOperator(_basis(0, 6, False), [np.array([0.2, 0.3, -0.1])], [-units.AU_DIP])
+    E = field * np.array([[1, 0, 0], [0.6, 0.8, 0], [0.3, -0.4, 0.5]])
+    fp = slot_products(kop, [E])
+    X = _rows(kop.n, 3, 5)
+    X /= np.linalg.norm(X, axis=1)[:, None]
+    f = -1j * 0.1 / (field * units.AU_DIP)   # a time step of |f H| ~ 0.03
+    out = {}
+    for prec in ("fp64", "fp32"):
+        dp = DeviceKronPlan(kop)
+        psi = torch.from_numpy(X).to(device)
+        dp.propagate(psi, fp, f, krylov_fixed=8, precision=prec)
+        out[prec] = psi.cpu().numpy()
+    assert np.abs(out["fp64"] - X).max() > 1e-3
+    assert np.abs(out["fp32"] - out["fp64"]).max() <= 4e-6
