@@ -6,13 +6,19 @@
 // functions, which only couples k1 - k2 = s, |s| <= w <= 2
 // (labtens.py:482-496).  C is unitary and acts on k alone, so the whole Krylov
 // recurrence of a step can run on X' = X C^T: the wavepackets are transformed
-// once before it and once after it (k_pr_tr, matrix cores), and inside it
-// the operator is a stencil,
+// once before it (k_pr_tr, matrix cores) and what the step adds to them once
+// after it, and inside it the operator is a stencil,
 //   Y'[J1](m1, k1) = sum_{J2, w} sum_sigma MF_sigma(m1) sum_s P_s(k1) X'[J2](m1 - sigma, k1 - s),
 // at most 5 x (5 + 5) complex multiply-adds per element and tensor rank instead
 // of a row of dense products over all k (9 x 161 per element at J = 80 for a
 // dipole and a polarizability).  The same operator, the same Lanczos
 // recurrence (tdse.py:417-486): results agree to rounding, as C is unitary.
+// The state's own part of a step, c_0 phi, is taken from psi and does not go
+// through C and back: C is unitary to 1e-15 only, which left an error of 1e-15
+// after one step and of 3-4e-13 after 1 000 (the dense form's norm drifts by
+// 0.3-0.9e-13 in these).  Now only what a step adds carries it: 1.6e-16 after one
+// step at J = 80 (dense form 2.0e-16), after 1 000 steps at J <= 20 a norm
+// drift of 0.2-1.0e-13 in a field of 1e9 V/m, 1.3-2.1e-13 in one of 5e9.
 //
 // Vectors are (wavepacket, internal order) arrays of complex values, as the
 // caller's rows: J blocks of (m, k), k fastest.  The basis is kept as the
@@ -26,8 +32,8 @@
 // rocBLAS products) takes 157.5 and 112.2 ms; J <= 31, 16 wavepackets, adaptive,
 // <cos^2> read: 0.37 ms per step against 4.8.  Of the 20.5 ms the stencils take
 // 10.7 (0.89 each), the vector updates 6.1 (0.55 each: 2.9 GB at 5.3 TB/s), the
-// final combination 1.9 (9.4 GB at 5.1 TB/s), the transforms 1.6.  Error
-// against 64-bit dense products 1e-15 (FP64); FP32 2.3e-9 (dense form 3.2e-9).
+// final combination 1.9 (9.4 GB at 5.1 TB/s), the transforms 1.6.  FP32 error
+// against 64-bit dense products 2.6e-9 (dense form 3.2e-9).
 
 #include <algorithm>
 #include <cmath>
@@ -345,8 +351,9 @@ __global__ __launch_bounds__(64 * SW) void k_pr_sten(const int4* __restrict__ it
 }
 
 // out[r][c] = sum_q in[r][q] T[q][c] per J on the matrix cores, rows r =
-// (wavepacket, m); FWD: in = phase x rows of psi, T = C^T; backward: out =
-// phase x result, T = conj(C).  TR x TC output tiles, the re and im parts of a
+// (wavepacket, m); FWD: in = phase x rows of psi, T = C^T; backward: T =
+// conj(C), and with c0 (the step's first coefficient per wavepacket, ldc0
+// apart) out = phase x (c0 phase out + result), psi's own part of the step.  TR x TC output tiles, the re and im parts of a
 // row as two rows of the real product (a real C) -- a quarter of the flops
 // of the complex product in real form -- or with a complex C two products
 // more.  One wave per 16 columns; the next TK-deep slice is loaded while the
@@ -356,7 +363,8 @@ template <bool CT, bool FWD>
 __global__ __launch_bounds__(256) void k_pr_tr(const int4* __restrict__ tiles, const PJ* __restrict__ pj,
                                                const int64_t* __restrict__ toff, const double* __restrict__ T,
                                                const double2* __restrict__ in, int64_t ldi, double2* __restrict__ out,
-                                               int64_t ldo, const double2* __restrict__ ph, int32_t ncols) {
+                                               int64_t ldo, const double2* __restrict__ ph, int32_t ncols,
+                                               const double2* __restrict__ c0_, int32_t ldc0) {
   typedef double V4 __attribute__((ext_vector_type(4)));
   constexpr int NP = CT ? 2 : 1;
   __shared__ double sA[2][2][TK][TR + 1];
@@ -455,8 +463,13 @@ __global__ __launch_bounds__(256) void k_pr_tr(const int4* __restrict__ tiles, c
       if (row >= M) continue;
       const int64_t b = row / d, m = row - b * d;
       double2 o = make_double2(acc[0][r][v], acc[1][r][v]);
-      if (!FWD && ph) o = cmul(o, ph[j.voff + m * d + c]);
-      out[b * ldo + j.voff + m * d + c] = o;
+      double2* q = out + b * ldo + j.voff + m * d + c;
+      if (!FWD) {
+        const double2 p = ph ? ph[j.voff + m * d + c] : make_double2(1.0, 0.0);
+        if (c0_) o = mac(c0_[b * ldc0], ph ? cmul(*q, p) : *q, o);
+        if (ph) o = cmul(o, p);
+      }
+      *q = o;
     }
 }
 
@@ -608,7 +621,7 @@ __global__ __launch_bounds__(64) void k_pr_expm(const double2* __restrict__ alph
   for (int i = l; i < m; i += 64) coef[(int64_t)b * kcap + i] = cscale(ibs[(int64_t)i * ncols + b], s_c[i]);
 }
 
-// W_0 <- sum_j coef_j W_j (kd: the wavepacket's own dimension, or NULL: m)
+// W_0 <- sum_{j > 0} coef_j W_j (kd: the wavepacket's own dimension, or NULL: m)
 __global__ __launch_bounds__(256) void k_pr_comb(int64_t n, double2* W0, int64_t vstride,
                                                  const double2* __restrict__ coef, int32_t m, int32_t kcap,
                                                  const int32_t* __restrict__ kd, int32_t* __restrict__ kused) {
@@ -623,7 +636,7 @@ __global__ __launch_bounds__(256) void k_pr_comb(int64_t n, double2* W0, int64_t
     const int64_t i = i0 + 256 * u;
     if (i >= n) break;
     double2 s = make_double2(0.0, 0.0);
-    for (int q = 0; q < m; ++q) s = mac(cf[q], W0[q * vstride + base + i], s);
+    for (int q = 1; q < m; ++q) s = mac(cf[q], W0[q * vstride + base + i], s);
     W0[base + i] = s;
   }
 }
@@ -786,11 +799,11 @@ int launch_sten(KPrim* p, const double2* W, int32_t ncols, const double* ib, voi
 }
 
 int launch_tr(KPrim* p, bool fwd, const double2* in, int64_t ldi, double2* out, int64_t ldo, const double2* ph,
-              int32_t ncols, hipStream_t s) {
+              int32_t ncols, hipStream_t s, const double2* c0 = nullptr, int32_t ldc0 = 0) {
   const dim3 g((unsigned)p->ntiles), b(256);
 #define RM_TR(CT, FWD)                                                                                          \
   hipLaunchKernelGGL((k_pr_tr<CT, FWD>), g, b, 0, s, p->d_tiles, p->d_pj, p->d_toff, p->d_T, in, ldi, out, ldo, \
-                     ph, ncols)
+                     ph, ncols, c0, ldc0)
   if (p->cplx) {
     if (fwd) RM_TR(true, true);
     else RM_TR(true, false);
@@ -1033,7 +1046,7 @@ int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t n
       hipLaunchKernelGGL(k_pr_comb, eg, eb, 0, s, p->n, w.W, w.vs, w.coef, kdim, m,
                          rule ? (const int32_t*)w.kdone : nullptr, ku);
       HIPCHK(hipGetLastError());
-      if ((rc = launch_tr(p, false, w.W, p->n, psi, ld, phase, ncols, s))) return rc;
+      if ((rc = launch_tr(p, false, w.W, p->n, psi, ld, phase, ncols, s, w.coef, m))) return rc;
     }
     if (obs) {
       // <S|O|S> in the primitive basis: the wavepackets once more forward,
