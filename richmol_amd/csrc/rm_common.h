@@ -168,7 +168,7 @@ struct rm_plan {
   // slice holds whole subspaces, or 64 rows of one; (first row, rows, pairs of
   // entries per row, row its columns count from).  Entries in pairs, pair p
   // of lane l at soff + 64 p + l: columns 16 bits each in units of 16 bytes
-  // of a vector, values real (sreal: every B_s entry real to 1e-14) or complex
+  // of a vector, values real (sreal: every B_s entry real, operator_flags) or complex
   int4* sslice = nullptr;
   int64_t* soff = nullptr;
   int32_t* srow = nullptr;       // [n] slice of each permuted row

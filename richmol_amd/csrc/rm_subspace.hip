@@ -959,15 +959,19 @@ std::vector<double2> entry_values(const rm_plan* p) {
   return B;
 }
 
-// All values real; and symmetric to 1e-14 (rows hold their columns ascending;
-// next[c]: the first entry of row c that no row above has passed).
+// All values real, and symmetric, to the rounding of the complex products and
+// sums that formed them: imaginary parts of at most 4 and pairs of entries
+// within 8 units in the last place (rotors and tops up to J = 62 in Z and XZ
+// fields: 1.6 and 4.3).  What is larger is the caller's and is kept, a NaN too.
+// (Rows hold their columns ascending; next[c]: the first entry of row c that no
+// row above has passed.)
 void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
                     const std::vector<double2>& cval) {
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   p->sreal = true;
   for (const double2& v : cval)
-    if (std::fabs(v.y) > 1e-14 * std::fabs(v.x)) {
+    if (!(std::fabs(v.y) <= 0x1p-50 * std::fabs(v.x))) {
       p->sreal = false;
       break;
     }
@@ -981,7 +985,7 @@ void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vecto
       const int64_t e2 = q < rp[c + 1] && ccol[q] == r ? q : -1;
       for (int32_t s = 0; s < nf; ++s) {
         const double x = cval[(size_t)s * nnz + e].x, y = e2 >= 0 ? cval[(size_t)s * nnz + e2].x : 0.0;
-        if (std::fabs(x - y) > 1e-14 * std::max(std::fabs(x), std::fabs(y))) p->ssym = false;
+        if (!(std::fabs(x - y) <= 0x1p-49 * std::max(std::fabs(x), std::fabs(y)))) p->ssym = false;
       }
     }
 }

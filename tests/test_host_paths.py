@@ -1,7 +1,8 @@
 """Host paths of the library on the CPU, in a process whose HIP runtime is
 hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
 recorded and allocations can be made to fail.  What a plan's launches read after
-an allocation failed, and after its arrays were replaced.
+an allocation failed, and after its arrays were replaced; which operators count
+as real and as symmetric.
 """
 import ctypes
 import os
@@ -31,32 +32,39 @@ def _matrix():
 
 class Stub:
     def __init__(self, lib_path, stub_path):
+        """The library and the stub; plan: a plan of _matrix()."""
         from richmol_amd import _lib
         self.lib, self.stub = ctypes.CDLL(lib_path), ctypes.CDLL(stub_path)
         for name, (res, args) in _lib.SIGNATURES.items():
             if hasattr(self.lib, name):
                 getattr(self.lib, name).restype, getattr(self.lib, name).argtypes = res, args
         self.stub.stub_launch.restype = P
-        self.rows, self.cols, self.vals = _matrix()
+        self.batch = P()
+        assert self.lib.rm_batch_create(ctypes.byref(self.batch)) == 0
+        assert self.lib.rm_batch_set_block_rows(self.batch, 64) == 0
         self.n = n = LONG + SHORT
+        self.table, self.flags = np.ones((3, 2), np.complex128), np.ones(3, np.int32)
+        self.psi, self.work = np.zeros((1, n), np.complex128), np.zeros((1, n), np.complex128)
+        self.rows, self.cols, self.vals = _matrix()
+        self.plan = self.make_plan(self.vals)
+
+    def make_plan(self, vals):
+        """A plan of the pattern with these values (2, entries)."""
+        from richmol_amd import _lib
+        n = self.n
         nnz = self.rows.size
         i64, i32 = np.int64, np.int32
         ptr = np.zeros(n + 1, i64)
         np.add.at(ptr, self.rows + 1, 1)
         ptr = np.cumsum(ptr).astype(i64)
-        kval = np.zeros((nnz, 2, 2))
-        kval[:, :, 0] = self.vals.T
+        kval = np.ascontiguousarray(np.asarray(vals, dtype=np.complex128).T).view(np.float64)
         a = [ptr, self.cols, np.arange(nnz + 1, dtype=i64) * 2, np.tile(np.array([0, 1], i32), nnz), kval,
              np.array([0, 1, 2], i64), np.array([0, 1], i32), np.array([1.0, 0.0, 1.0, 0.0]), np.zeros(2, i32)]
         q = [x.ctypes.data_as(t) for x, t in zip(a, _lib.SIGNATURES["rm_plan_create"][1][2:7])]
         t = [x.ctypes.data_as(t) for x, t in zip(a[5:], _lib.SIGNATURES["rm_plan_create"][1][8:12])]
-        self.plan = P()
-        assert self.lib.rm_plan_create(n, nnz, *q, 2, *t, 2, 1, ctypes.byref(self.plan)) == 0
-        self.batch = P()
-        assert self.lib.rm_batch_create(ctypes.byref(self.batch)) == 0
-        assert self.lib.rm_batch_set_block_rows(self.batch, 64) == 0
-        self.table, self.flags = np.ones((3, 2), np.complex128), np.ones(3, i32)
-        self.psi, self.work = np.zeros((1, n), np.complex128), np.zeros((1, n), np.complex128)
+        plan = P()
+        assert self.lib.rm_plan_create(n, nnz, *q, 2, *t, 2, 1, ctypes.byref(plan)) == 0
+        return plan
 
     def job(self, lo, n):
         """A batch job on one domain; the library's status."""
@@ -150,6 +158,31 @@ def case_kept_lists(s):
     check()
 
 
+def case_real_operators(s):
+    """An operator runs as a real one, and as a symmetric one, only where the
+    rest is rounding: what the caller put there stays, a NaN too."""
+    sym = np.empty_like(s.vals)
+    for q in range(2):
+        A = np.zeros((s.n, s.n))
+        A[s.rows, s.cols] = s.vals[q]
+        sym[q] = (A + A.T)[s.rows, s.cols]
+    one = np.zeros(s.rows.size)
+    one[np.flatnonzero((s.rows == LONG + 40) & (s.cols == LONG + 41))] = 1.0
+    for vals, real, symmetric in ((sym, True, True), (s.vals, True, False), (sym * (1 + 2.0 ** -51 * 1j), True, True),
+                                  (sym * (1 + 2.0 ** -49 * 1j * one), False, False),
+                                  (sym + np.where(one > 0, complex(0, np.nan), 0), False, False),
+                                  (sym * (1 + 2.0 ** -50 * one), True, True),
+                                  (sym * (1 + 2.0 ** -47 * one), True, False)):
+        s.plan = s.make_plan(vals)
+        assert s.job(LONG, SHORT) == 0
+        kernels = [n for n in (ctypes.string_at(s.stub.stub_launch(i)).decode() for i in range(s.stub.stub_count()))
+                   if "k_blkILb" in n]   # k_blk<FIXED, F32, REAL, ...>
+        (words, _, _), = s.launches("k_blk")
+        flags = int(np.frombuffer(ctypes.string_at(words[0] + 8 * 14, 4), np.int32)[0])
+        assert len(kernels) == 1 and ("k_blkILb1ELb0ELb%d" % real) in kernels[0]
+        assert flags == (1 if real and symmetric else 0)
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
@@ -158,7 +191,7 @@ def stub(tmp_path_factory):
     return so
 
 
-@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists"])
+@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators"])
 def test_host_path(stub, case):
     from richmol_amd import _build
     if not os.path.exists(_build.LIB_PATH):
