@@ -1315,9 +1315,22 @@ constexpr int COMPLEX4_CLASS = 14;
 constexpr int PAIR_MAX_M = 16;
 constexpr int CLASS_R[NCLASS] = {1, 2, 4, 4, 8, 16, 1, 1, 1, 2, 1, 1, 1, 1, 1};
 
+// Whether k_wav holds the domain's rows (len <= 64): 32 pairs of entries per
+// lane, 16 with two wavepackets per wave.  A row without repeated columns
+// always fits; one that names columns more than once may not.
+bool wav_holds(const rm_plan* p, int lo, int len) {
+  const int64_t most = len <= 32 ? 32 : 64;
+  if (p->sub_w <= most) return true;
+  for (int r = lo; r < lo + len; ++r) {
+    const int32_t i = p->h_sub_perm[r];
+    if (p->h_row_ptr[i + 1] - p->h_row_ptr[i] > most) return false;
+  }
+  return true;
+}
+
 int sub_class(const rm_plan* p, int lo, int len) {
   const bool narrow = p->sub_w <= 4;
-  if (len <= 64 && p->h_srow[lo] == p->h_srow[lo + len - 1])
+  if (len <= 64 && p->h_srow[lo] == p->h_srow[lo + len - 1] && wav_holds(p, lo, len))
     return p->sreal ? (narrow ? 0 : 8) : (narrow ? COMPLEX4_CLASS : 12);
   if (len <= 128) return narrow ? 1 : 9;
   if (len <= 256) return narrow ? 2 : 3;

@@ -2,7 +2,7 @@
 hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
 recorded and allocations can be made to fail.  What a plan's launches read after
 an allocation failed, and after its arrays were replaced; which operators count
-as real and as symmetric.
+as real and as symmetric; where rows with repeated columns run.
 """
 import ctypes
 import os
@@ -48,17 +48,17 @@ class Stub:
         self.rows, self.cols, self.vals = _matrix()
         self.plan = self.make_plan(self.vals)
 
-    def make_plan(self, vals):
-        """A plan of the pattern with these values (2, entries)."""
+    def make_plan(self, vals, rows=None, cols=None, n=None):
+        """A plan of these values (2, entries) on _matrix()'s pattern or another."""
         from richmol_amd import _lib
-        n = self.n
-        nnz = self.rows.size
+        rows, cols, n = (self.rows, self.cols, self.n) if rows is None else (rows, cols, n)
+        nnz = rows.size
         i64, i32 = np.int64, np.int32
         ptr = np.zeros(n + 1, i64)
-        np.add.at(ptr, self.rows + 1, 1)
+        np.add.at(ptr, rows + 1, 1)
         ptr = np.cumsum(ptr).astype(i64)
         kval = np.ascontiguousarray(np.asarray(vals, dtype=np.complex128).T).view(np.float64)
-        a = [ptr, self.cols, np.arange(nnz + 1, dtype=i64) * 2, np.tile(np.array([0, 1], i32), nnz), kval,
+        a = [ptr, cols, np.arange(nnz + 1, dtype=i64) * 2, np.tile(np.array([0, 1], i32), nnz), kval,
              np.array([0, 1, 2], i64), np.array([0, 1], i32), np.array([1.0, 0.0, 1.0, 0.0]), np.zeros(2, i32)]
         q = [x.ctypes.data_as(t) for x, t in zip(a, _lib.SIGNATURES["rm_plan_create"][1][2:7])]
         t = [x.ctypes.data_as(t) for x, t in zip(a[5:], _lib.SIGNATURES["rm_plan_create"][1][8:12])]
@@ -183,6 +183,20 @@ def case_real_operators(s):
         assert flags == (1 if real and symmetric else 0)
 
 
+def case_repeated_columns(s):
+    """20-row domains, in one of which every column of a row is named twice (40
+    entries): that one runs on the kernel that reads any number of entries,
+    its neighbour on the one that holds 32 per row."""
+    r, c = (x.ravel() for x in np.meshgrid(np.arange(20), np.arange(20), indexing="ij"))
+    rows, cols = np.concatenate([r, r, 20 + r]), np.concatenate([c, c, 20 + c]).astype(np.int32)
+    order = np.lexsort((cols, rows))
+    s.plan = s.make_plan(np.ones((2, rows.size)), rows[order], cols[order], 40)
+    s.n, s.psi = 40, np.zeros((1, 40), np.complex128)
+    for lo, kernel in ((0, "k_sub_prop"), (20, "k_wav")):
+        assert s.job(lo, 20) == 0
+        assert [k for k in ("k_sub_prop", "k_wav", "k_sub_pair") if s.launches(k)] == [kernel]
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
@@ -191,7 +205,7 @@ def stub(tmp_path_factory):
     return so
 
 
-@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators"])
+@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators", "repeated_columns"])
 def test_host_path(stub, case):
     from richmol_amd import _build
     if not os.path.exists(_build.LIB_PATH):
