@@ -88,6 +88,17 @@ def _kdiag(P, J1, J2):
     return out
 
 
+def _rounding(d):
+    """What products over d elements of size one leave by rounding (tops of
+    J <= 31 reach a third of it, in C^H C and in C1 K C2^H)."""
+    return 4 * np.finfo(np.float64).eps * math.sqrt(d)
+
+
+def _unitary(C):
+    """Whether every coefficient matrix is unitary to rounding."""
+    return all(np.abs(c.conj().T @ c - np.eye(c.shape[1])).max() <= _rounding(c.shape[0]) for c in C.values())
+
+
 def _mdiag(ucols_w, w, J1, J2, ncart):
     """Diagonals of M_w,cart (rot._m_block with all m): for every sigma,
     the (ncart, 2J1+1) values at m2 = m1 - sigma (0 where m2 is out of
@@ -121,7 +132,7 @@ class KronOperator:
     factors: (C, P) with K = C[J1]^H P C[J2]: per J the coefficient matrix C
     (primitive k, state) and per block the diagonals of P (_kdiag), which the
     device plan's primitive-basis form works on; None when the K blocks'
-    primitive basis is not known.
+    primitive basis is not known or C is not unitary.
     """
     factors = None
 
@@ -161,7 +172,8 @@ class KronOperator:
                             continue
                         self.blocks.append((li, J1, J2, w, K * scale, md))
                         Pd.append(_kdiag(P, J1, J2) * scale)
-        self.factors = (C, Pd)
+        if _unitary(C):
+            self.factors = (C, Pd)
         # internal layout and the permutation from the reference's full-form order
         off, pos = {}, 0
         for J in self.Jlist:
@@ -270,20 +282,21 @@ class KronOperator:
 
     def _find_factors(self, coef):
         """The primitive-basis factors of blocks read from a CarTens, when its
-        builder left the coefficients: P = C1 K C2^H must be banded and give K
-        back to rounding (a tensor changed since does not, and keeps the
-        dense form)."""
+        builder left the coefficients: they must be unitary and P = C1 K C2^H
+        banded, both to rounding (a tensor changed since is not, and keeps
+        the dense form)."""
         if coef is None or any(J not in coef or coef[J].shape != (2 * J + 1, 2 * J + 1) for J in self.Jlist):
             return
-        for J in self.Jlist:
-            if np.abs(coef[J].conj().T @ coef[J] - np.eye(2 * J + 1)).max() > 1e-12:
-                return
+        if not _unitary({J: coef[J] for J in self.Jlist}):
+            return
         Pd = []
         for _, J1, J2, _, K, _ in self.blocks:
+            if abs(J1 - J2) > 2:
+                return
             P = coef[J1] @ K @ coef[J2].conj().T
             d = _kdiag(P, J1, J2)
-            tol = 1e-13 * np.abs(K).max()
-            d[np.abs(d) < 1e-2 * tol] = 0
+            tol = _rounding(2 * max(J1, J2) + 1) * np.abs(K).max()
+            d[np.abs(d) < 1e-15 * np.abs(K).max()] = 0
             k1 = np.arange(-J1, J1 + 1)
             for s in range(-2, 3):
                 ok = np.abs(k1 - s) <= J2

@@ -4,6 +4,7 @@ against the oracle's block operator (CarTens.vec, field.py:1145-1245) on an
 asymmetric top with a dipole and a full polarizability under a general field."""
 import numpy as np
 import pytest
+from scipy.sparse import csr_matrix
 
 from _fixtures import large_top, large_top_tensors
 from richmol_amd import kron, rot
@@ -124,3 +125,31 @@ def test_from_cartens_refuses_thresholds_and_partial_m():
     t0.field([0, 0, 1.0])
     with pytest.raises(ValueError):
         kron.KronOperator.from_cartens(t0)
+
+
+def test_factors_only_to_rounding():
+    """The primitive-basis factors are taken where they give K back to rounding
+    and the coefficients are unitary to rounding, not a little beyond."""
+    bas = rot.asymtop_basis(9.0, 6.0, 4.0, 6)
+
+    def leaf():
+        T = rot.tensor(np.array([0.2, 0.3, -0.1]), bas)
+        T.field([1e8, 2e8, -3e8])
+        return T
+
+    assert kron.KronOperator.from_cartens(leaf())[0].factors is not None
+    T = leaf()
+    (sym, K), = [(s, d[1]) for s, d in T.kmat[(6, 5)].items() if 1 in d][:1]
+    top = max(abs(d[1]).max() for d in T.kmat[(6, 5)].values() if 1 in d)
+    K = K.toarray()
+    K[0, -1] += 5e-14 * top
+    T.kmat[(6, 5)][sym][1] = csr_matrix(K)
+    assert kron.KronOperator.from_cartens(T)[0].factors is None
+    T = leaf()
+    T._kcoef[4] = T._kcoef[4] * (1 + 2e-13)
+    assert kron.KronOperator.from_cartens(T)[0].factors is None
+
+    assert kron.KronOperator(bas, [np.array([0.2, 0.3, -0.1])]).factors is not None
+    for s, (kp, c) in bas.kfun[4].items():
+        bas.kfun[4][s] = (kp, c * (1 + 2e-13))
+    assert kron.KronOperator(bas, [np.array([0.2, 0.3, -0.1])]).factors is None
