@@ -248,7 +248,11 @@ int rm_plan_set_kernel(rm_plan* plan, int32_t variant);
  *                    RM_SUBSPACE_MAX_ROWS) take the long-domain forms;
  *  RM_TUNE_COOP_MIN_ENTRIES  the cooperative form only while every long
  *                    domain holds at least (their count) x this many stored
- *                    entries (default 100000: it runs them one at a time).
+ *                    entries (default 100000: it runs them one at a time);
+ *  RM_TUNE_OPERATOR_KIB  KiB that the block kernel's operators, formed ahead
+ *                    for as many steps as fit and shared by a call's
+ *                    wavepackets, may take (default 262144; 0, or no room on
+ *                    the device: every workgroup forms its own).
  * Results do not depend on these choices beyond summation order.  A change
  * drops the launch lists kept for domain reuse. */
 #define RM_TUNE_PAIR       0
@@ -257,6 +261,7 @@ int rm_plan_set_kernel(rm_plan* plan, int32_t variant);
 #define RM_TUNE_FORK       3
 #define RM_TUNE_WAVE_MAX_ROWS    4
 #define RM_TUNE_COOP_MIN_ENTRIES 5
+#define RM_TUNE_OPERATOR_KIB     6
 int rm_plan_set_tuning(rm_plan* plan, int32_t knob, int32_t value);
 
 /* Launch configuration i of the ELL kernel: threads per workgroup, rows per

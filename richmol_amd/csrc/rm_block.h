@@ -17,7 +17,8 @@ int blk_variant(int64_t nslices, bool real);
 // Pairs of entries per lane of a domain of nslices slices, the longest of
 // maxpairs: its launch keeps them in registers up to BLK_PAIRS.
 int blk_part_pairs(int64_t nslices, int64_t maxpairs);
-// Launches items [first, first + count) of one variant (by falling ppairs) on s; ws: workspace grown in place.
+// Launches items [first, first + count) of one variant (by falling ppairs) on s; ws: workspace grown in place;
+// pre_bytes: what operators formed ahead for all wavepackets of a job may take.
 int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, const int4* d_items,
             const std::vector<LongItem>& items, size_t first, size_t count, int variant, int32_t kcap, int32_t fixed_m,
-            int32_t maxorder, double tol, bool f32, int n_cu, hipStream_t s);
+            int32_t maxorder, double tol, bool f32, int n_cu, size_t pre_bytes, hipStream_t s);

@@ -583,8 +583,6 @@ __global__ __launch_bounds__(NT) void k_blk(BlkArgs a) {
   }
 }
 
-constexpr size_t PRE_BYTES = (size_t)256 << 20;
-
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 template <int RS, bool REG>
@@ -613,7 +611,7 @@ int blk_part_pairs(int64_t nslices, int64_t maxpairs) {
 
 int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, const int4* d_items,
             const std::vector<LongItem>& items, size_t first, size_t count, int variant, int32_t kcap, int32_t fixed_m,
-            int32_t maxorder, double tol, bool f32, int n_cu, hipStream_t s) {
+            int32_t maxorder, double tol, bool f32, int n_cu, size_t pre_bytes, hipStream_t s) {
   const int rs = (variant + 1) / 2;   // 1, 2 or 3 (5 slices per wave)
   const bool real = (variant & 1) == 0, fixed = fixed_m > 0;
   // the items come by falling pairs per lane: those that fit the registers last
@@ -621,7 +619,7 @@ int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, c
   while (mem < count && items[first + mem].ppairs > BLK_PAIRS(f32, real)) ++mem;
   if (mem > 0 && mem < count) {
     const int rc = blk_run(ws, ws_bytes, d_ops, op0, d_items, items, first, mem, variant, kcap, fixed_m, maxorder, tol,
-                           f32, n_cu, s);
+                           f32, n_cu, pre_bytes, s);
     if (rc) return rc;
     first += mem;
     count -= mem;
@@ -637,30 +635,36 @@ int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, c
     lmax = std::max<int64_t>(lmax, items[i].item.z);
     if (items[i].nslot > 1) pmax = std::max<int64_t>(pmax, items[i].npairs);
   }
-  // one job by value: its steps' operators are formed once for all its
-  // wavepackets, for as many steps as PRE_BYTES hold, and the launch is cut
-  // there (the state is in psi between launches)
   int64_t q0 = INT64_MAX, q1 = 0;
   for (size_t i = first; i < first + count; ++i) {
     q0 = std::min(q0, items[i].pair0);
     q1 = std::max(q1, items[i].pair0 + items[i].npairs);
   }
+  // one job by value: its steps' operators are formed once for all its
+  // wavepackets, for as many steps as pre_bytes hold, and the launch is cut
+  // there (the state is in psi between launches).  Where one step's do not fit,
+  // or the device has no room for them, every workgroup forms its own
   const size_t b_step = (size_t)(f32 ? 8 : 16) * (real ? 1 : 2) * (size_t)std::max<int64_t>(q1 - q0, 1);
-  const bool pre = !reg && op0 && op0->nslot > 1 && op0->nsteps > 0;
-  const int chunk = !pre ? INT32_MAX : (int)std::max<int64_t>(1, std::min<int64_t>(op0->nsteps, PRE_BYTES / b_step));
-  const size_t b_pre = pre ? al256(b_step * (size_t)chunk) : 0;
+  bool pre = !reg && op0 && op0->nslot > 1 && op0->nsteps > 0 && b_step <= pre_bytes;
+  const int chunk = pre ? (int)std::min<int64_t>(op0->nsteps, pre_bytes / b_step) : INT32_MAX;
   const size_t lds = lds_bytes(lmax);
   int occ = 0;
   HIPCHK(occupancy(kern, NT, lds, &occ));
   if (occ < 1) return fail(RM_ERR_ARG, "block propagation: a domain of %lld rows does not fit LDS", (long long)lmax);
   const int grid = (int)std::min<int64_t>((int64_t)count, (int64_t)occ * n_cu);
   const size_t b_v = al256(sizeof(double2) * (size_t)kcap * lmax);
-  const size_t b_a = pre ? 0 : al256((f32 ? 8 : 16) * (real ? 1 : 2) * (size_t)std::max<int64_t>(pmax, 1));
+  const size_t b_own = al256((f32 ? 8 : 16) * (real ? 1 : 2) * (size_t)std::max<int64_t>(pmax, 1));
   const size_t b_g = fixed ? 0 : al256(sizeof(double2) * ((size_t)kcap * kcap + 2 * (size_t)kcap));
-  a.offA = (int64_t)b_v;
-  a.offG = (int64_t)(b_v + b_a);
-  a.wg_bytes = (int64_t)(b_v + b_a + b_g);
-  const size_t need = b_pre + (size_t)a.wg_bytes * (size_t)grid;
+  size_t b_pre = 0;
+  auto layout = [&]() {
+    const size_t b_a = pre ? 0 : b_own;
+    b_pre = pre ? al256(b_step * (size_t)chunk) : 0;
+    a.offA = (int64_t)b_v;
+    a.offG = (int64_t)(b_v + b_a);
+    a.wg_bytes = (int64_t)(b_v + b_a + b_g);
+    return b_pre + (size_t)a.wg_bytes * (size_t)grid;
+  };
+  size_t need = layout();
   if (*ws_bytes < need) {
     if (*ws) {
       HIPCHK(hipDeviceSynchronize());
@@ -668,7 +672,15 @@ int blk_run(void** ws, size_t* ws_bytes, const SubOp* d_ops, const SubOp* op0, c
       *ws = nullptr;
       *ws_bytes = 0;
     }
-    HIPCHK(hipMalloc(ws, need));
+    hipError_t e = hipMalloc(ws, need);
+    if (e == hipErrorOutOfMemory && pre) {
+      (void)hipGetLastError();
+      pre = false;
+      need = layout();
+      e = hipMalloc(ws, need);
+    }
+    if (e != hipSuccess) *ws = nullptr;
+    HIPCHK(e);
     *ws_bytes = need;
   }
   a.ops = op0 ? nullptr : d_ops;

@@ -100,6 +100,7 @@ struct RmTuning {
   int32_t fork = 1;        // launch classes of a call side by side on auxiliary streams
   int32_t wave_max_rows = 64;       // domains longer than this leave the one-wave kernels
   int32_t coop_min_entries = 100000;  // stored entries per cooperative wavepacket at least
+  int32_t operator_kib = 262144;      // KiB of a block launch's operators formed ahead
 };
 
 struct rm_plan {

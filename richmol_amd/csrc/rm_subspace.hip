@@ -1646,7 +1646,7 @@ int launch_all(SubScratch* sc, const SubArgs& a0, const int4* const (&items)[NCL
     size_t e = nb;
     while (e < blk.size() && blk[e].variant == blk[nb].variant) ++e;
     rc = blk_run(&sc->blk_ws, &sc->blk_ws_bytes, a0.ops, a0.ops ? nullptr : &a0.op0, d_blk, blk, nb, e - nb,
-                 blk[nb].variant, kcap, fixed_m, maxorder, tol, f32, n_cu, bs);
+                 blk[nb].variant, kcap, fixed_m, maxorder, tol, f32, n_cu, (size_t)tn.operator_kib << 10, bs);
     if (rc) return rc;
     nb = e;
   }
@@ -1843,6 +1843,10 @@ extern "C" int rm_plan_set_tuning(rm_plan* p, int32_t knob, int32_t value) {
     case RM_TUNE_COOP_MIN_ENTRIES:
       if (value < 0) return fail(RM_ERR_ARG, "rm_plan_set_tuning: negative entry count %d", value);
       p->tune.coop_min_entries = value;
+      break;
+    case RM_TUNE_OPERATOR_KIB:
+      if (value < 0) return fail(RM_ERR_ARG, "rm_plan_set_tuning: negative size %d", value);
+      p->tune.operator_kib = value;
       break;
     default:
       return fail(RM_ERR_ARG, "rm_plan_set_tuning: unknown knob %d", knob);

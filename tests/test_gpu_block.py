@@ -83,3 +83,32 @@ def test_fp32(device, jmax):
         e.propagate(fields)
         out.append(e.psi.cpu().numpy())
     assert 0 < np.abs(out[0] - out[1]).max() <= 2e-6
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("fixed", [0, 9])
+@pytest.mark.parametrize("kib", [0, 256, 512])
+def test_launches_cut_between_steps(device, kib, fixed, prec):
+    """Domains of 990 to 2 025 rows whose operators are formed ahead for one or
+    two steps a launch, or by every workgroup (0): amplitudes, observable and
+    Krylov dimensions bit for bit those of the uncut run.  A zero-field step and
+    repeated products come right after a cut."""
+    import torch
+    h0, H, cos2, bas = linear_rotor(44)
+    X = _columns(2025, 44)
+    fields = [[a * c for c in XZ] for a in (6e8, 9e8, 0.0, 1.1e9, 1.1e9, 1.1e9, 7e8)]
+    H.field(fields[0])
+    O = ensemble.Ensemble.observable_plan(cos2)
+    out = []
+    for k in (kib, 1 << 18):
+        e = ensemble.Ensemble(H, h0, -0.0019j, X, krylov_fixed=fixed)
+        e.set_kernel("block")
+        e.set_precision(prec)
+        e.set_tuning(operator_kib=k)
+        ku = torch.full((7, 3), -1, dtype=torch.int32, device=device)
+        ex, _ = e.propagate(None, table=e.prepare(fields), obs=O, kused=ku)
+        out.append((e.psi.cpu().numpy(), ex.cpu().numpy(), ku.cpu().numpy()))
+        e.set_tuning()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert np.all((out[0][2] == 0) == (np.arange(7) == 2)[:, None])

@@ -2,7 +2,8 @@
 hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
 recorded and allocations can be made to fail.  What a plan's launches read after
 an allocation failed, and after its arrays were replaced; which operators count
-as real and as symmetric; where rows with repeated columns run.
+as real and as symmetric; where rows with repeated columns run; a device with no
+room for operators formed ahead.
 """
 import ctypes
 import os
@@ -197,6 +198,23 @@ def case_repeated_columns(s):
         assert [k for k in ("k_sub_prop", "k_wav", "k_sub_pair") if s.launches(k)] == [kernel]
 
 
+def case_no_room_for_operators(s):
+    """A device with no room for the operators of all steps: the call runs
+    with every workgroup forming its own, as it does when asked to."""
+    s.psi[0, LONG + 5] = 1.0
+    assert s.lib.rm_plan_set_kernel(s.plan, 6) == 0
+    assert s.lib.rm_plan_set_domain_reuse(s.plan, 1) == 0
+    # three steps' operators: 937 kB; one workgroup's region with its own: 341 kB
+    for kib, limit, ahead in ((0, 0, 0), (1 << 18, 600000, 0), (1 << 18, 0, 1), (0, 0, 0)):
+        assert s.lib.rm_plan_set_tuning(s.plan, 6, kib) == 0
+        s.stub.stub_limit(ctypes.c_size_t(limit))
+        assert s.propagate() == 0, s.lib.rm_last_error()
+        assert len(s.launches("k_blk_operators")) == ahead and len(s.launches("k_blkILb")) == 1
+    assert s.lib.rm_plan_set_tuning(s.plan, 6, 350) == 0   # one step a launch
+    assert s.propagate() == 0
+    assert len(s.launches("k_blk_operators")) == 3 and len(s.launches("k_blkILb")) == 3
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
@@ -205,7 +223,8 @@ def stub(tmp_path_factory):
     return so
 
 
-@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators", "repeated_columns"])
+@pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators", "repeated_columns",
+                                  "no_room_for_operators"])
 def test_host_path(stub, case):
     from richmol_amd import _build
     if not os.path.exists(_build.LIB_PATH):
