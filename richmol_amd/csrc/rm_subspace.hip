@@ -2437,7 +2437,8 @@ extern "C" int rm_batch_propagate(rm_batch* bt, const rm_job* jobs, int32_t njob
 // library holds it while the process runs); host code reaches it only
 // through the address hipGetSymbolAddress returns for the current device.
 
-static constexpr size_t STATIC_STAGE_BYTES = (size_t)RM_STATIC_MAX_JOBS * (sizeof(SubOp) + sizeof(int4)) + 512;
+// a job's descriptor and two items (a pair's other half stays empty: every job has an operator of its own)
+static constexpr size_t STATIC_STAGE_BYTES = (size_t)RM_STATIC_MAX_JOBS * (sizeof(SubOp) + 2 * sizeof(int4)) + 512;
 static_assert(STATIC_STAGE_BYTES < (size_t)RM_STATIC_SCRATCH_BYTES / 4, "descriptor staging exceeds its share");
 static __device__ __align__(256) char scratch[RM_STATIC_SCRATCH_BYTES];
 

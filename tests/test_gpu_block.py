@@ -42,11 +42,11 @@ def test_against_oracle(device, jmax, axis, fixed):
         assert np.array_equal(k_d, k_o)
 
 
-@pytest.mark.parametrize("jmax,axis", [(11, XZ), (44, XZ), (50, XYZ), (62, XZ)])
+@pytest.mark.parametrize("jmax,axis", [(11, XZ), (44, XZ), (50, XYZ), (62, XZ), (63, XZ)])
 @pytest.mark.parametrize("factor", [1.0, 0.8 + 0.1j])
 @pytest.mark.parametrize("fixed", [0, 9])
 def test_against_full_vector_kernel(device, jmax, axis, factor, fixed):
-    """Up to 3 969 rows in a domain (several slices per wave); the field
+    """Up to 4 096 rows in a domain (several slices per wave); the field
     table also with complex products (real operator entries, slot by slot)."""
     import torch
     h0, H, cos2, bas = linear_rotor(jmax)

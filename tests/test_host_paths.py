@@ -3,10 +3,11 @@ hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
 recorded and allocations can be made to fail.  What a plan's launches read after
 an allocation failed, and after its arrays were replaced; which operators count
 as real and as symmetric; where rows with repeated columns run; a device with no
-room for operators formed ahead.
+room for operators formed ahead; as many static jobs as the header allows.
 """
 import ctypes
 import os
+import re
 import subprocess
 import sys
 
@@ -67,12 +68,15 @@ class Stub:
         assert self.lib.rm_plan_create(n, nnz, *q, 2, *t, 2, 1, ctypes.byref(plan)) == 0
         return plan
 
+    def job_record(self, lo, n):
+        from richmol_amd import _lib
+        return _lib.RmJob(plan=self.plan, psi=self.psi.ctypes.data, ld=self.n, col=0, lo=lo, len=n,
+                          fprod_dev=self.table.ctypes.data, sflag_dev=self.flags.ctypes.data, nsteps=3, f_re=0.0,
+                          f_im=-0.1, phase=None, kused=None, status=None)
+
     def job(self, lo, n):
         """A batch job on one domain; the library's status."""
-        from richmol_amd import _lib
-        j = _lib.RmJob(plan=self.plan, psi=self.psi.ctypes.data, ld=self.n, col=0, lo=lo, len=n,
-                       fprod_dev=self.table.ctypes.data, sflag_dev=self.flags.ctypes.data, nsteps=3, f_re=0.0,
-                       f_im=-0.1, phase=None, kused=None, status=None)
+        j = self.job_record(lo, n)
         self.stub.stub_clear()
         return self.lib.rm_batch_propagate(self.batch, ctypes.byref(j), 1, ctypes.sizeof(j), 6, 100, 1e-15, 0, None)
 
@@ -215,6 +219,24 @@ def case_no_room_for_operators(s):
     assert len(s.launches("k_blk_operators")) == 3 and len(s.launches("k_blkILb")) == 3
 
 
+def case_static_jobs(s):
+    """RM_STATIC_MAX_JOBS jobs on short domains, under the adaptive rule and
+    with a fixed dimension: every launch form takes them."""
+    src = open(os.path.join(os.path.dirname(HERE), "include", "richmol_amd.h")).read()
+    count = int(re.search(r"#define RM_STATIC_MAX_JOBS (\d+)", src).group(1))
+    r, c = (x.ravel() for x in np.meshgrid(np.arange(20), np.arange(20), indexing="ij"))
+    for width in (1, 19):   # banded and full rows
+        on = np.abs(r - c) <= width
+        s.plan = s.make_plan(np.ones((2, int(on.sum()))), r[on], c[on].astype(np.int32), 20)
+        s.n, s.psi = 20, np.zeros((1, 20), np.complex128)
+        assert s.lib.rm_plan_subspaces(s.plan, None, None) >= 0
+        jobs = (type(s.job_record(0, 20)) * count)(*[s.job_record(0, 20)] * count)
+        for fixed in (0, 9, 20):
+            rc = s.lib.rm_batch_propagate_static(ctypes.byref(jobs), count, ctypes.sizeof(jobs[0]), fixed, 100, 1e-15,
+                                                 0, None)
+            assert rc == 0, s.lib.rm_last_error()
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
@@ -224,7 +246,7 @@ def stub(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators", "repeated_columns",
-                                  "no_room_for_operators"])
+                                  "no_room_for_operators", "static_jobs"])
 def test_host_path(stub, case):
     from richmol_amd import _build
     if not os.path.exists(_build.LIB_PATH):
