@@ -207,16 +207,17 @@ int rm_plan_kernel_time(rm_plan* plan, double* total_ms, int64_t* launches);
  * equal the full-vector kernels' to rounding (entries outside the domain stay
  * exactly zero).  Domains of more than 64 rows (RM_TUNE_WAVE_MAX_ROWS; at most
  * RM_SUBSPACE_MAX_ROWS) are advanced by teams of workgroups side by side (a
- * few wavepackets with real operators in FP64, 961 to 3840 rows each), by a
- * cooperative launch (many workgroups on one wavepacket, grid barriers between the Lanczos
- * reductions) when there are at most 8 of them and each holds at least
- * their count x 100000 stored entries (RM_TUNE_COOP_MAX,
- * RM_TUNE_COOP_MIN_ENTRIES), otherwise by the block kernel (one workgroup
- * per wavepacket, all in one launch).
+ * few wavepackets with real operators in FP64, 961 to 3840 rows each:
+ * rm_team_size), by a cooperative launch (many workgroups on one wavepacket,
+ * grid barriers between the Lanczos reductions) when there are at most 8 of
+ * them and each holds at least their count x 100000 stored entries
+ * (RM_TUNE_COOP_MAX, RM_TUNE_COOP_MIN_ENTRIES), otherwise by the block kernel
+ * (one workgroup per wavepacket, all in one launch).
  *
  * RM_KERNEL_COOP, RM_KERNEL_BLOCK (rm_propagate only): every wavepacket
- * through the cooperative, or the block, kernel whatever its domain (no MF
- * thresholds). */
+ * through several workgroups (teams where they hold all domains, else the
+ * cooperative kernel, which RM_TUNE_COOP_MAX 0 selects for all), or through
+ * the block kernel, whatever its domain (no MF thresholds). */
 #define RM_KERNEL_AUTO      0
 #define RM_KERNEL_GLOBAL    1
 #define RM_KERNEL_RESIDENT  2
@@ -239,7 +240,8 @@ int rm_plan_set_kernel(rm_plan* plan, int32_t variant);
  *                    0: one wave each;
  *  RM_TUNE_COOP_MAX  long-domain wavepackets per call up to which the
  *                    cooperative form runs (default 8; more go one workgroup
- *                    each);
+ *                    each); teams are limited by the device's room alone, 0
+ *                    switches them off too;
  *  RM_TUNE_COOP_GRID workgroups of a cooperative launch at most (default 0:
  *                    one per 64-row group of the domain, up to one per CU);
  *  RM_TUNE_FORK      1 (default): the launch classes of a call side by side
@@ -431,7 +433,9 @@ int rm_kplan_destroy(rm_kplan* plan);
 int rm_kplan_info(const rm_kplan* plan, int64_t* n, double* gemm_flops_per_col);
 /* Matvec form (no reference counterpart).  RM_KKERNEL_PRIM (default of a plan
  * with K factors, rm_kplan_set_factors): the operator as a stencil in the
- * primitive symmetric-top basis.  RM_KKERNEL_GEMM (default without): the
+ * primitive symmetric-top basis.  (rm_kplan_propagate_expect runs in it when the
+ * observable's plan is in this form with the same C too, else in the dense
+ * form.)  RM_KKERNEL_GEMM (default without): the
  * m-mixed input (MF_w X) stored, then one rocBLAS product per output J, the
  * build of the next J chunk overlapping the products of the last.
  * RM_KKERNEL_FUSED: one launch per matvec on the matrix cores, the m-mixed

@@ -727,25 +727,21 @@ __global__ __launch_bounds__(64) void k_sub_pair(SubArgs a) {
           vp = vk;
           vk = cscale(ib, Wr);
         } else {
-          // exact breakdown: Gram-Schmidt of ones against the basis (tdse.py:459-465);
-          // once the basis spans the domain (nothing left, the vector is zero)
-          // every later one is zero too
+          // exact breakdown: Gram-Schmidt of ones against the basis (tdse.py:459-465)
           vp = vk;
-          {
-            Wr = ok ? make_double2(1.0, 0.0) : zero;
-            for (int j = 0; j < it; ++j) {
-              double d0 = 0.0, d1 = 0.0;
-              if (ok) {
-                const double2 x = s_V[j * 64 + l];
-                d0 = x.x * Wr.x + x.y * Wr.y;
-                d1 = x.x * Wr.y - x.y * Wr.x;
-              }
-              const double2 proj = make_double2(half_allsum32(d0), half_allsum32(d1));
-              if (ok) Wr = csub(Wr, cmul(proj, s_V[j * 64 + l]));
+          Wr = ok ? make_double2(1.0, 0.0) : zero;
+          for (int j = 0; j < it; ++j) {
+            double d0 = 0.0, d1 = 0.0;
+            if (ok) {
+              const double2 x = s_V[j * 64 + l];
+              d0 = x.x * Wr.x + x.y * Wr.y;
+              d1 = x.x * Wr.y - x.y * Wr.x;
             }
-            const double nv = sqrt(half_allsum32(Wr.x * Wr.x + Wr.y * Wr.y));
-            vk = nv > 0.0 ? make_double2(Wr.x / nv, Wr.y / nv) : zero;
+            const double2 proj = make_double2(half_allsum32(d0), half_allsum32(d1));
+            if (ok) Wr = csub(Wr, cmul(proj, s_V[j * 64 + l]));
           }
+          const double nv = sqrt(half_allsum32(Wr.x * Wr.x + Wr.y * Wr.y));
+          vk = nv > 0.0 ? make_double2(Wr.x / nv, Wr.y / nv) : zero;
         }
         s_V[it * 64 + l] = vk;
         sb[it] = beta;
@@ -1922,12 +1918,14 @@ void sort_long(std::vector<LongItem>& v) {
 // The subspace path of rm_propagate.  Arguments are validated by the caller
 // (ld, ncols, Krylov parameters, pointers).  Domains of up to
 // p->tune.wave_max_rows rows (64 unless tuned, at most RM_SUBSPACE_MAX_ROWS)
-// go to the one-wave kernels; longer ones to the cooperative kernel when
-// there are at most p->tune.coop_max of them and each holds at least
-// their count times p->tune.coop_min_entries stored entries, else to the
-// block kernel.  force: RM_KERNEL_COOP / RM_KERNEL_BLOCK send every
-// wavepacket to that kernel (0: the rule above).  *done = false when the
-// path does not apply; nothing has then been written to psi.
+// go to the one-wave kernels; longer ones to teams of workgroups where
+// team_size takes them all (FP64, and p->tune.coop_max not 0), else to the
+// cooperative kernel when there are at most p->tune.coop_max of them and each
+// holds at least their count times p->tune.coop_min_entries stored entries,
+// else to the block kernel.  force: RM_KERNEL_COOP sends every wavepacket to
+// teams or the cooperative kernel, RM_KERNEL_BLOCK to the block kernel (0: the
+// rule above).  *done = false when the path does not apply; nothing has then
+// been written to psi.
 // The observable plan's matrix in p's permuted ELL form (p->obs_col,
 // p->obs_val, width p->obs_w), rebuilt when the plan or its matrix changed.
 __global__ void k_obs_ell(int64_t n, int32_t ow, const int32_t* __restrict__ perm,

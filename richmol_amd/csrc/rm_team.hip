@@ -551,9 +551,11 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 
-// A step of the team kernel takes 36 us + 0.24 us per workgroup of the launch,
-// one of the block kernel 25 us + 0.4-0.6 ns per stored entry.  Measured (water-
-// like top, adaptive rule with 4 vectors, us per step, block / team):
+// The teams are as large as the device and the domains allow: fewer members
+// would hold more entries each but poll less, which was not measured apart.  The
+// bound on the launch's workgroups (800 entries of the smallest domain for each)
+// lies where the block kernel's step gets shorter.  Measured (water-like top,
+// adaptive rule with 4 vectors, us per step, block / team):
 //   90 372 entries, 1 wavepacket 56 / 40, 4: 56 / 47, 8: 57 / 64
 //  153 186 entries, 1 wavepacket 74 / 43, 4: 75 / 57, 8: 76 / 85
 //  370 802 entries, 1 wavepacket 194 / 51, 4: 236 / 87

@@ -112,3 +112,33 @@ def test_launches_cut_between_steps(device, kib, fixed, prec):
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     assert np.all((out[0][2] == 0) == (np.arange(7) == 2)[:, None])
+
+
+@pytest.mark.parametrize("jmax", [8, 14])
+def test_fp32_of_one_slot_over_many_steps(device, jmax):
+    """One field slot: B_0's entries rounded to FP32 are the same at every step,
+    so their error adds up -- to at most steps |f F| 2^-24 times the operator's
+    largest row sum (registers and memory forms, 200 steps)."""
+    from _fixtures import water
+    h0, leaves, bas = water(jmax)
+    H = leaves[0]
+    n = sum((2 * J + 1) ** 2 for J in range(jmax + 1))
+    X = np.zeros((2, n), dtype=np.complex128)
+    X[0, 0] = 1.0
+    X[1, [0, 1, 5]] = 3.0 ** -0.5
+    amp = 3e8 * (1.0 + 0.5 * np.cos(0.1 * np.arange(200)))
+    fields = [[a, 0.0, 0.0] for a in amp]
+    f = -0.00094j
+    out = []
+    for prec in ("fp64", "fp32"):
+        H.field(fields[0])
+        e = ensemble.Ensemble(H, h0, f, X, krylov_fixed=8)
+        e.set_kernel("block")
+        e.set_precision(prec)
+        e.propagate(fields)
+        out.append(e.psi.cpu().numpy())
+    row = float(abs(H.tomat(form="full", cart="x")).sum(axis=1).max())
+    bound = abs(f) * amp.sum() * row * 2.0 ** -24
+    err = np.linalg.norm(out[0] - out[1], axis=1).max()
+    print(f"J<={jmax}: FP32 error {err:.2e} after 200 steps, bound {bound:.2e}", flush=True)
+    assert 0 < err <= bound

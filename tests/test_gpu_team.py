@@ -95,3 +95,23 @@ def test_unequal_domains(device, order, fixed, kernel):
         out.append((e.psi.cpu().numpy(), ku.cpu().numpy()))
     assert np.abs(out[0][0] - out[1][0]).max() <= 1e-11
     assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("fixed", [0, 9])
+def test_cooperative_form_at_these_sizes(device, fixed):
+    """The grid form of the cooperative kernel on domains teams would take
+    (kernel 'coop' with coop_max 0): the full-vector kernel's amplitudes."""
+    h0, leaves, bas = water(14)
+    n = sum((2 * J + 1) ** 2 for J in range(15))
+    fields = water_fields(395.0 + DT * np.arange(3))
+    f = TDSE(t_end=20.0, dt=DT, t_units="fs").exp_fac
+    H = _summed(leaves, fields, 0)
+    out = []
+    for kern in ("coop", "global"):
+        e = ensemble.Ensemble(H, h0, f, _rows(n, 3, 4)[1:], krylov_fixed=fixed)
+        e.set_kernel(kern)
+        e.set_tuning(coop_max=0 if kern == "coop" else 8)
+        e.propagate(None, table=e.prepare(fields, per_term=True))
+        out.append(e.psi.cpu().numpy())
+        e.set_tuning()
+    assert np.abs(out[0] - out[1]).max() <= 1e-11
