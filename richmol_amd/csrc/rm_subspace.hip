@@ -958,7 +958,10 @@ std::vector<double2> entry_values(const rm_plan* p) {
 // All values real, and symmetric, to the rounding of the complex products and
 // sums that formed them: imaginary parts of at most 4 and pairs of entries
 // within 8 units in the last place (rotors and tops up to J = 62 in Z and XZ
-// fields: 1.6 and 4.3).  What is larger is the caller's and is kept, a NaN too.
+// fields: 1.6 and 4.3).  Entries that are themselves rounding (an
+// element of 1e-34 beside ones of 1e-18, as a cancelled sum leaves) may have any
+// imaginary part below 2^-60 of their slot's largest element, less than the
+// row sums round.  What is larger is the caller's and is kept, a NaN too.
 // (Rows hold their columns ascending; next[c]: the first entry of row c that no
 // row above has passed.)
 void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
@@ -966,11 +969,13 @@ void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vecto
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   p->sreal = true;
-  for (const double2& v : cval)
-    if (!(std::fabs(v.y) <= 0x1p-50 * std::fabs(v.x))) {
-      p->sreal = false;
-      break;
-    }
+  for (int32_t s = 0; s < nf && p->sreal; ++s) {
+    const double2* v = cval.data() + (size_t)s * nnz;
+    double top = 0.0;
+    for (int64_t e = 0; e < nnz; ++e) top = std::max(top, std::fabs(v[e].x));
+    for (int64_t e = 0; e < nnz && p->sreal; ++e)
+      p->sreal = std::fabs(v[e].y) <= std::max(0x1p-50 * std::fabs(v[e].x), 0x1p-60 * top);
+  }
   p->ssym = p->sreal;
   std::vector<int64_t> next(rp.begin(), rp.end() - 1);
   for (int64_t r = 0; r < n && p->ssym; ++r)

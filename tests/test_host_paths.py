@@ -176,6 +176,8 @@ def case_real_operators(s):
     for vals, real, symmetric in ((sym, True, True), (s.vals, True, False), (sym * (1 + 2.0 ** -51 * 1j), True, True),
                                   (sym * (1 + 2.0 ** -49 * 1j * one), False, False),
                                   (sym + np.where(one > 0, complex(0, np.nan), 0), False, False),
+                                  (np.where(one > 0, 1e-25 * (1 + 0.4j), sym), True, False),
+                                  (np.where(one > 0, 1e-15 * (1 + 0.4j), sym), False, False),
                                   (sym * (1 + 2.0 ** -50 * one), True, True),
                                   (sym * (1 + 2.0 ** -47 * one), True, False)):
         s.plan = s.make_plan(vals)
