@@ -163,7 +163,7 @@ struct rm_plan {
   int64_t* sub_rp = nullptr;     // [n+1]
   int32_t* sub_ccol = nullptr;   // [nnz] permuted column
   double2* sub_cval = nullptr;   // [nfield][nnz]
-  float2* sub_cval32 = nullptr;  // [nfield][nnz] the same in FP32 (FP32-mode matvecs read it)
+  float2* sub_cval32 = nullptr;  // [nnz] the same in FP32, with one slot (what its FP32 matvecs read)
   std::vector<int64_t> h_sub_rp;
   // the same entries in slices of up to 64 permuted rows (rm_block.hip): a
   // slice holds whole subspaces, or 64 rows of one; (first row, rows, pairs of

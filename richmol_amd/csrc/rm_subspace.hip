@@ -964,17 +964,24 @@ std::vector<double2> entry_values(const rm_plan* p) {
 // row sums round.  What is larger is the caller's and is kept, a NaN too.
 // (Rows hold their columns ascending; next[c]: the first entry of row c that no
 // row above has passed.)
-void operator_flags(rm_plan* p, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
-                    const std::vector<double2>& cval) {
+void operator_flags(rm_plan* p, const std::vector<double2>& cval) {
+  const std::vector<int64_t>& rp = p->h_row_ptr;
+  const std::vector<int32_t>& ccol = p->h_col;
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   p->sreal = true;
   for (int32_t s = 0; s < nf && p->sreal; ++s) {
     const double2* v = cval.data() + (size_t)s * nnz;
-    double top = 0.0;
-    for (int64_t e = 0; e < nnz; ++e) top = std::max(top, std::fabs(v[e].x));
-    for (int64_t e = 0; e < nnz && p->sreal; ++e)
-      p->sreal = std::fabs(v[e].y) <= std::max(0x1p-50 * std::fabs(v[e].x), 0x1p-60 * top);
+    double top = 0.0, rest = 0.0;   // the largest real part, the largest imaginary part beyond 4 ulp
+    for (int64_t e = 0; e < nnz && p->sreal; ++e) {
+      const double x = std::fabs(v[e].x), y = std::fabs(v[e].y);
+      top = std::max(top, x);
+      if (!(y <= 0x1p-50 * x)) {
+        rest = std::max(rest, y);
+        p->sreal = std::isfinite(v[e].x) && std::isfinite(v[e].y);
+      }
+    }
+    p->sreal = p->sreal && rest <= 0x1p-60 * top;
   }
   p->ssym = p->sreal;
   std::vector<int64_t> next(rp.begin(), rp.end() - 1);
@@ -1018,29 +1025,29 @@ void slice_shape(rm_plan* p, int32_t max_rows, const std::vector<int64_t>& rp, s
   }
 }
 
-// The sliced form of the permuted CSR arrays (rm_block.hip) of subspaces of at
-// most RM_SUBSPACE_MAX_ROWS rows, packed here with the plan.
-int slice_build(rm_plan* p, Uploader& up, const std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
-                const std::vector<double2>& cval) {
+// The sliced form of the operator (rm_block.hip) in the permuted order, of
+// subspaces of at most RM_SUBSPACE_MAX_ROWS rows, packed here with the plan.
+int slice_build(rm_plan* p, Uploader& up, const std::vector<int32_t>& iperm, const std::vector<double2>& B) {
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   std::vector<int4> sl;
   std::vector<int64_t> off;
-  slice_shape(p, RM_SUBSPACE_MAX_ROWS, rp, sl, off);
+  slice_shape(p, RM_SUBSPACE_MAX_ROWS, p->h_sub_rp, sl, off);
   const int64_t np = off.back();
   const int q = p->sreal ? 2 : 4;   // values of a pair
   std::vector<uint32_t> col((size_t)std::max<int64_t>(np, 1), 0);
   std::vector<double> val((size_t)(nf * np * q), 0.0);
   for (size_t i = 0; i < sl.size(); ++i)
     for (int32_t l = 0; l < sl[i].y && sl[i].z > 0; ++l) {
-      const int64_t e0 = rp[sl[i].x + l], len = rp[sl[i].x + l + 1] - e0;
+      const int32_t r = p->h_sub_perm[sl[i].x + l];
+      const int64_t e0 = p->h_row_ptr[r], len = p->h_row_ptr[r + 1] - e0;
       const uint32_t self = (uint32_t)((sl[i].x + l - sl[i].w) * 16);   // padding: the row's own column
       for (int64_t j = 0; j < 2 * (int64_t)sl[i].z; ++j) {
         const int64_t at = off[i] + 64 * (j / 2) + l;
-        col[(size_t)at] |= (j < len ? (uint32_t)((ccol[e0 + j] - sl[i].w) * 16) : self) << (16 * (j & 1));
+        col[(size_t)at] |= (j < len ? (uint32_t)((iperm[p->h_col[e0 + j]] - sl[i].w) * 16) : self) << (16 * (j & 1));
         if (j >= len) continue;
         for (int32_t s = 0; s < nf; ++s) {
-          const double2 v = cval[(size_t)s * nnz + e0 + j];
+          const double2 v = B[(size_t)s * nnz + e0 + j];
           double* d = val.data() + (size_t)((s * np + at) * q);
           if (p->sreal) {
             d[j & 1] = v.x;
@@ -1051,7 +1058,8 @@ int slice_build(rm_plan* p, Uploader& up, const std::vector<int64_t>& rp, const 
         }
       }
     }
-  const std::vector<float> val32(val.begin(), val.end());
+  // (read with one slot only: with several the kernels round the step's sums)
+  const std::vector<float> val32(val.begin(), nf == 1 ? val.end() : val.begin());
   up.add(&p->sslice, sl.data(), (int64_t)sl.size());
   up.add(&p->soff, off.data(), (int64_t)off.size());
   up.add(&p->srow, p->h_srow.data(), n);
@@ -1068,55 +1076,29 @@ int slice_build(rm_plan* p, Uploader& up, const std::vector<int64_t>& rp, const 
 
 // The B_s as CSR in permuted row and column order (the cooperative kernel's
 // operator); rows keep the order of their entries.
-void csr_host(const rm_plan* p, const std::vector<double2>& B, std::vector<int64_t>& rp, std::vector<int32_t>& ccol,
-              std::vector<double2>& cval) {
+int csr_build(rm_plan* p, const std::vector<double2>& B) {
+  if (p->sub_rp) return RM_OK;
   const int64_t n = p->n, nnz = p->nnz;
   const int32_t nf = std::max(p->nfield, 1);
   const std::vector<int32_t>& perm = p->h_sub_perm;
   std::vector<int32_t> iperm((size_t)n);
   for (int64_t ip = 0; ip < n; ++ip) iperm[perm[ip]] = (int32_t)ip;
-  rp.assign((size_t)n + 1, 0);
+  std::vector<int32_t> ccol((size_t)nnz);
+  std::vector<double2> cval((size_t)nf * (size_t)nnz);
   for (int64_t ip = 0; ip < n; ++ip) {
-    const int32_t i = perm[ip];
-    rp[ip + 1] = rp[ip] + (p->h_row_ptr[i + 1] - p->h_row_ptr[i]);
+    const int64_t r0 = p->h_row_ptr[perm[ip]], c0 = p->h_sub_rp[ip], len = p->h_sub_rp[ip + 1] - c0;
+    for (int64_t j = 0; j < len; ++j) ccol[c0 + j] = iperm[p->h_col[r0 + j]];
+    for (int32_t s = 0; s < nf; ++s)
+      std::copy_n(B.begin() + ((int64_t)s * nnz + r0), len, cval.begin() + ((int64_t)s * nnz + c0));
   }
-  ccol.resize((size_t)nnz);
-  cval.resize((size_t)nf * (size_t)nnz);
-  for (int64_t ip = 0; ip < n; ++ip) {
-    const int32_t i = perm[ip];
-    const int64_t r0 = p->h_row_ptr[i], len = p->h_row_ptr[i + 1] - r0;
-    for (int64_t j = 0; j < len; ++j) {
-      ccol[(size_t)(rp[ip] + j)] = iperm[p->h_col[r0 + j]];
-      for (int32_t s = 0; s < nf; ++s)
-        cval[(size_t)s * nnz + (size_t)(rp[ip] + j)] = B[(size_t)s * nnz + (size_t)(r0 + j)];
-    }
-  }
-}
-
-int csr_upload(rm_plan* p, std::vector<int64_t>& rp, const std::vector<int32_t>& ccol,
-               const std::vector<double2>& cval) {
-  const int64_t n = p->n, nnz = p->nnz;
-  const int32_t nf = std::max(p->nfield, 1);
-  std::vector<float2> cval32(cval.size());
-  for (size_t q = 0; q < cval.size(); ++q) cval32[q] = make_float2((float)cval[q].x, (float)cval[q].y);
+  std::vector<float2> cval32(nf == 1 ? cval.size() : 0);   // read with one slot only
+  for (size_t q = 0; q < cval32.size(); ++q) cval32[q] = make_float2((float)cval[q].x, (float)cval[q].y);
   Uploader up;
-  up.add(&p->sub_rp, rp.data(), n + 1);
+  up.add(&p->sub_rp, p->h_sub_rp.data(), n + 1);
   up.add(&p->sub_ccol, ccol.data(), nnz);
   up.add(&p->sub_cval, cval.data(), (int64_t)nf * nnz);
-  up.add(&p->sub_cval32, cval32.data(), (int64_t)nf * nnz);
-  const int rc = up.commit(p->arenas);
-  if (rc) return rc;
-  p->h_sub_rp.swap(rp);
-  return RM_OK;
-}
-
-int csr_build(rm_plan* p, const std::vector<double2>& B) {
-  if (p->sub_rp) return RM_OK;
-  std::vector<int64_t> rp;
-  std::vector<int32_t> ccol;
-  std::vector<double2> cval;
-  csr_host(p, B, rp, ccol, cval);
-  return csr_upload(p, rp, ccol, cval);
+  up.add(&p->sub_cval32, cval32.data(), (int64_t)cval32.size());
+  return up.commit(p->arenas);
 }
 
 // A workgroup per slice: its entries from the CSR arrays (slice_build's packing).
@@ -1141,10 +1123,10 @@ __global__ __launch_bounds__(256) void k_slice_pack(const int4* __restrict__ ssl
         const double2 v = 2 * p + j < len ? cval[(int64_t)s * nnz + e0 + 2 * p + j] : make_double2(0.0, 0.0);
         const int64_t d = (s * np + at) * q + (q / 2) * j;
         sval[d] = v.x;
-        sval32[d] = (float)v.x;
-        if (!real) {
-          sval[d + 1] = v.y;
-          sval32[d + 1] = (float)v.y;
+        if (!real) sval[d + 1] = v.y;
+        if (sval32) {
+          sval32[d] = (float)v.x;
+          if (!real) sval32[d + 1] = (float)v.y;
         }
       }
   }
@@ -1158,12 +1140,16 @@ __global__ __launch_bounds__(256) void k_slice_pack(const int4* __restrict__ ssl
 // stay with the plan: launches may still read them.
 int slice_need(rm_plan* p, int32_t len) {
   if (len <= p->slice_rows || len > BLK_MAX_ROWS) return RM_OK;
+  int rc = RM_OK;
+  if (!p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
   std::vector<int4> sl;
   std::vector<int64_t> off;
   slice_shape(p, BLK_MAX_ROWS, p->h_sub_rp, sl, off);
   const int64_t np = off.back(), nval = (int64_t)std::max(p->nfield, 1) * np * (p->sreal ? 2 : 4);
+  const bool f32 = p->nfield <= 1;   // FP32 copies are read with one slot only
   const size_t bytes[6] = {sizeof(int4) * sl.size(), sizeof(int64_t) * off.size(), sizeof(int32_t) * (size_t)p->n,
-                           sizeof(uint32_t) * (size_t)np, sizeof(double) * (size_t)nval, sizeof(float) * (size_t)nval};
+                           sizeof(uint32_t) * (size_t)np, sizeof(double) * (size_t)nval,
+                           sizeof(float) * (size_t)(f32 ? nval : 0)};
   const void* src[6] = {sl.data(), off.data(), p->h_srow.data(), nullptr, nullptr, nullptr};
   size_t at[7] = {0};
   for (int i = 0; i < 6; ++i) at[i + 1] = (at[i] + bytes[i] + 255) & ~(size_t)255;
@@ -1174,12 +1160,12 @@ int slice_need(rm_plan* p, int32_t len) {
     hipLaunchKernelGGL(k_slice_pack, dim3((unsigned)sl.size()), dim3(256), 0, 0, (const int4*)(d + at[0]),
                        (const int64_t*)(d + at[1]), p->sub_rp, p->sub_ccol, p->sub_cval, p->nnz,
                        std::max(p->nfield, 1), np, p->sreal ? 1 : 0, (uint32_t*)(d + at[3]), (double*)(d + at[4]),
-                       (float*)(d + at[5]));
+                       f32 ? (float*)(d + at[5]) : nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(0));
     return RM_OK;
   };
-  const int rc = fill();
+  rc = fill();
   if (rc) {
     (void)hipFree(d);
     return rc;
@@ -1190,7 +1176,7 @@ int slice_need(rm_plan* p, int32_t len) {
   p->srow = (int32_t*)(d + at[2]);
   p->scol = (uint32_t*)(d + at[3]);
   p->sval = (double*)(d + at[4]);
-  p->sval32 = (float*)(d + at[5]);
+  p->sval32 = f32 ? (float*)(d + at[5]) : nullptr;
   p->spairs = np;
   p->slice_rows = BLK_MAX_ROWS;
   p->h_soff.swap(off);
@@ -1281,14 +1267,13 @@ int sub_build(rm_plan* p) {
     up.add(&p->sub_val, (const double2*)hval.data(), (int64_t)((size_t)nf * ne));
   }
   p->h_sub_perm = perm;
-  std::vector<int64_t> rp;
-  std::vector<int32_t> ccol;
-  std::vector<double2> cval;
-  csr_host(p, B, rp, ccol, cval);
-  operator_flags(p, rp, ccol, cval);
-  if ((rc = slice_build(p, up, rp, ccol, cval))) return rc;
+  p->h_sub_rp.assign((size_t)n + 1, 0);
+  for (int64_t ip = 0; ip < n; ++ip)
+    p->h_sub_rp[ip + 1] = p->h_sub_rp[ip] + (p->h_row_ptr[perm[ip] + 1] - p->h_row_ptr[perm[ip]]);
+  operator_flags(p, B);
+  if ((rc = slice_build(p, up, iperm, B))) return rc;
   // CSR (row-major, permuted) for the cooperative kernel: if some subspace does not fit
-  if (mx > RM_SUBSPACE_MAX_ROWS && (rc = csr_upload(p, rp, ccol, cval))) return rc;
+  if (mx > RM_SUBSPACE_MAX_ROWS && (rc = csr_build(p, B))) return rc;
   p->sub_w = W;
   p->sub_ready = 1;
   return RM_OK;
@@ -2125,7 +2110,6 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
         if (known) *known = (int8_t)cl;
       }
     }
-    if (!big.empty() && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
     // a few real ones in FP64 go to teams of workgroups (rm_team.hip).  Else
     // the cooperative form runs its wavepackets one launch after another on
     // many workgroups, the block form all of them at once, one workgroup
@@ -2150,12 +2134,15 @@ int sub_propagate(rm_plan* p, void* psi, int64_t ld, int64_t ncols, int64_t nste
     const bool to_coop = force == RM_KERNEL_COOP || team > 0 ||
                          (force == 0 && (int64_t)big.size() <= p->tune.coop_max &&
                           (int64_t)big.size() * p->tune.coop_min_entries <= emin);
+    bool csr = false;   // some item is for the kernels of rm_coop.hip, which read the CSR arrays
     // before the items that are kept: they hold their domains' slice widths
     if ((!to_coop || team > 0) && (rc = slice_need(p, longest))) return rc;
     for (const int4& it : big) {
       (to_coop ? sc->kept_coop : sc->kept_blk).push_back(long_item(p, it.x, it.y, it.z, 0));
       if (to_coop) sc->kept_coop.back().team = team;
+      csr |= to_coop ? team == 0 : sc->kept_blk.back().variant == 0;
     }
+    if (csr && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
     sort_long(sc->kept_blk);
     for (auto& v : sc->kept_cls) longest_first(v);
     group_pairs(sc->kept_cls, krylov_fixed, p->tune.pair != 0, p->sreal ? 0 : COMPLEX4_CLASS);
@@ -2360,8 +2347,12 @@ static int collect_jobs(const char* who, const rm_job* jobs, int32_t njobs, int3
       return fail(RM_ERR_ARG, "%s: job %d: a domain of %d rows needs the block kernel, whose workspace this "
                   "entry point does not hold (at most %d rows; use rm_batch_propagate)", who, j, len,
                   RM_SUBSPACE_MAX_ROWS);
-    if (longdom && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
-    if (longdom && (rc = slice_need(p, len))) return rc;
+    LongItem li;
+    if (longdom) {
+      if ((rc = slice_need(p, len))) return rc;
+      li = long_item(p, jb.col, lo, len, (int)ops.size());
+      if (li.variant == 0 && !p->sub_rp && (rc = csr_build(p, entry_values(p)))) return rc;
+    }
     SubOp op = plan_op(p);
     op.phase = (const double2*)jb.phase;
     op.table = (const double2*)jb.fprod_dev;
@@ -2375,7 +2366,7 @@ static int collect_jobs(const char* who, const rm_job* jobs, int32_t njobs, int3
     op.f = make_double2(jb.f_re, jb.f_im);
     op.nsteps = jb.nsteps;
     if (longdom) {
-      blk.push_back(long_item(p, jb.col, lo, len, (int)ops.size()));
+      blk.push_back(li);
       blk_work.push_back((int64_t)jb.nsteps * blk.back().nent);
     } else {
       const int c = sub_class(p, lo, len);

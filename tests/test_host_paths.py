@@ -3,7 +3,8 @@ hip_host_stub.cpp: memory is host memory, kernels do not run, launches are
 recorded and allocations can be made to fail.  What a plan's launches read after
 an allocation failed, and after its arrays were replaced; which operators count
 as real and as symmetric; where rows with repeated columns run; a device with no
-room for operators formed ahead; as many static jobs as the header allows.
+room for operators formed ahead; as many static jobs as the header allows;
+the arrays a call is built from.
 """
 import ctypes
 import os
@@ -239,6 +240,22 @@ def case_static_jobs(s):
             assert rc == 0, s.lib.rm_last_error()
 
 
+def case_arrays_of_a_call(s):
+    """A mid-size domain's block launch is built without the CSR arrays that only
+    the cooperative kernels read; the cooperative form on the same plan gets them."""
+    on = s.rows >= LONG
+    s.plan = s.make_plan(s.vals[:, on], s.rows[on] - LONG, s.cols[on] - LONG, SHORT)
+    s.n, s.psi, s.work = SHORT, np.zeros((1, SHORT), np.complex128), np.zeros((1, SHORT), np.complex128)
+    s.psi[0, 3] = 1.0
+    for kernel, launch, csr in ((6, "k_blkILb", False), (5, "k_longILi", True)):
+        assert s.lib.rm_plan_set_kernel(s.plan, kernel) == 0
+        assert s.propagate() == 0 and len(s.launches(launch)) == 1
+        assert s.job(0, SHORT) == 0
+        (words, _, _), = s.launches("k_blkILb")
+        rp = int(np.frombuffer(ctypes.string_at(words[0] + 8 * 2, 8), np.uint64)[0])
+        assert (rp != 0) == csr
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
@@ -248,7 +265,7 @@ def stub(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["failed_allocation", "kept_lists", "real_operators", "repeated_columns",
-                                  "no_room_for_operators", "static_jobs"])
+                                  "no_room_for_operators", "static_jobs", "arrays_of_a_call"])
 def test_host_path(stub, case):
     from richmol_amd import _build
     if not os.path.exists(_build.LIB_PATH):
