@@ -18,7 +18,8 @@
 // after one step and of 3-4e-13 after 1 000 (the dense form's norm drifts by
 // 0.3-0.9e-13 in these).  Now only what a step adds carries it: 1.6e-16 after one
 // step at J = 80 (dense form 2.0e-16), after 1 000 steps at J <= 20 a norm
-// drift of 0.2-1.0e-13 in a field of 1e9 V/m, 1.3-2.1e-13 in one of 5e9.
+// drift of 0.2-1.0e-13 in a field of 1e9 V/m, 1.3-2.1e-13 in one of 5e9; at
+// J = 80 in one of 1e8 7.6e-14 (dense form 7.9e-14).
 //
 // Vectors are (wavepacket, internal order) arrays of complex values, as the
 // caller's rows: J blocks of (m, k), k fastest.  The basis is kept as the
@@ -27,12 +28,12 @@
 // 16 n bytes per wavepacket.
 //
 // Measured (MI355X, J <= 80 all m: 708 561 states, 64 wavepackets, Krylov
-// dimension 12, dipole + full polarizability in an XY field): 20.5 ms per step
-// FP64, 17.7 ms with FP32 products, where the dense form (m-mixed input stored,
+// dimension 12, dipole + full polarizability in an XY field): 20.4 ms per step
+// FP64, 17.6 ms with FP32 products, where the dense form (m-mixed input stored,
 // rocBLAS products) takes 157.5 and 112.2 ms; J <= 31, 16 wavepackets, adaptive,
-// <cos^2> read: 0.37 ms per step against 4.8.  Of the 20.5 ms the stencils take
-// 10.7 (0.89 each), the vector updates 6.1 (0.55 each: 2.9 GB at 5.3 TB/s), the
-// final combination 1.9 (9.4 GB at 5.1 TB/s), the transforms 1.6.  FP32 error
+// <cos^2> read: 0.36 ms per step against 4.8.  Of the 20.4 ms the stencils take
+// 10.8 (0.90 each), the vector updates 6.0 (0.55 each: 2.9 GB at 5.2 TB/s), the
+// final combination 1.7 (8.9 GB at 5.2 TB/s), the transforms 1.7.  FP32 error
 // against 64-bit dense products 2.6e-9 (dense form 3.2e-9).
 
 #include <algorithm>
