@@ -92,8 +92,8 @@ class Ensemble:
             self._apply_kernel()
 
     def set_tuning(self, **choices):
-        """Launch choices of the subspace path (pair, coop_max, coop_grid,
-        fork; see Plan.set_tuning) for this ensemble's calls."""
+        """Launch choices of the subspace path (DevicePlan.set_tuning) for this
+        ensemble's calls."""
         self.tuning = dict(choices)
         if self.plan is not None:
             self._apply_kernel()

@@ -299,7 +299,8 @@ class DevicePlan:
 
     def set_tuning(self, **choices):
         """Launch choices of rm_propagate's subspace path (rm_plan_set_tuning):
-        pair, coop_max, coop_grid, fork; a choice not given returns to its
+        pair, coop_max, coop_grid, fork, wave_max_rows, coop_min_entries,
+        operator_kib; a choice not given returns to its
         default."""
         want = dict(_lib.TUNE_DEFAULTS)
         for k, v in choices.items():
