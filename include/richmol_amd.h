@@ -434,8 +434,7 @@ int rm_kplan_info(const rm_kplan* plan, int64_t* n, double* gemm_flops_per_col);
 /* Matvec form (no reference counterpart).  RM_KKERNEL_PRIM (default of a plan
  * with K factors, rm_kplan_set_factors): the operator as a stencil in the
  * primitive symmetric-top basis.  (rm_kplan_propagate_expect runs in it when the
- * observable's plan is in this form with the same C too, else in the dense
- * form.)  RM_KKERNEL_GEMM (default without): the
+ * observable's plan is in this form too, else in the dense form.)  RM_KKERNEL_GEMM (default without): the
  * m-mixed input (MF_w X) stored, then one rocBLAS product per output J, the
  * build of the next J chunk overlapping the products of the last.
  * RM_KKERNEL_FUSED: one launch per matvec on the matrix cores, the m-mixed

@@ -20,14 +20,12 @@ struct KPrimBlock {
 int kprim_create(KPrim** out, const std::vector<int32_t>& Js, const std::vector<int64_t>& voff, int64_t n,
                  const std::vector<KPrimBlock>& blk, const double2* mdiag, const double* C, const double* P);
 void kprim_free(KPrim* p);
-// do both work in the same primitive basis (same J list, bit-equal C)?
-bool kprim_same_basis(const KPrim* a, const KPrim* b);
 // y = H(F) x (rows of stride ld, the plan's internal order)
 int kprim_matvec(KPrim* p, const double2* x, double2* y, int64_t ld, int32_t ncols, const double2* fprod, bool f32,
                  hipStream_t s);
 // rm_kplan_propagate on this form; d_fp: the steps' field products on the
-// device, fprod: the same on the host.  obs (may be NULL): an observable in
-// the same basis, d_ofp its products; ex: [nsteps][ncols] values.
+// device, fprod: the same on the host.  obs (may be NULL): an observable on
+// the same states, d_ofp its products; ex: [nsteps][ncols] values.
 int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t nsteps, int32_t nslot,
                     const double* fprod, const double2* d_fp, double2 f, const double2* phase, int32_t krylov_fixed,
                     int32_t maxorder, double tol, int32_t* kused, int32_t* status, bool f32, KPrim* obs,

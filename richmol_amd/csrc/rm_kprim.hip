@@ -81,7 +81,6 @@ struct KPrim {
   std::vector<int32_t> Js;
   std::vector<int64_t> voff;
   int64_t n = 0;
-  std::vector<double> h_C;
   bool cplx = false;               // some C has an imaginary part
   int32_t nblk = 0;
   std::vector<PMf> h_mfd;
@@ -819,11 +818,6 @@ int launch_tr(KPrim* p, bool fwd, const double2* in, int64_t ldi, double2* out, 
 
 }  // namespace
 
-bool kprim_same_basis(const KPrim* a, const KPrim* b) {
-  return a && b && a->Js == b->Js && a->h_C.size() == b->h_C.size() &&
-         memcmp(a->h_C.data(), b->h_C.data(), sizeof(double) * a->h_C.size()) == 0;
-}
-
 void kprim_free(KPrim* p) {
   if (!p) return;
   void* bufs[] = {p->d_pj, p->d_task, p->d_mfd, p->d_gpat, p->d_p, p->d_p32, p->d_mf, p->d_mf32, p->d_T, p->d_toff,
@@ -848,7 +842,6 @@ int kprim_create(KPrim** out, const std::vector<int32_t>& Js, const std::vector<
   // transforms: T forward [s][k] = C[k][s], backward [k][s] = conj(C[k][s]); re plane, then im
   int64_t cpos = 0;
   for (int a = 0; a < nJ; ++a) cpos += jd(Js[a]) * jd(Js[a]);
-  p->h_C.assign(C, C + 2 * cpos);
   for (int64_t i = 0; i < cpos && !p->cplx; ++i) p->cplx = C[2 * i + 1] != 0.0;
   const int np = p->cplx ? 2 : 1;
   std::vector<double> T((size_t)(2 * np * cpos));
@@ -1050,9 +1043,9 @@ int kprim_propagate(KPrim* p, double2* psi, int64_t ld, int32_t ncols, int64_t n
       if ((rc = launch_tr(p, false, w.W, p->n, psi, ld, phase, ncols, s, w.coef, m))) return rc;
     }
     if (obs) {
-      // <S|O|S> in the primitive basis: the wavepackets once more forward,
-      // the observable's stencil with its partial sums (FP64, output not kept)
-      if ((rc = launch_tr(p, true, psi, ld, w.W, p->n, nullptr, ncols, s))) return rc;
+      // <S|O|S> in the observable's primitive basis: the wavepackets once more
+      // forward, its stencil with its partial sums (FP64, output not kept)
+      if ((rc = launch_tr(obs, true, psi, ld, w.W, p->n, nullptr, ncols, s))) return rc;
       if ((rc = launch_sten<double, double>(obs, w.W, ncols, nullptr, nullptr, w.part, s))) return rc;
       hipLaunchKernelGGL(k_pr_ofin, cg, cb, 0, s, w.part, obs->nslots, ex + st * ncols);
       HIPCHK(hipGetLastError());

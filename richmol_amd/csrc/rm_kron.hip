@@ -1640,8 +1640,7 @@ static int kplan_propagate(rm_kplan* p, void* psi, int64_t ld, int32_t ncols, in
   if ((rc = grow(&p->d_fp, &p->fp_cap, nsteps * nf))) return rc;
   if (p->nslot)
     HIPCHK(hipMemcpyAsync(p->d_fp, fprod, sizeof(double2) * nsteps * p->nslot, hipMemcpyHostToDevice, s));
-  if (p->kernel == RM_KKERNEL_PRIM &&
-      (!obs || (obs->kernel == RM_KKERNEL_PRIM && kprim_same_basis(p->prim, obs->prim)))) {
+  if (p->kernel == RM_KKERNEL_PRIM && (!obs || obs->kernel == RM_KKERNEL_PRIM)) {
     double2* ex = expect;
     if (obs) {
       if (!ex) {

@@ -439,8 +439,8 @@ class DeviceKronPlan:
         """'prim' (default with kop.factors): a stencil in the primitive
         symmetric-top basis, the wavepackets transformed once before and
         after each step's Krylov recurrence;
-        With an observable whose plan has another kernel or other
-        coefficients the call runs in the dense form, 4 to 8 times slower;
+        With an observable whose plan has another kernel the call runs in
+        the dense form, 4 to 8 times slower;
         'gemm' (default without): the m-mixed input stored, rocBLAS per output J;
         'mfma': the m-mixed input stored, the library's own matrix-core
         product per J chunk; 'fused': one MFMA launch per matvec, the m-mixed

@@ -193,3 +193,36 @@ def test_no_drift_against_dense_form(device, jmax):
         dp.propagate(psi, fp, -0.0019j, phase=dp.phases(-0.0019j), krylov_fixed=10)
         out.append(psi.cpu().numpy())
     assert np.all(np.linalg.norm(out[0] - out[1], axis=1) <= 1000 * 2.0 ** -53)
+
+
+@pytest.mark.parametrize("other", ["coefficients", "gemm"])
+def test_observable_plan_of_its_own(device, other):
+    """An observable whose coefficients differ in their last bits from the
+    operator's (another build of the same basis), or whose plan is in the dense
+    form: the values of the dense form (1e-11)."""
+    import torch
+    bas = _basis(0, 6, False)
+    kop = KronOperator(bas, *large_top_tensors())
+    if other == "coefficients":
+        for J in bas.Jlist:
+            for s, (kp, c) in bas.kfun[J].items():
+                bas.kfun[J][s] = (kp, c * (1 + 2.0 ** -52))
+    kc = KronOperator(bas, [np.diag([0.0, 0.0, 1.0])], [1.0])
+    E = 3e9 * np.array([[1, 0, 0], [0.6, 0.8, 0], [0.3, -0.4, 0.5]])
+    fp = slot_products(kop, [E, E])
+    ofp = slot_products(kc, [np.array([[0.0, 0.0, 1.0]])])[0]
+    X = _rows(kop.n, 3, 7)
+    X /= np.linalg.norm(X, axis=1)[:, None]
+    out = []
+    for kern in ("prim", "gemm"):
+        dp, dc = DeviceKronPlan(kop), DeviceKronPlan(kc)
+        assert dc.kernel == "prim"
+        dp.set_kernel(kern)
+        if other == "gemm" or kern == "gemm":
+            dc.set_kernel("gemm")
+        psi = torch.from_numpy(X).to(device)
+        ex = torch.empty((3, 3), dtype=torch.complex128, device=device)
+        dp.propagate(psi, fp, -0.002j, phase=dp.phases(-0.002j), krylov_fixed=9, obs=dc, obs_fprod=ofp, expect=ex)
+        out.append((psi.cpu().numpy(), ex.cpu().numpy()))
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() <= 1e-11
